@@ -18,11 +18,8 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;     // 4 wave64 per workgroup
 constexpr int kWave = 64;
-constexpr int kMaxGroup = 64;     // units per workgroup of the grouped copy kernels
-constexpr int kGatherUnroll = 16;  // 16-byte vectors per lane per half per round
-constexpr int kScatterUnroll = 16;
+constexpr int kScatterUnroll = 16;  // 16-byte V vectors per lane per round (pair-task kernel)
 constexpr int kRotCopyUnroll = 8;  // copy of unrotated pages inside the re-rotation kernels
-constexpr int kHndUnroll = 8;      // head-major page copies
 constexpr int kRotUnroll = 4;      // rotation tasks per lane per round (pair-task kernel)
 constexpr int kMaxRotHalf = 512;   // LDS table capacity: rot_dim <= 1024
 constexpr int kXcds = 8;           // MI355X: 8 XCDs, workgroups dealt round-robin
@@ -33,6 +30,10 @@ constexpr int kXcds = 8;           // MI355X: 8 XCDs, workgroups dealt round-rob
 // default-policy stores at the Llama-3-8B shape).
 constexpr int kLoadPolicy = 2;
 constexpr int kStorePolicy = 17;
+// The flat copies' stores: nt for launches that the caches can absorb, nt sc0
+// sc1 above (copy_shape in kv_move.hip).
+constexpr int kStoreNt = 2;
+constexpr int kStoreNtSc = 19;
 // Launch-shape overrides for measurements and tests, set through
 // dsr_set_tuning() (0 = the geometry's own choice). Nothing reads the
 // environment: a serving process gets the defaults unless its code asks.

@@ -10,19 +10,15 @@
 // Work decomposition. A vLLM page (block_size tokens x H heads x D dims) is
 // contiguous inside each per-layer cache; only the block index is permuted.
 // The unit of work is therefore one (page, layer): two contiguous runs of
-// page_bytes (K and V) on each side. One 256-lane workgroup owns one unit and
-// moves it with 16-byte lane vectors (buffer_load_dwordx4 /
-// buffer_store_dwordx4 through a descriptor bounded to the run), issuing
-// every load of a round before any store so each lane keeps up to 2*U
-// 16-byte requests in flight. No LDS is needed for the copy: both sides are
-// contiguous within a unit. The re-rotation kernels keep the unit's
-// (cos, sin) table in LDS.
+// page_bytes (K and V) on each side, moved with 16-byte lane vectors
+// (buffer_load_dwordx4 / buffer_store_dwordx4 through descriptors bounded to
+// the run) by waves of 1 KiB each way (kv_flat.h). No LDS is needed for the
+// copy: both sides are contiguous within a unit. The re-rotation kernels
+// keep the unit's (cos, sin) table in LDS.
 //
 // Kernel choice, by page and row geometry (all inside the entry points):
-//   gather / scatter: one unit per workgroup; pages of at most 4 KiB
-//     (scatter) or under 4 KiB (gather) take several units per workgroup
-//     (kv_copy_grouped_kernel); pages above 32 KiB take one workgroup per
-//     32 KiB part, and gathers of few units split their units further.
+//   gather / scatter, every page size, token-major and head-major:
+//     kv_flat_copy_kernel (1 KiB pieces, one per wave).
 //   re-rotation: kv_scatter_rerotate_grouped_kernel for pages below U * 4
 //     KiB and 16-bit pages of exactly U * 4 KiB (and 16-bit token-major pages
 //     of several such parts, one workgroup each); kv_scatter_rerotate_contig_
@@ -36,8 +32,8 @@
 //   split-x K pages (dsr_scatter_rerotate_kx): the contig and grouped
 //     kernels with the KX flag, or the pair-task kernel.
 //   head-major cache pages (dsr_*_hnd): the same kernels as token-major
-//     pages of that size with the HND flag (kv_copy_hnd_kernel for one unit
-//     per workgroup), whose cache-side offsets go through hnd_vec.
+//     pages of that size with the HND flag, whose cache-side offsets go
+//     through hnd_vec.
 // Calls too large for one launch run as several over page (token) ranges.
 //
 // Reference being replaced: the Python per-(request, block, layer) torch
@@ -55,6 +51,7 @@
 
 #include "kv_common.h"
 #include "kv_page_kernels.h"
+#include "kv_flat.h"
 #include "kv_rotate.h"
 #include "kv_slots.h"
 #include "kv_fanout.h"
@@ -151,6 +148,32 @@ int launch_page_ranges(const UnitArgs& a, int n_pages, int G, F launch) {
   return DSR_OK;
 }
 
+// Launches of a flat kernel over every piece of `a` (one launch unless the
+// workgroups exceed max_wg_per_launch()), `minor` the inner extent of its unit
+// order: launch(map, grid).
+template <class F>
+int launch_flat(const UnitArgs& a, int64_t pieces_per_unit, int64_t minor, bool chunked, F launch) {
+  constexpr int kWaves = kThreads / kWave;
+  const int64_t total = a.n_units * pieces_per_unit;
+  const int64_t per = max_wg_per_launch() * kWaves;
+  for (int64_t g0 = 0; g0 < total; g0 += per) {
+    const int64_t n = total - g0 < per ? total - g0 : per;
+    const unsigned grid = (unsigned)((n + kWaves - 1) / kWaves);
+    FlatMap m;
+    m.per_unit = fast_div((uint32_t)pieces_per_unit);
+    m.minor = fast_div((uint32_t)minor);
+    m.unit0 = (uint32_t)(g0 / pieces_per_unit);
+    m.wave0 = (uint32_t)(g0 % pieces_per_unit);
+    m.n_waves = (uint32_t)n;
+    constexpr unsigned kRound = kXcds << kChunkLog2;
+    m.chunked = chunked ? grid / kRound * kRound : 0;
+    launch(m, grid);
+    const int rc = (int)hipGetLastError();
+    if (rc != 0) return rc;
+  }
+  return DSR_OK;
+}
+
 // Workgroups per CU for the re-rotation kernel, applied with dynamic LDS
 // sized from the CU's LDS capacity (the DSR_TUNE_ROT_WG_PER_CU override changes it, for
 // tuning). Measured in-process at the Llama-3-8B shapes: 16-bit K (64 KiB
@@ -206,61 +229,65 @@ size_t rot_occupancy_lds(int wg_per_cu) {
   return occupancy_lds(wg_per_cu, (int64_t)sizeof(float2) * kMaxRotHalf);
 }
 
-// Workgroups per CU for the one-unit page copies (0: no limit; the copy
-// kernels' registers allow 3). Units in flight per CU are limited to about
-// 64 KiB of pages (K + V): one workgroup per CU at 32 KiB pages, two at 16
-// KiB. Measured in-process (ms, 3 per CU -> this policy): Llama-3-8B bf16
-// (32 KiB pages) scatter 12.08 -> 11.97 (stream kernel), gather 11.75 ->
-// 11.60, on three boxes alike; e4m3 (16 KiB pages) scatter 24.71 -> 24.07,
-// gather 22.07 -> 22.09. More than 64 KiB in flight per CU makes the DRAM
-// side slower, not faster (fewer, longer-waiting requests win); one
-// workgroup per CU at 16 KiB pages leaves the CU idle between units (28.4 ms).
-// Launches of fewer than kPacedMinUnits units (a single layer's save of a
-// step, ...) keep the registers' three workgroups per CU, with dynamic LDS
-// sized for three (one layer's scatter of 1,024-4,096 pages: 23.1 vs 24.4
-// and 83.4 vs 86.0 us without LDS; gathers alike): they end before a steady
-// state, and one per CU measured 0-11% slower there (one layer, 1,024-4,096
-// pages: gather 21.8 vs 19.6 us, 99 vs 94 us), against 1% faster from 8,192
-// units.
-constexpr int64_t kPacedMinUnits = 8192;
-int copy_wg_per_cu(int64_t page_bytes, int64_t n_units) {
-  if (const int64_t t = tune(DSR_TUNE_COPY_WG_PER_CU)) return (int)t;
-  if (n_units < kPacedMinUnits) return 3;
-  const int64_t w = (64 << 10) / (2 * page_bytes);
-  return w >= 3 ? 0 : (int)(w < 1 ? 1 : w);
+// Launch shape of a page copy, by the bytes it moves (read + written).
+// Measured per kernel in graphs of some 100 launches on 8 to 16 sets of buffers
+// in turn (more than the memory-side cache holds), Llama-3-8B pages, one
+// workgroup per unit -> the class's choice:
+//   up to 200 MiB: nt stores, which the L2s absorb while the pages are read:
+//     one-chunk loads 4.98 -> 2.92 us at 8.4 MB, 5.82 -> 4.52 at 17 MB, 20.9 ->
+//     18.1 at 101 MB, 32.7 -> 28.4 at 168 MB (sc0 sc1 stores 3.84, 5.45, 19.5,
+//     29.9); a layer's save 4.27 -> 3.17 us at 8.4 MB, 5.49 -> 4.52 at 17 MB;
+//   of these, from 20 to 32 MiB, which is one workgroup per CU: each wave holds
+//     8 KiB of K and of V, so that no second generation of waves starts: 7.14 ->
+//     5.77 us at 29 MB (single pieces 6.53), a layer's save 7.24 -> 6.24 at 34;
+//   above: nt sc0 sc1 stores, in chunks of workgroups (kChunkLog2): 50.3 -> 42.1
+//     us at 268 MB (nt 42.9), 185 -> 163 at 1.07 GB (nt 169), 738 -> 664 at 4.3
+//     GB (nt 681).
+// Where the same few buffers stay in the memory-side cache, sc0 sc1 stores are
+// up to 8% ahead of nt between 60 and 170 MB; a load's pages and records are
+// not there.
+// Four workgroups of single pieces per CU: 32 KiB of reads in flight there hide
+// the latency, and 6 or 8 per CU widen the written window (0-8% slower).
+constexpr int kCopyWgPerCu = 4;
+struct CopyShape {
+  bool nt;       // stores: nt, else nt sc0 sc1
+  bool whole;    // 8 pieces per wave
+  bool chunked;  // workgroups dealt in chunks
+};
+CopyShape copy_shape(const UnitArgs& a) {
+  const int64_t moved = 4 * a.page_bytes * a.n_units;
+  const bool large = moved > (200 << 20);
+  CopyShape c{!large, moved > (20 << 20) && moved <= (32 << 20), large};
+  if (const int64_t t = tune(DSR_TUNE_COPY_STORES)) c.nt = t == 1;
+  if (const int64_t t = tune(DSR_TUNE_COPY_PIECES)) c.whole = t == 8;
+  if (a.page_bytes % (8 * kPiece)) c.whole = false;
+  return c;
 }
 
-// Workgroups per unit of a one-unit gather launch (a layer's save of a
-// serving step moves 16-4,096 pages). Few units leave most CUs idle; split
-// units finish sooner. A part stays a whole number of 4 KiB (one vector per
-// lane). Measured per launch at the Llama-3-8B shape (32 KiB pages, rocprofv3
-// kernel durations, medians of 128 launches; split 1 -> chosen): 16 pages
-// 4.32 -> 3.32 us (8), 64 pages 5.36 -> 4.32 (8), 128 pages 6.16 -> 5.68
-// (4; 8: 6.52), 512 pages 14.5-15.2 -> 13.8 (2), 1,024 pages 26.9-27.5 ->
-// 25.0 (2), 2,048 pages 49.5 -> 46.9 (2), 4,096 pages 93.3 -> 90.8 (2); at
-// 256 pages (7.7-7.8 vs 7.9-8.2) and from 6,144 pages (equal, 4 slower)
-// one workgroup per unit stays. The DSR_TUNE_GATHER_SPLIT override sets it
-// (1: off).
-int gather_split(int64_t page_bytes, int64_t n_units) {
-  int64_t s = tune(DSR_TUNE_GATHER_SPLIT);
-  if (!s)
-    s = n_units <= 64 ? 8 : n_units <= 128 ? 4 : n_units >= 512 && n_units <= 4096 ? 2 : 1;
-  while (s > 1 && (page_bytes % (s * kThreads * 16) != 0 || n_units * s > max_wg_per_launch()))
-    s /= 2;
-  return (int)(s < 1 ? 1 : s);
+template <bool kGather>
+int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s) {
+  const CopyShape c = copy_shape(a);
+  const int64_t pieces = c.whole ? a.page_bytes / (8 * kPiece) : (a.page_bytes + kPiece - 1) / kPiece;
+  const int64_t t = tune(DSR_TUNE_COPY_WG_PER_CU);
+  const size_t dyn = occupancy_lds(t ? (int)t : kCopyWgPerCu, 0);
+  return launch_flat(a, pieces, kGather ? a.n_layers : n_pages, c.chunked,
+                     [&](const FlatMap& m, unsigned grid) {
+#define DSR_COPY(HND, POLICY, U) \
+  kv_flat_copy_kernel<kGather, HND, POLICY, U><<<grid, kThreads, dyn, s>>>(a, m)
+    if (a.hnd_heads) {
+      if (c.whole) DSR_COPY(true, kStoreNt, 8);
+      else if (c.nt) DSR_COPY(true, kStoreNt, 1);
+      else DSR_COPY(true, kStoreNtSc, 1);
+    } else {
+      if (c.whole) DSR_COPY(false, kStoreNt, 8);
+      else if (c.nt) DSR_COPY(false, kStoreNt, 1);
+      else DSR_COPY(false, kStoreNtSc, 1);
+    }
+#undef DSR_COPY
+  });
 }
 
-// Parts of a page above 32 KiB for the one-unit gather and the streaming
-// scatter: 32 KiB each (the copies' tuned unit; a workgroup's later rounds
-// would wait for its earlier stores, since vmcnt counts both). The
-// DSR_TUNE_PAGE_PARTS override sets it (1: whole pages).
 constexpr int64_t kPartBytes = 32 << 10;
-int page_parts(int64_t page_bytes) {
-  if (const int64_t t = tune(DSR_TUNE_PAGE_PARTS))
-    return page_bytes % (t * kThreads * 16) == 0 ? (int)t : 1;
-  return page_bytes > kPartBytes && page_bytes % kPartBytes == 0 ? (int)(page_bytes / kPartBytes)
-                                                                 : 1;
-}
 
 template <int DT>
 int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipStream_t s,
@@ -443,32 +470,7 @@ int dsr_gather(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
   UnitArgs a = make_unit(layer_base, n_layers, kv_stride, page_stride, page_bytes,
                          num_blocks, page_ids, slot_offsets, n_pages, staging,
                          staging_bytes, layer_bytes, layer0);
-  // Grouped only below one workgroup's 4 KiB: from 4 KiB up the one-unit
-  // kernel measured faster (6.14 vs 5.57 TB/s at 4 KiB pages; 3-8% at 8, 16
-  // and 32 KiB).
-  const int G = page_bytes < kThreads * 16 ? units_per_group(page_bytes, kGatherUnroll, kMaxGroup) : 1;
-  int split = 1;
-  if (G == 1) {
-    const int pp = page_parts(page_bytes);
-    split = gather_split(page_bytes / pp, a.n_units * pp);
-    a.parts = pp * split;
-  }
-  return launch_page_ranges(a, n_pages, G, [&](const UnitArgs& b, unsigned grid) {
-    const hipStream_t st = (hipStream_t)stream;
-    if (G > 1) {
-      kv_copy_grouped_kernel<true, kGatherUnroll><<<grid, kThreads, 0, st>>>(b, G);
-    } else {
-      // launches split for lack of units keep the registers' three
-      // workgroups per CU (they end before a steady state)
-      const int64_t wus = b.n_units * b.parts;  // workgroup-sized units
-      const size_t dyn =
-          occupancy_lds(split > 1 ? 3 : copy_wg_per_cu(page_bytes / b.parts, wus), 0);
-      if (b.parts > 1)
-        kv_gather_kernel<true><<<grid, kThreads, dyn, st>>>(b);
-      else
-        kv_gather_kernel<false><<<grid, kThreads, dyn, st>>>(b);
-    }
-  });
+  return launch_copy<true>(a, n_pages, (hipStream_t)stream);
 }
 
 int dsr_scatter_ex(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
@@ -483,56 +485,8 @@ int dsr_scatter_ex(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
   UnitArgs a = make_unit(layer_base, n_layers, kv_stride, page_stride, page_bytes,
                          num_blocks, page_ids, slot_offsets, n_pages, staging,
                          staging_bytes, layer_bytes, layer0);
-  // Grouped up to 4 KiB pages (6.47 vs 5.04 TB/s at 4 KiB); at 8-32 KiB the
-  // one-unit kernel measured equal or faster.
-  const int G = page_bytes <= kThreads * 16 ? units_per_group(page_bytes, kScatterUnroll, kMaxGroup) : 1;
-  // records read by several pages are partly served by the caches, so
-  // more bytes in flight pay (the 70B share's 64 shared chunks: 50.5 ms at
-  // the registers' 3 workgroups per CU vs 52.6 ms at one)
-  const bool shared = (flags & DSR_SHARED_RECORDS) && !tune(DSR_TUNE_COPY_WG_PER_CU);
-  // the streaming kernel moves pages above 32 KiB as 32 KiB parts, one
-  // workgroup each; U vectors per lane per round (8 for multiples of 32 KiB,
-  // 4 for 16 KiB multiples)
-  const int pp = G == 1 && !shared ? page_parts(page_bytes) : 1;
-  const int64_t part_bytes = page_bytes / pp;
-  const int su = part_bytes % (kThreads * 8 * 16) == 0 ? 8
-                 : part_bytes % (kThreads * 4 * 16) == 0 ? 4 : 0;
-  const int64_t pick = tune(DSR_TUNE_SCATTER_KERNEL);
-  const int wpc_part = shared ? 0 : copy_wg_per_cu(part_bytes, a.n_units * pp);
-  const int64_t kind = pick ? pick : wpc_part == 1 && su == 8 ? 2 : 1;
-  const bool stream_k = G == 1 && (kind == 2 || kind == 3) && su != 0;
-  if (stream_k) a.parts = pp;
-  const int wpc = stream_k ? wpc_part : shared ? 0 : copy_wg_per_cu(page_bytes, a.n_units);
-  return launch_page_ranges(a, n_pages, G, [&](const UnitArgs& b, unsigned grid) {
-    const hipStream_t st = (hipStream_t)stream;
-    if (G > 1) {
-      // dynamic LDS for the registers' three workgroups per CU: 6.95 vs
-      // 7.10 ms at the 70B TP8 share's 4 KiB pages (the same effect as for
-      // the token kernels; the gather measured alike with and without)
-      kv_copy_grouped_kernel<false, kScatterUnroll><<<grid, kThreads, occupancy_lds(3, 0), st>>>(b, G);
-      return;
-    }
-    const size_t dyn = occupancy_lds(wpc, 0);
-    const bool hw = kind == 2, split = b.parts > 1;
-    if (!stream_k)
-      kv_scatter_kernel<<<grid, kThreads, dyn, st>>>(b);
-    else if (su == 8 && hw && split)
-      kv_scatter_stream_kernel<8, true, true><<<grid, kThreads, dyn, st>>>(b);
-    else if (su == 8 && hw)
-      kv_scatter_stream_kernel<8, true><<<grid, kThreads, dyn, st>>>(b);
-    else if (su == 8 && split)
-      kv_scatter_stream_kernel<8, false, true><<<grid, kThreads, dyn, st>>>(b);
-    else if (su == 8)
-      kv_scatter_stream_kernel<8, false><<<grid, kThreads, dyn, st>>>(b);
-    else if (hw && split)
-      kv_scatter_stream_kernel<4, true, true><<<grid, kThreads, dyn, st>>>(b);
-    else if (hw)
-      kv_scatter_stream_kernel<4, true><<<grid, kThreads, dyn, st>>>(b);
-    else if (split)
-      kv_scatter_stream_kernel<4, false, true><<<grid, kThreads, dyn, st>>>(b);
-    else
-      kv_scatter_stream_kernel<4, false><<<grid, kThreads, dyn, st>>>(b);
-  });
+  (void)flags;  // the flat copy is the choice for shared records too
+  return launch_copy<false>(a, n_pages, (hipStream_t)stream);
 }
 
 int dsr_scatter(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
@@ -766,7 +720,7 @@ int dsr_scatter_rerotate_hnd(const uint64_t* layer_base, int n_layers,
 
 namespace {
 
-// Head-major copies: the unit geometry, then one unit per workgroup.
+// Head-major copies: the unit geometry, then the flat copies.
 int copy_hnd(bool gather, const uint64_t* layer_base, int n_layers, int64_t kv_stride,
              int64_t page_stride, int64_t page_bytes, int64_t num_blocks,
              const int32_t* page_ids, const int64_t* slot_offsets, int n_pages,
@@ -786,24 +740,8 @@ int copy_hnd(bool gather, const uint64_t* layer_base, int n_layers, int64_t kv_s
   a.hnd_heads = num_heads;
   a.hnd_block = block_size;
   a.hnd_row_vecs = (int)(page_bytes / rows / 16);
-  // units per workgroup as for token-major pages (dsr_gather / dsr_scatter)
-  const int G = gather ? (page_bytes < kThreads * 16
-                              ? units_per_group(page_bytes, kGatherUnroll, kMaxGroup) : 1)
-                       : (page_bytes <= kThreads * 16
-                              ? units_per_group(page_bytes, kScatterUnroll, kMaxGroup) : 1);
-  hipStream_t s = (hipStream_t)stream;
-  return launch_page_ranges(a, n_pages, G, [&](const UnitArgs& b, unsigned grid) {
-    if (G > 1 && gather)
-      kv_copy_grouped_kernel<true, kGatherUnroll, true><<<grid, kThreads, 0, s>>>(b, G);
-    else if (G > 1)
-      kv_copy_grouped_kernel<false, kScatterUnroll, true><<<grid, kThreads, 0, s>>>(b, G);
-    else if (gather)  // the page copies' occupancy policy: 11.26 vs 11.49 ms at
-      kv_copy_hnd_kernel<true><<<grid, kThreads,  // config 2's pages head-major
-                                 occupancy_lds(copy_wg_per_cu(page_bytes, b.n_units), 0), s>>>(b);
-    else  // 12.52 vs 12.71 ms
-      kv_copy_hnd_kernel<false><<<grid, kThreads,
-                                  occupancy_lds(copy_wg_per_cu(page_bytes, b.n_units), 0), s>>>(b);
-  });
+  return gather ? launch_copy<true>(a, n_pages, (hipStream_t)stream)
+                : launch_copy<false>(a, n_pages, (hipStream_t)stream);
 }
 
 }  // namespace

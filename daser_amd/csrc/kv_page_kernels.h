@@ -1,5 +1,5 @@
-// kv_page_kernels.h -- page gather and scatter, one unit per workgroup and grouped
-// (several units per workgroup for small pages).
+// kv_page_kernels.h -- units of the grouped kernels (several units per workgroup
+// for small pages).
 // Part of libdaser_kv: included by kv_move.hip, one translation unit.
 
 #pragma once
@@ -7,99 +7,6 @@
 #include "kv_common.h"
 
 namespace {
-
-// Gather: one workgroup per (page, layer) unit, XCD-contiguous order. The
-// kSplit instance has a.parts consecutive workgroups share a unit, each
-// copying its part of both runs; it is a separate instance because the
-// split arithmetic cost 1.7% at 4 KiB pages.
-template <bool kSplit>
-__global__ __launch_bounds__(kThreads) void kv_gather_kernel(UnitArgs a) {
-  const int64_t w = xcd_unit(kSplit ? a.n_units * a.parts : a.n_units);
-  if (w < 0) return;
-  const int64_t u = kSplit ? udiv32(w, a.parts) : w;
-  const int64_t bytes = kSplit ? a.page_bytes / a.parts : a.page_bytes;
-  const int64_t part = kSplit ? bytes * (w - u * a.parts) : 0;
-  uint8_t *cache, *rec;
-  int l;
-  if (!unit_addresses(a, u, &cache, &rec, &l)) return;
-  copy_halves<kGatherUnroll>(cache + part, cache + a.kv_stride + part, rec + part,
-                             rec + a.page_bytes + part, bytes);
-}
-
-// Scatter: one workgroup per unit, layer-major per XCD (the host orders the
-// page list by destination block, which keeps each layer's page writes
-// near-sequential).
-__global__ __launch_bounds__(kThreads) void kv_scatter_kernel(UnitArgs a) {
-  uint8_t *cache, *rec;
-  int l;
-  const int64_t u = layer_major_unit(a.n_units, a.n_layers);
-  if (u < 0 || !unit_addresses(a, u, &cache, &rec, &l)) return;
-  copy_halves<kScatterUnroll>(rec, rec + a.page_bytes, cache, cache + a.kv_stride,
-                              a.page_bytes);
-}
-
-// Scatter of pages of 32 KiB and up (larger ones in 32 KiB parts),
-// launched at one workgroup per CU (the launch policy keeps about 64 KiB of
-// each CU's units in flight; see copy_wg_per_cu in kv_move.hip). Each lane keeps U (8 at 32 KiB)
-// vectors of K and of V in flight, and every store follows its own load's
-// arrival (no wait for the whole round): at one workgroup per CU the waves
-// stream instead of alternating a load burst with a store burst. Measured
-// in-process at the Llama-3-8B shape (32 KiB pages) on three boxes: 12.27 vs
-// 12.60 ms, 11.98 vs 12.08, 11.97 vs 12.09 for kv_scatter_kernel at its
-// register-limited 3 workgroups per CU; kv_scatter_kernel itself at one
-// workgroup per CU 12.54-12.56 ms. Units in hardware dispatch order
-// (kHwOrder): a further 3.5%. Pages above 32 KiB go as 32 KiB parts, one
-// workgroup each (kSplit): a workgroup's second round waits for its first
-// round's stores (vmcnt counts both), and parts measured 13% faster at 64
-// KiB pages (Llama-3-8B with block_size 32: 5.10 vs 5.75 ms). U = 4 serves 16 KiB
-// pages (e4m3) for measurements: at two workgroups per CU it measured
-// 23.0-23.6 ms at config 4 in three processes on one box against
-// 21.8-24.0 ms for kv_scatter_kernel, the spread being the buffers'
-// placement, so the default stays kv_scatter_kernel there.
-template <int U, bool kHwOrder, bool kSplit = false>
-__global__ __launch_bounds__(kThreads) void kv_scatter_stream_kernel(UnitArgs a) {
-  uint8_t *cache, *rec;
-  int l;
-  // kSplit: a.parts consecutive workgroups share a unit (pages above 32
-  // KiB: one round of U vectors per lane each), as consecutive units of the
-  // same order
-  const int64_t nw = kSplit ? a.n_units * a.parts : a.n_units;
-  const int64_t b = kHwOrder ? ((int64_t)blockIdx.x < nw ? (int64_t)blockIdx.x : -1)
-                             : xcd_unit(nw);
-  if (b < 0) return;
-  const int64_t v = kSplit ? udiv32(b, a.parts) : b;
-  const int64_t u = layer_major_of(v, a.n_units, a.n_layers);
-  if (!unit_addresses(a, u, &cache, &rec, &l)) return;
-  const int64_t pb = kSplit ? a.page_bytes / a.parts : a.page_bytes;
-  const int64_t part = kSplit ? pb * (b - v * a.parts) : 0;
-  const rsrc_t sk = make_rsrc(rec + part, pb), sv = make_rsrc(rec + a.page_bytes + part, pb);
-  const rsrc_t dk = make_rsrc(cache + part, pb), dv = make_rsrc(cache + a.kv_stride + part, pb);
-  const int nvec = (int)(pb >> 4);
-  for (int base = threadIdx.x; base < nvec; base += kThreads * U) {
-    u32x4 xk[U], xv[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      xk[k] = bload(sk, (base + k * kThreads) << 4);
-      xv[k] = bload(sv, (base + k * kThreads) << 4);
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      bstore(dk, (base + k * kThreads) << 4, xk[k]);
-      bstore(dv, (base + k * kThreads) << 4, xv[k]);
-    }
-  }
-}
-
-// Gather and scatter of head-major cache pages (records in token-major
-// order), one unit per workgroup, in the unit orders above.
-template <bool kGather>
-__global__ __launch_bounds__(kThreads) void kv_copy_hnd_kernel(UnitArgs a) {
-  uint8_t *cache, *rec;
-  int l;
-  const int64_t u = kGather ? xcd_unit(a.n_units) : layer_major_unit(a.n_units, a.n_layers);
-  if (u < 0 || !unit_addresses(a, u, &cache, &rec, &l)) return;
-  copy_halves_hnd<kHndUnroll, kGather>(a, cache, rec);
-}
 
 // ---------------------------------------------------------------------------
 // Small pages: several units per workgroup.
@@ -207,47 +114,6 @@ __device__ __forceinline__ int64_t group_start(const UnitArgs& a, int64_t g, int
     *p0 = v0 - (int64_t)*l0 * n_pages;
   }
   return a.n_units - v0 < G ? a.n_units - v0 : G;
-}
-
-// Gather (kGather: page-major, cache -> records) or scatter (layer-major,
-// records -> cache) over G units per workgroup. HND: head-major cache pages
-// (the cache side of each vector goes through hnd_vec).
-template <bool kGather, int U, bool HND = false>
-__global__ __launch_bounds__(kThreads) void kv_copy_grouped_kernel(UnitArgs a, int G) {
-  const int64_t g = xcd_unit(udiv32(a.n_units + G - 1, G));
-  if (g < 0) return;
-  const int64_t n_pages = udiv32(a.n_units, a.n_layers);
-  const int nvec = (int)(a.page_bytes >> 4);
-  int64_t p0;
-  int l0;
-  const int64_t n_here = group_start<kGather>(a, g, G, n_pages, &p0, &l0);
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-  const int lane = (int)threadIdx.x % kWave;
-  u32x4 rk[U], rv[U];
-  rsrc_t dk[U], dv[U];
-  int off[U], doff[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    const int fw = k * kThreads + wave * kWave;  // first flat vector of this wave
-    const int j = fw / nvec;
-    off[k] = (fw - j * nvec + lane) << 4;
-    const int coff = HND ? hnd_vec(a, off[k] >> 4) << 4 : off[k];  // cache side
-    const UnitRsrc u = unit_rsrc<kGather>(a, n_pages, p0, l0, j, n_here);
-    const uint8_t* src = kGather ? u.cache : u.rec;
-    const uint8_t* src_v = kGather ? u.cache + a.kv_stride : u.rec + a.page_bytes;
-    const uint8_t* dst = kGather ? u.rec : u.cache;
-    const uint8_t* dst_v = kGather ? u.rec + a.page_bytes : u.cache + a.kv_stride;
-    rk[k] = bload(make_rsrc(src, u.n), kGather ? coff : off[k]);
-    rv[k] = bload(make_rsrc(src_v, u.n), kGather ? coff : off[k]);
-    dk[k] = make_rsrc(dst, u.n);
-    dv[k] = make_rsrc(dst_v, u.n);
-    doff[k] = kGather ? off[k] : coff;
-  }
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    bstore(dk[k], doff[k], rk[k]);
-    bstore(dv[k], doff[k], rv[k]);
-  }
 }
 
 }  // namespace

@@ -71,19 +71,14 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  *   DSR_TUNE_SLOTS_KERNEL         1: rows of <= 8 vectors take the small-row
  *                                 kernel instead of the packed one
  *   DSR_TUNE_SLOTS_UNROLL         4|8 instructions per wave of the packed kernel
- *   DSR_TUNE_COPY_WG_PER_CU       workgroups per CU of the one-unit page
- *                                 gather / scatter
- *   DSR_TUNE_SCATTER_KERNEL       one-unit page scatter: 1 the load-all-then-
- *                                 store kernel, 2 the streaming kernel in
- *                                 hardware dispatch order, 3 the streaming
- *                                 kernel in per-XCD layer-major order
- *                                 (streaming: pages of 16 KiB multiples)
- *   DSR_TUNE_GATHER_SPLIT         workgroups per (page, layer) unit of a
- *                                 one-unit page gather (1: no split)
- *   DSR_TUNE_PAGE_PARTS           parts (one workgroup each) of a page in
- *                                 the one-unit gather and streaming scatter
- *                                 (1: whole pages; default: 32 KiB parts of
- *                                 larger pages)
+ *   DSR_TUNE_COPY_WG_PER_CU       workgroups per CU of the page gather / scatter
+ *   DSR_TUNE_COPY_STORES          (DSR_TUNE_SCATTER_KERNEL) store policy of the
+ *                                 page gather / scatter: 1 nt, else nt sc0 sc1
+ *   DSR_TUNE_COPY_PIECES          (DSR_TUNE_GATHER_SPLIT) 1 KiB pieces per wave
+ *                                 of the page gather / scatter: 8, else 1
+ *   DSR_TUNE_PAGE_PARTS           parts (one workgroup each) of a page in the
+ *                                 re-rotation (1: whole pages; default: 32 KiB
+ *                                 parts of larger pages)
  *   DSR_TUNE_SLOTS_ORDER          unit order of the large-row token scatters
  *                                 (plain and re-rotating): 1 per-XCD
  *                                 layer-major, 2 layer-major in hardware
@@ -104,7 +99,9 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
 #define DSR_TUNE_SLOTS_UNROLL 7
 #define DSR_TUNE_COPY_WG_PER_CU 8
 #define DSR_TUNE_SCATTER_KERNEL 9
+#define DSR_TUNE_COPY_STORES DSR_TUNE_SCATTER_KERNEL
 #define DSR_TUNE_GATHER_SPLIT 10
+#define DSR_TUNE_COPY_PIECES DSR_TUNE_GATHER_SPLIT
 #define DSR_TUNE_PAGE_PARTS 11
 #define DSR_TUNE_SLOTS_ORDER 12
 #define DSR_TUNE_SLOTS_WG_PER_CU 13

@@ -38,7 +38,7 @@ constexpr int kStoreNtSc = 19;
 // dsr_set_tuning() (0 = the geometry's own choice). Nothing reads the
 // environment: a serving process gets the defaults unless its code asks.
 // Relaxed atomics, read once per call.
-enum RotKernelOverride { kRotAuto = 0, kRotPairs = 1, kRotContig = 2, kRotGrouped = 3 };
+enum RotKernelOverride { kRotAuto = 0, kRotPairs = 1 };
 struct TuningKnobs {
   std::atomic<int64_t> v[DSR_TUNE_COUNT_];
 };
@@ -68,11 +68,6 @@ struct UnitArgs {
   int32_t hnd_heads = 0;
   int32_t hnd_block = 0;
   int32_t hnd_row_vecs = 0;
-  // Workgroups per unit of the one-unit gather and streaming scatter (1, or
-  // a count whose share of the page is a whole number of 4 KiB blocks):
-  // pages above 32 KiB, and launches with too few units to fill the chip,
-  // split each unit's two runs into equal parts.
-  int32_t parts = 1;
 };
 
 // Workgroup -> unit. Hardware deals consecutive workgroup ids round-robin
@@ -194,42 +189,6 @@ __device__ __forceinline__ void copy_halves(const uint8_t* src_k, const uint8_t*
       if (i < nvec) {
         bstore(dk, i << 4, rk[k]);
         bstore(dv, i << 4, rv[k]);
-      }
-    }
-  }
-}
-
-// copy_halves between a head-major cache page and its record: the record
-// side is walked lane-consecutively, the cache side through hnd_vec (whole
-// rows stay contiguous, so a row's lanes still coalesce). Vectors past the
-// page are skipped, as in copy_halves (issuing them against an empty range
-// cost 40% at 4 KiB pages).
-template <int U, bool kGather>
-__device__ __forceinline__ void copy_halves_hnd(const UnitArgs& a, uint8_t* cache,
-                                                uint8_t* rec) {
-  const int64_t pb = a.page_bytes;
-  const rsrc_t ck = make_rsrc(cache, pb), cv = make_rsrc(cache + a.kv_stride, pb);
-  const rsrc_t rk = make_rsrc(rec, pb), rv = make_rsrc(rec + pb, pb);
-  const int nvec = (int)(pb >> 4);
-  for (int base = threadIdx.x; base < nvec; base += kThreads * U) {
-    u32x4 xk[U], xv[U];
-    int ro[U], co[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = base + k * kThreads;
-      if (i < nvec) {
-        ro[k] = i << 4;
-        co[k] = hnd_vec(a, i) << 4;
-        xk[k] = bload(kGather ? ck : rk, kGather ? co[k] : ro[k]);
-        xv[k] = bload(kGather ? cv : rv, kGather ? co[k] : ro[k]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = base + k * kThreads;
-      if (i < nvec) {
-        bstore(kGather ? rk : ck, kGather ? ro[k] : co[k], xk[k]);
-        bstore(kGather ? rv : cv, kGather ? ro[k] : co[k], xv[k]);
       }
     }
   }

@@ -131,11 +131,11 @@ __global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa) {
         if (i >= nvec) continue;
         const int p = LAYOUT == kFanKx ? kx_phys(ra, i) : i;  // record-side vector
         const int o = LAYOUT == kFanHnd ? hnd_vec(a, i) : p;  // cache-side vector
+        const int c = k_column<LAYOUT == kFanKx>(ra, p);
+        const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
         bstore(kd, o << 4,
                ti < 0 ? kk.r[k]
-                      : rotate_vec<DT, STYLE>(ra, kk.r[k], q[k],
-                                              k_column<LAYOUT == kFanKx>(ra, p), tab, scale,
-                                              inv_scale));
+                      : rotate_vec<DT, STYLE>(ra, kk.r[k], q[k], c, tab + j0, scale, inv_scale));
       }
     }
   }

@@ -19,18 +19,16 @@
 // Kernel choice, by page and row geometry (all inside the entry points):
 //   gather / scatter, every page size, token-major and head-major:
 //     kv_flat_copy_kernel (1 KiB pieces, one per wave).
-//   re-rotation: kv_scatter_rerotate_grouped_kernel for pages below U * 4
-//     KiB and 16-bit pages of exactly U * 4 KiB (and 16-bit token-major pages
-//     of several such parts, one workgroup each); kv_scatter_rerotate_contig_
-//     kernel for other larger pages with a power-of-two partner distance;
-//     kv_scatter_rerotate_rows_kernel for other neox rows of <= 64 vectors;
-//     the pair-task kv_scatter_rerotate_kernel otherwise; rotary widths that
-//     are not whole 16-byte vectors: kv_scatter_rerotate_lds_kernel.
+//   re-rotation: kv_flat_rerotate_kernel (1 KiB pieces, or the whole rows in 64
+//     vectors) for gptj, for neox rows with a power-of-two partner distance
+//     and for other neox rows of <= 64 vectors; the pair-task
+//     kv_scatter_rerotate_kernel otherwise; rotary widths that are not whole
+//     16-byte vectors: kv_scatter_rerotate_lds_kernel.
 //   token form (dsr_gather_slots / dsr_scatter_slots): kv_slots_packed_kernel
 //     for power-of-two rows of <= 8 vectors, kv_slots_small_kernel for other
 //     rows of <= 32 vectors, kv_slots_kernel above.
-//   split-x K pages (dsr_scatter_rerotate_kx): the contig and grouped
-//     kernels with the KX flag, or the pair-task kernel.
+//   split-x K pages (dsr_scatter_rerotate_kx): the flat kernel with the
+//     split-x vector map, or the pair-task kernel.
 //   head-major cache pages (dsr_*_hnd): the same kernels as token-major
 //     pages of that size with the HND flag, whose cache-side offsets go
 //     through hnd_vec.
@@ -50,7 +48,6 @@
 #include "daser_kv.h"
 
 #include "kv_common.h"
-#include "kv_page_kernels.h"
 #include "kv_flat.h"
 #include "kv_rotate.h"
 #include "kv_slots.h"
@@ -129,9 +126,8 @@ int64_t items_per_launch(int n_layers, int64_t per_wg) {
 // the XCD count so that the XCD remap covers every unit. Returns the first
 // launch error.
 template <class F>
-int launch_page_ranges(const UnitArgs& a, int n_pages, int G, F launch) {
-  // a.parts workgroups per unit (the split kernels) count as a.parts units
-  const int64_t per = items_per_launch(a.n_layers * a.parts, G);
+int launch_page_ranges(const UnitArgs& a, int n_pages, F launch) {
+  const int64_t per = items_per_launch(a.n_layers, 1);
   if (per <= 0) return DSR_ERR_ARG;
   for (int64_t p0 = 0; p0 < n_pages; p0 += per) {
     const int64_t n = n_pages - p0 < per ? n_pages - p0 : per;
@@ -139,8 +135,7 @@ int launch_page_ranges(const UnitArgs& a, int n_pages, int G, F launch) {
     b.page_ids += p0;
     b.slot_offsets += p0;
     b.n_units = n * a.n_layers;
-    const unsigned grid =
-        (unsigned)(((b.n_units * a.parts + G - 1) / G + kXcds - 1) / kXcds * kXcds);
+    const unsigned grid = (unsigned)((b.n_units + kXcds - 1) / kXcds * kXcds);
     launch(b, grid);
     const int rc = (int)hipGetLastError();
     if (rc != 0) return rc;
@@ -174,35 +169,13 @@ int launch_flat(const UnitArgs& a, int64_t pieces_per_unit, int64_t minor, bool 
   return DSR_OK;
 }
 
-// Workgroups per CU for the re-rotation kernel, applied with dynamic LDS
-// sized from the CU's LDS capacity (the DSR_TUNE_ROT_WG_PER_CU override changes it, for
-// tuning). Measured in-process at the Llama-3-8B shapes: 16-bit K (64 KiB
-// per unit) runs best at 2-3 per CU (7.67 ms vs 7.87 ms at 4-8 and 11.0 ms
-// at 1); e4m3 (32 KiB per unit) at 4 per CU (24.17 ms; 24.4-24.5 ms at 6-12,
-// 30.1 ms at 2).
+// Workgroups per CU for the pair-task re-rotation kernel, applied with dynamic
+// LDS sized from the CU's LDS capacity: 16-bit K (64 KiB per unit at the
+// Llama-3-8B shape) ran best at 2-3 per CU, e4m3 (32 KiB) at 4.
 template <int DT>
 constexpr int rot_wg_per_cu() {
   return is_fp8<DT>() ? 4 : 2;
 }
-// The same for the grouped re-rotation kernel (pages below U * 4 KiB; env
-// DSR_ROT_GROUPED_WG_PER_CU overrides). Measured in-process at the
-// Llama-3-70B TP8 share: 16-bit K 6.97 ms at 4 per CU (7.41 at 2, 7.07 at
-// 8); e4m3 with 2 KiB pages 3.24 ms at 8 per CU (3.56 at 4), with 8 KiB
-// pages 12.96 ms at 8 (13.72 at 4).
-template <int DT>
-constexpr int rot_grouped_wg_per_cu() {
-  return is_fp8<DT>() ? 8 : 4;
-}
-// The grouped kernel with one unit per workgroup (16-bit pages of exactly
-// U * 4 KiB, the Llama-3-8B/70B shapes): 3 per CU. Measured in-process:
-// config 3 7.05 ms at 2-3 per CU, 7.36 at 4-5 (the contig kernel 7.68);
-// config 5 55.1 ms at 2-3, 50.4 at 4-6 (contig 55.4), where the shared
-// source chunks' reads hit the memory-side cache. 3 is taken for the
-// HBM-bound case, 4 when the caller flags shared records
-// (DSR_REROTATE_SHARED_RECORDS). e4m3 keeps the contig kernel (24.05 vs
-// 24.22 ms at config 4).
-constexpr int kRotSingleWgPerCu = 3;
-constexpr int kRotSingleSharedWgPerCu = 4;
 // Dynamic LDS that limits a kernel with `static_lds` bytes of static LDS to
 // wg_per_cu workgroups per CU on the current device (0 if the capacity cannot
 // be read). The capacity is read once per device.
@@ -224,9 +197,6 @@ size_t occupancy_lds(int wg_per_cu, int64_t static_lds) {
   const int64_t share = (int64_t)lds / wg_per_cu / kLdsGranule * kLdsGranule;
   const int64_t want = share - static_lds;
   return want > 0 ? (size_t)want : 0;
-}
-size_t rot_occupancy_lds(int wg_per_cu) {
-  return occupancy_lds(wg_per_cu, (int64_t)sizeof(float2) * kMaxRotHalf);
 }
 
 // Launch shape of a page copy, by the bytes it moves (read + written).
@@ -287,17 +257,65 @@ int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s) {
   });
 }
 
-constexpr int64_t kPartBytes = 32 << 10;
+
+// The pair-task kernel alone: the split-x K layout, whose rotation partners
+// are a whole block of vectors apart.
+template <int DT>
+int launch_rerotate_pairs(const RotArgs& ra, int n_pages, int style, hipStream_t s) {
+  const size_t dyn =
+      occupancy_lds(rot_wg_per_cu<DT>(), (int64_t)sizeof(float2) * kMaxRotHalf);
+  return launch_page_ranges(ra.u, n_pages, [&](const UnitArgs& b, unsigned grid) {
+    RotArgs rb = ra;
+    rb.u = b;
+    rb.rope_idx = ra.rope_idx + (b.page_ids - ra.u.page_ids);
+    if (style == DSR_ROPE_NEOX)
+      kv_scatter_rerotate_kernel<DT, DSR_ROPE_NEOX><<<grid, kThreads, dyn, s>>>(rb);
+    else
+      kv_scatter_rerotate_kernel<DT, DSR_ROPE_GPTJ><<<grid, kThreads, dyn, s>>>(rb);
+  });
+}
+
+// Workgroups per CU of the flat re-rotation: 6. A wave lives longer than a
+// copying one (its table, its rotation), so 4 keep too little in flight and 8
+// widen the written window: Llama-3-8B pages e4m3 5.73 / 5.87 / 5.74 TB/s at 4 / 6
+// / 8, Gemma-2-9B bf16 5.96 / 6.46 / 6.45, 70B TP8 bf16 5.99 / 6.13 / 5.84, 8B bf16 of
+// 2,900 pages 6.46 / 6.46 / 6.19.
+constexpr int kRotFlatWgPerCu = 6;
+
+template <int DT, int LAYOUT>
+int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_vecs,
+                         hipStream_t s) {
+  const CopyShape c = copy_shape(ra.u);
+  const int64_t nvec = ra.u.page_bytes >> 4;
+  const FastDiv row = fast_div((uint32_t)ra.row_vecs);
+  int wg = kRotFlatWgPerCu;
+  if (const int64_t t = tune(DSR_TUNE_ROT_WG_PER_CU)) wg = (int)t;
+  const int col = (is_fp8<DT>() ? 16 : 8) / (style == DSR_ROPE_NEOX ? 1 : 2);  // pairs
+  const size_t tabs = sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave);
+  const size_t lds = occupancy_lds(wg, 0);
+  const size_t dyn = lds > tabs ? lds : tabs;
+  return launch_flat(ra.u, (nvec + piece_vecs - 1) / piece_vecs, n_pages, c.chunked,
+                     [&](const FlatMap& m, unsigned grid) {
+#define DSR_ROT(STYLE, POLICY)                                                          \
+  kv_flat_rerotate_kernel<DT, STYLE, LAYOUT, POLICY><<<grid, kThreads, dyn, s>>>(ra, m, row, \
+                                                                                 piece_vecs)
+    if (style == DSR_ROPE_NEOX) {
+      if (c.nt) DSR_ROT(DSR_ROPE_NEOX, kStoreNt);
+      else DSR_ROT(DSR_ROPE_NEOX, kStoreNtSc);
+    } else {
+      if (c.nt) DSR_ROT(DSR_ROPE_GPTJ, kStoreNt);
+      else DSR_ROT(DSR_ROPE_GPTJ, kStoreNtSc);
+    }
+#undef DSR_ROT
+  });
+}
 
 template <int DT>
 int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipStream_t s,
-                    bool kx, unsigned flags, bool hnd = false) {
+                    int layout) {
   const int h = ra.half_vecs;
-  int wg = rot_wg_per_cu<DT>();
-  if (const int64_t t = tune(DSR_TUNE_ROT_WG_PER_CU)) wg = t > 0 ? (int)t : wg;
-  const int64_t rot_kernel = tune(DSR_TUNE_ROT_KERNEL);
   if (!vec_ok) {  // rotary width not in whole vectors: the LDS kernel
-    return launch_page_ranges(ra.u, n_pages, 1, [&](const UnitArgs& b, unsigned grid) {
+    return launch_page_ranges(ra.u, n_pages, [&](const UnitArgs& b, unsigned grid) {
       RotArgs rb = ra;
       rb.u = b;
       rb.rope_idx = ra.rope_idx + (b.page_ids - ra.u.page_ids);
@@ -307,122 +325,20 @@ int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipS
         kv_scatter_rerotate_lds_kernel<DT, DSR_ROPE_GPTJ><<<grid, kThreads, 0, s>>>(rb);
     });
   }
-  // split-x K (kx): the caller checked the kx_phys conditions, which make
-  // every neox partner lane ^ 32
-  const bool contig = kx || hnd || style == DSR_ROPE_GPTJ ||
+  // split-x K: the caller checked the kx_phys conditions, which make every
+  // neox partner lane ^ 32
+  if (layout == kRotKx) return launch_flat_rerotate<DT, kRotKx>(ra, n_pages, style, kWave, s);
+  if (layout == kRotHnd) return launch_flat_rerotate<DT, kRotHnd>(ra, n_pages, style, kWave, s);
+  const bool contig = style == DSR_ROPE_GPTJ ||
                       (h > 0 && h <= 32 && (h & (h - 1)) == 0 && ra.row_vecs % (2 * h) == 0);
-  const int G = contig ? units_per_group(ra.u.page_bytes, rot_contig_unroll<DT>(),
-                                         kMaxRotHalf / ra.rot_half)
-                       : 1;
-  // neox rows of <= 64 vectors whatever the partner distance: the row-aligned
-  // kernel (the DSR_TUNE_ROT_KERNEL override "pairs" keeps the pair-task kernel).
-  bool rows_ok = !contig && style == DSR_ROPE_NEOX && ra.row_vecs <= kWave && h > 0 &&
-                 2 * h <= ra.row_vecs;
-  if (rot_kernel == kRotPairs) rows_ok = false;
-  // The grouped kernel also serves pages of exactly U vectors per lane
-  // (G = 1), for 16-bit K. The DSR_TUNE_ROT_KERNEL override (contig, grouped) changes the
-  // choice where both apply, for in-process comparisons.
-  // 16-bit token-major pages above 32 KiB run the grouped kernel's single-
-  // unit path on 32 KiB parts, one workgroup each (the DSR_TUNE_PAGE_PARTS
-  // override 1 keeps whole pages on the contig kernel)
-  const int64_t part_vecs = (int64_t)rot_contig_unroll<DT>() * kThreads;
-  const int64_t row_bytes = (int64_t)ra.row_vecs * 16;
-  int parts = 1;
-  if (contig && !kx && !hnd && !is_fp8<DT>() && tune(DSR_TUNE_PAGE_PARTS) != 1 &&
-      (ra.u.page_bytes >> 4) > part_vecs && (ra.u.page_bytes >> 4) % part_vecs == 0 &&
-      (part_vecs * 16) % row_bytes == 0)
-    parts = (int)((ra.u.page_bytes >> 4) / part_vecs);
-  const int64_t nvec = (ra.u.page_bytes >> 4) / parts;
-  const bool single = contig && nvec % kThreads == 0 && nvec == part_vecs;
-  bool grouped = G > 1 || (single && !is_fp8<DT>());
-  if (rot_kernel == kRotContig && contig && parts == 1) grouped = false;
-  if (rot_kernel == kRotGrouped && (G > 1 || single)) grouped = true;
-  if (grouped) {
-    wg = G > 1 ? rot_grouped_wg_per_cu<DT>()
-         : (flags & DSR_REROTATE_SHARED_RECORDS) ? kRotSingleSharedWgPerCu
-                                                 : kRotSingleWgPerCu;
-    if (const int64_t t = tune(DSR_TUNE_ROT_GROUPED_WG_PER_CU)) wg = t > 0 ? (int)t : wg;
-  }
-  const size_t dyn = rot_occupancy_lds(wg);
-  // units per workgroup of the kernel actually launched: the one-unit
-  // kernels (an override may pick contig where G > 1) take one
-  const int GL = grouped ? G : 1;
-  UnitArgs ua = ra.u;
-  ua.parts = grouped ? parts : 1;
-  if (!grouped && !contig && rows_ok) {
-    // the row-aligned kernel on large pages: parts of whole rows near 32 KiB
-    const int64_t pbytes = ra.u.page_bytes;
-    int best = 1;
-    if (const int64_t t = tune(DSR_TUNE_PAGE_PARTS)) {
-      if (pbytes % t == 0 && (pbytes / t) % row_bytes == 0) best = (int)t;
-    } else if (pbytes > kPartBytes) {
-      int64_t bd = pbytes - kPartBytes;
-      for (int q = 2; q <= 8; ++q) {
-        const int64_t pt = pbytes / q;
-        if (pbytes % q || pt % row_bytes || pt < (16 << 10)) continue;
-        const int64_t d = pt > kPartBytes ? pt - kPartBytes : kPartBytes - pt;
-        if (d < bd) bd = d, best = q;
-      }
-    }
-    ua.parts = best;
-  }
-  return launch_page_ranges(ua, n_pages, GL, [&](const UnitArgs& b, unsigned grid) {
-    RotArgs rb = ra;
-    rb.u = b;
-    // one unit per workgroup over distinct records: the whole chip on one
-    // stretch of one layer, as the streaming scatter (config 3: 6.89-6.92 vs
-    // 7.04-7.05 ms on two boxes); several units per workgroup (8.1% slower
-    // at the TP8 share) and shared records (equal) keep the XCD order
-    rb.hw_order = grouped && GL == 1 && !(flags & DSR_SHARED_RECORDS);
-    rb.rope_idx = ra.rope_idx + (b.page_ids - ra.u.page_ids);
-    if (grouped) {
-      if (hnd && style == DSR_ROPE_NEOX)
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_NEOX, false, true><<<grid, kThreads, dyn, s>>>(rb, GL);
-      else if (hnd)
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_GPTJ, false, true><<<grid, kThreads, dyn, s>>>(rb, GL);
-      else if (style == DSR_ROPE_NEOX && kx)
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_NEOX, true><<<grid, kThreads, dyn, s>>>(rb, GL);
-      else if (style == DSR_ROPE_NEOX)
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_NEOX, false><<<grid, kThreads, dyn, s>>>(rb, GL);
-      else if (kx)
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_GPTJ, true><<<grid, kThreads, dyn, s>>>(rb, GL);
-      else
-        kv_scatter_rerotate_grouped_kernel<DT, DSR_ROPE_GPTJ, false><<<grid, kThreads, dyn, s>>>(rb, GL);
-    } else if (contig) {
-      if (hnd && style == DSR_ROPE_NEOX)
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_NEOX, false, true><<<grid, kThreads, dyn, s>>>(rb);
-      else if (hnd)
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_GPTJ, false, true><<<grid, kThreads, dyn, s>>>(rb);
-      else if (style == DSR_ROPE_NEOX && kx)
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_NEOX, true><<<grid, kThreads, dyn, s>>>(rb);
-      else if (style == DSR_ROPE_NEOX)
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_NEOX, false><<<grid, kThreads, dyn, s>>>(rb);
-      else if (kx)
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_GPTJ, true><<<grid, kThreads, dyn, s>>>(rb);
-      else
-        kv_scatter_rerotate_contig_kernel<DT, DSR_ROPE_GPTJ, false><<<grid, kThreads, dyn, s>>>(rb);
-    } else if (rows_ok) {
-      kv_scatter_rerotate_rows_kernel<DT><<<grid, kThreads, dyn, s>>>(rb);
-    } else {
-      kv_scatter_rerotate_kernel<DT, DSR_ROPE_NEOX><<<grid, kThreads, dyn, s>>>(rb);
-    }
-  });
-}
-
-// The pair-task kernel alone: the split-x K layout, whose rotation partners
-// are a whole block of vectors apart.
-template <int DT>
-int launch_rerotate_pairs(const RotArgs& ra, int n_pages, int style, hipStream_t s) {
-  const size_t dyn = rot_occupancy_lds(rot_wg_per_cu<DT>());
-  return launch_page_ranges(ra.u, n_pages, 1, [&](const UnitArgs& b, unsigned grid) {
-    RotArgs rb = ra;
-    rb.u = b;
-    rb.rope_idx = ra.rope_idx + (b.page_ids - ra.u.page_ids);
-    if (style == DSR_ROPE_NEOX)
-      kv_scatter_rerotate_kernel<DT, DSR_ROPE_NEOX><<<grid, kThreads, dyn, s>>>(rb);
-    else
-      kv_scatter_rerotate_kernel<DT, DSR_ROPE_GPTJ><<<grid, kThreads, dyn, s>>>(rb);
-  });
+  // other neox rows of <= 64 vectors: pieces of whole rows (the
+  // DSR_TUNE_ROT_KERNEL override "pairs" takes the pair-task kernel)
+  const bool rows = !contig && ra.row_vecs <= kWave && h > 0 && 2 * h <= ra.row_vecs &&
+                    tune(DSR_TUNE_ROT_KERNEL) != kRotPairs;
+  if (contig || rows)
+    return launch_flat_rerotate<DT, kRotNhd>(
+        ra, n_pages, style, contig ? kWave : kWave / ra.row_vecs * ra.row_vecs, s);
+  return launch_rerotate_pairs<DT>(ra, n_pages, style, s);
 }
 
 }  // namespace
@@ -594,17 +510,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
     ra.u.hnd_row_vecs = ra.row_vecs;
     switch (dtype) {
       case DSR_DTYPE_BF16:
-        return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, false, flags,
-                                               true);
+        return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, kRotHnd);
       case DSR_DTYPE_FP16:
-        return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, false, flags,
-                                               true);
+        return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, kRotHnd);
       case DSR_DTYPE_FP8_E4M3:
-        return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, false,
-                                                   flags, true);
+        return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, kRotHnd);
       default:
-        return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, false,
-                                                   flags, true);
+        return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, kRotHnd);
     }
   }
   if (kx_block > 0) {
@@ -622,13 +534,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
       ra.row_vecs = (int)hv;
       switch (dtype) {
         case DSR_DTYPE_BF16:
-          return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, true, flags);
+          return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, kRotKx);
         case DSR_DTYPE_FP16:
-          return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, true, flags);
+          return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, kRotKx);
         case DSR_DTYPE_FP8_E4M3:
-          return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, true, flags);
+          return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, kRotKx);
         default:
-          return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, true, flags);
+          return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, kRotKx);
       }
     }
     switch (dtype) {
@@ -644,13 +556,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
   }
   switch (dtype) {
     case DSR_DTYPE_BF16:
-      return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, vec_ok, s, false, flags);
+      return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
     case DSR_DTYPE_FP16:
-      return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, vec_ok, s, false, flags);
+      return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
     case DSR_DTYPE_FP8_E4M3:
-      return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, vec_ok, s, false, flags);
+      return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
     default:
-      return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, vec_ok, s, false, flags);
+      return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
   }
 }
 

@@ -1,10 +1,10 @@
-// kv_rotate.h -- element codecs and the re-rotation kernels (contiguous,
-// row-aligned, pair-task, element-wise LDS and grouped).
+// kv_rotate.h -- element codecs and the re-rotation kernels (flat, pair-task and
+// element-wise LDS).
 // Part of libdaser_kv: included by kv_move.hip, one translation unit.
 
 #pragma once
 
-#include "kv_page_kernels.h"
+#include "kv_flat.h"
 
 namespace {
 
@@ -25,11 +25,17 @@ __device__ __forceinline__ uint32_t f32_to_bf16(float f) {
 __device__ __forceinline__ float fp16_to_f32(uint32_t h) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
-// fp32 -> fp16 by the hardware conversion (round-to-nearest-even);
-// NaN -> 0x7E00.
+// fp32 -> fp16 by the hardware conversion (round-to-nearest-even), of the fp32
+// value itself: a multiply-add that the compiler fuses with the conversion
+// (v_fma_mixlo_f16) rounds otherwise, here and there by kernel.
+__device__ __forceinline__ uint32_t f32_bits_fp16(float f) {
+  asm("" : "+v"(f));
+  return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
+}
+// The same with NaN -> 0x7E00.
 __device__ __forceinline__ uint32_t f32_to_fp16(float f) {
   if (__builtin_isnan(f)) return 0x7e00u;
-  return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
+  return f32_bits_fp16(f);
 }
 
 // OCP e4m3fn (bias 7, no infinities, S.1111.111 = NaN) through the gfx950
@@ -100,6 +106,11 @@ constexpr bool is_fp8() {
   return DT == DSR_DTYPE_FP8_E4M3 || DT == DSR_DTYPE_FP8_E5M2;
 }
 
+// The codecs' quick encoders round by the hardware's conversion alone, and say
+// whether a result may need more (NaN, or a value outside the format): those
+// vectors go through encode. A rotated page holds next to none of them.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
 template <int DT>
 struct Codec;
 
@@ -120,6 +131,18 @@ struct Codec<DSR_DTYPE_BF16> {
       v[k] = f32_to_bf16(y[2 * k]) | (f32_to_bf16(y[2 * k + 1]) << 16);
     return v;
   }
+  static constexpr uint32_t kSigns = 0x80008000u;
+  __device__ static bool encode_quick(const float* y, u32x4* v) {
+    uint32_t odd = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x2 f = {y[2 * k], y[2 * k + 1]};
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+      odd |= (w & 0x7fff7fffu) + 0x007f007fu;  // past infinity: bit 15
+      (*v)[k] = w;
+    }
+    return odd & kSigns;
+  }
 };
 
 template <>
@@ -139,6 +162,17 @@ struct Codec<DSR_DTYPE_FP16> {
       v[k] = f32_to_fp16(y[2 * k]) | (f32_to_fp16(y[2 * k + 1]) << 16);
     return v;
   }
+  static constexpr uint32_t kSigns = 0x80008000u;
+  __device__ static bool encode_quick(const float* y, u32x4* v) {
+    uint32_t odd = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t w = f32_bits_fp16(y[2 * k]) | f32_bits_fp16(y[2 * k + 1]) << 16;
+      odd |= (w & 0x7fff7fffu) + 0x03ff03ffu;  // past infinity: bit 15
+      (*v)[k] = w;
+    }
+    return odd & kSigns;
+  }
 };
 
 template <>
@@ -154,6 +188,19 @@ struct Codec<DSR_DTYPE_FP8_E4M3> {
     for (int k = 0; k < 4; ++k) v[k] = f32x4_to_e4m3(y + 4 * k);
     return v;
   }
+  static constexpr uint32_t kSigns = 0x80808080u;
+  // without the clamp, values past +-464 encode as NaN too
+  __device__ static bool encode_quick(const float* y, u32x4* v) {
+    uint32_t odd = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      int e = __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * k], y[4 * k + 1], 0, false);
+      e = __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * k + 2], y[4 * k + 3], e, true);
+      odd |= ((uint32_t)e & 0x7f7f7f7fu) + 0x01010101u;  // 0x7F: bit 7
+      (*v)[k] = (uint32_t)e;
+    }
+    return odd & kSigns;
+  }
 };
 
 template <>
@@ -168,6 +215,19 @@ struct Codec<DSR_DTYPE_FP8_E5M2> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = f32x4_to_e5m2(y + 4 * k);
     return v;
+  }
+  static constexpr uint32_t kSigns = 0x80808080u;
+  // without the clamp, values past the largest finite one encode as infinity
+  __device__ static bool encode_quick(const float* y, u32x4* v) {
+    uint32_t odd = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      int e = __builtin_amdgcn_cvt_pk_bf8_f32(y[4 * k], y[4 * k + 1], 0, false);
+      e = __builtin_amdgcn_cvt_pk_bf8_f32(y[4 * k + 2], y[4 * k + 3], e, true);
+      odd |= ((uint32_t)e & 0x7c7c7c7cu) + 0x04040404u;  // exponent all ones: bit 7
+      (*v)[k] = (uint32_t)e;
+    }
+    return odd & kSigns;
   }
 };
 
@@ -191,15 +251,12 @@ struct RotArgs {
   // [head_dim / X][block_size][X] block and vector c holds dims
   // (c / block_size) * X ... + X - 1 of token c % block_size.
   int32_t col_div = 1;
-  // Contig and grouped kernels on split-x K pages (KX = true): head blocks
-  // of 2^kx_row_shift vectors, block_size 2^kx_bs_shift, neox partners
+  // Flat and fan-out kernels on split-x K pages: head blocks of
+  // 2^kx_row_shift vectors, block_size 2^kx_bs_shift, neox partners
   // kx_dist vectors apart (0 for gptj).
   int32_t kx_row_shift = 0;
   int32_t kx_bs_shift = 0;
   int32_t kx_dist = 0;
-  // Grouped kernel: walk its groups in hardware dispatch order (consecutive
-  // workgroups take consecutive groups) instead of XCD-contiguous eighths.
-  int32_t hw_order = 0;
 };
 
 // Split-x K: the lane-consecutive vector index i of a page -> the vector it
@@ -232,6 +289,72 @@ __device__ __forceinline__ int rope_table(const RotArgs& ra, int64_t p, int l) {
   if (!ra.layer_group) return ti;
   const int g = ra.layer_group[ra.u.layer0 + l];
   return g < 0 || g >= ra.n_groups ? -1 : g * ra.n_tables + ti;
+}
+
+// First table pair of a row's vector column c (neox: both halves of a row use
+// the first half's columns).
+template <int DT, int STYLE>
+__device__ __forceinline__ int table_column(const RotArgs& ra, int c) {
+  if (STYLE == DSR_ROPE_NEOX)
+    return (c < ra.half_vecs ? c : c - ra.half_vecs) * Codec<DT>::VE;
+  return c * (Codec<DT>::VE / 2);
+}
+
+// One K vector after rotation: c is its vector column in the row, own its
+// bytes, partner (neox) the bytes of the vector half a rotation away, cs the
+// pairs of its column. Vectors past the rotated region are returned unchanged.
+// kScaled: the values are multiplied by the layer's scale first and by its
+// inverse after. The sums are fused by name, so that every kernel rounds alike.
+template <int DT, int STYLE, bool kScaled>
+__device__ __forceinline__ u32x4 rotate_pairs(const RotArgs& ra, u32x4 own, u32x4 partner, int c,
+                                              const float2* cs, float scale, float inv_scale) {
+  using C = Codec<DT>;
+  constexpr int VE = C::VE;
+  float x[VE];
+  C::decode(own, x);
+  if (STYLE == DSR_ROPE_NEOX) {
+    // first half: x c - p s; second half: x c + p s. The sign goes into the
+    // partner's bits, which is exact.
+    const uint32_t flip = c < ra.half_vecs ? C::kSigns : 0u;
+    float z[VE];
+    C::decode(partner ^ flip, z);
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+      const float xo = kScaled ? x[e] * scale : x[e];
+      const float xp = kScaled ? z[e] * scale : z[e];
+      const float y = __builtin_fmaf(xp, cs[e].y, xo * cs[e].x);
+      x[e] = kScaled ? y * inv_scale : y;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < VE / 2; ++e) {
+      const float x1 = kScaled ? x[2 * e] * scale : x[2 * e];
+      const float x2 = kScaled ? x[2 * e + 1] * scale : x[2 * e + 1];
+      const float y1 = __builtin_fmaf(-x2, cs[e].y, x1 * cs[e].x);
+      const float y2 = __builtin_fmaf(x1, cs[e].y, x2 * cs[e].x);
+      x[2 * e] = kScaled ? y1 * inv_scale : y1;
+      x[2 * e + 1] = kScaled ? y2 * inv_scale : y2;
+    }
+  }
+  u32x4 v;
+  if (C::encode_quick(x, &v)) v = C::encode(x);
+  return c >= ra.rot_vecs ? own : v;
+}
+
+// The scale of an 8-bit layer cancels: R(s k) / s = R(k), with two roundings
+// less for each value. Scales whose inverse or products leave fp32's range
+// (zero, infinities, NaN among them) keep the multiplications and what they
+// give.
+__device__ __forceinline__ bool scale_cancels(float scale) {
+  const float m = __builtin_fabsf(scale);
+  return m >= 0x1p-100f && m <= 0x1p+100f;
+}
+template <int DT, int STYLE>
+__device__ __forceinline__ u32x4 rotate_vec(const RotArgs& ra, u32x4 own, u32x4 partner, int c,
+                                            const float2* cs, float scale, float inv_scale) {
+  if (is_fp8<DT>() && !scale_cancels(scale))
+    return rotate_pairs<DT, STYLE, true>(ra, own, partner, c, cs, scale, inv_scale);
+  return rotate_pairs<DT, STYLE, false>(ra, own, partner, c, cs, scale, inv_scale);
 }
 
 // K-page rotation in rounds of kRotUnroll tasks per lane. Task t covers row
@@ -278,47 +401,19 @@ struct KRound {
     }
   }
 
-  __device__ __forceinline__ void store(rsrc_t rd, const float2* tab, int half_off,
-                                        float scale, float inv_scale) {
-    using C = Codec<DT>;
-    constexpr bool kScaled = is_fp8<DT>();
+  __device__ __forceinline__ void store(const RotArgs& ra, rsrc_t rd, const float2* tab,
+                                        int half_off, float scale, float inv_scale) {
 #pragma unroll
     for (int k = 0; k < kRotUnroll; ++k) {
       if (kind[k] == 1) {
         bstore(rd, off[k], a[k]);
       } else if (kind[k] == 0) {
-        float x[VE];
-        C::decode(a[k], x);
-        if (STYLE == DSR_ROPE_NEOX) {
-          float z[VE];
-          C::decode(b[k], z);
-          const int j0 = c_of[k] * VE;
-#pragma unroll
-          for (int e = 0; e < VE; ++e) {
-            const float2 cs = tab[j0 + e];
-            const float x1 = kScaled ? x[e] * scale : x[e];
-            const float x2 = kScaled ? z[e] * scale : z[e];
-            const float y1 = x1 * cs.x - x2 * cs.y;
-            const float y2 = x2 * cs.x + x1 * cs.y;
-            x[e] = kScaled ? y1 * inv_scale : y1;
-            z[e] = kScaled ? y2 * inv_scale : y2;
-          }
-          bstore(rd, off[k], C::encode(x));
-          bstore(rd, off[k] + half_off, C::encode(z));
-        } else {
-          const int j0 = c_of[k] * (VE / 2);
-#pragma unroll
-          for (int e = 0; e < VE / 2; ++e) {
-            const float2 cs = tab[j0 + e];
-            const float x1 = kScaled ? x[2 * e] * scale : x[2 * e];
-            const float x2 = kScaled ? x[2 * e + 1] * scale : x[2 * e + 1];
-            const float y1 = x1 * cs.x - x2 * cs.y;
-            const float y2 = x2 * cs.x + x1 * cs.y;
-            x[2 * e] = kScaled ? y1 * inv_scale : y1;
-            x[2 * e + 1] = kScaled ? y2 * inv_scale : y2;
-          }
-          bstore(rd, off[k], C::encode(x));
-        }
+        const int c = c_of[k];
+        const float2* cs = tab + table_column<DT, STYLE>(ra, c);
+        bstore(rd, off[k], rotate_vec<DT, STYLE>(ra, a[k], b[k], c, cs, scale, inv_scale));
+        if (STYLE == DSR_ROPE_NEOX)
+          bstore(rd, off[k] + half_off,
+                 rotate_vec<DT, STYLE>(ra, b[k], a[k], c + ra.half_vecs, cs, scale, inv_scale));
       }
     }
   }
@@ -370,22 +465,13 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_kernel(RotArgs r
   __shared__ float2 tab[kMaxRotHalf];
   uint8_t *cache, *rec;
   int l;
-  // ra.u.parts consecutive workgroups share a unit (large pages), each
-  // moving a part of whole rows of both runs
-  const int parts = ra.u.parts;
-  const int64_t w = xcd_unit(ra.u.n_units * parts);
-  if (w < 0) return;
-  const int64_t vu = parts > 1 ? udiv32(w, parts) : w;
-  const int64_t u = layer_major_of(vu, ra.u.n_units, ra.u.n_layers);
-  if (!unit_addresses(ra.u, u, &cache, &rec, &l)) return;
+  const int64_t u = layer_major_unit(ra.u.n_units, ra.u.n_layers);
+  if (u < 0 || !unit_addresses(ra.u, u, &cache, &rec, &l)) return;
   const int64_t p = udiv32(u, ra.u.n_layers);
   const int ti = rope_table(ra, p, l);
-  const int64_t pb = ra.u.page_bytes / parts;
-  const int64_t po = pb * (w - vu * parts);
-  uint8_t* const vrec = rec + ra.u.page_bytes + po;
-  uint8_t* const vcache = cache + ra.u.kv_stride + po;
-  rec += po;
-  cache += po;
+  const int64_t pb = ra.u.page_bytes;
+  uint8_t* const vrec = rec + pb;
+  uint8_t* const vcache = cache + ra.u.kv_stride;
   if (ti < 0) {
     copy_halves<kRotCopyUnroll>(rec, vrec, cache, vcache, pb);
     return;
@@ -412,7 +498,7 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_kernel(RotArgs r
   __syncthreads();
 
   v.store(vd, threadIdx.x, nvec);
-  k.store(kd, tab, half_off, scale, inv_scale);
+  k.store(ra, kd, tab, half_off, scale, inv_scale);
   for (int base = threadIdx.x + kThreads * kScatterUnroll; base < nvec;
        base += kThreads * kScatterUnroll) {
     v.load(vs, base, nvec);
@@ -421,228 +507,86 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_kernel(RotArgs r
   for (int base = threadIdx.x + kThreads * kRotUnroll; base < ntask;
        base += kThreads * kRotUnroll) {
     k.load(ra, ks, base, ntask, row_bytes, half_off);
-    k.store(kd, tab, half_off, scale, inv_scale);
+    k.store(ra, kd, tab, half_off, scale, inv_scale);
   }
 }
 
-// One K vector after rotation: c is its vector column in the row, own its
-// bytes, partner (neox) the bytes of the vector half a rotation away.
-// Vectors past the rotated region are returned unchanged.
-template <int DT, int STYLE>
-__device__ __forceinline__ u32x4 rotate_vec(const RotArgs& ra, u32x4 own, u32x4 partner, int c,
-                                            const float2* tab, float scale, float inv_scale) {
-  using C = Codec<DT>;
-  constexpr int VE = C::VE;
-  constexpr bool kScaled = is_fp8<DT>();
-  if (c >= ra.rot_vecs) return own;
-  float x[VE];
-  C::decode(own, x);
-  if (STYLE == DSR_ROPE_NEOX) {
-    float z[VE];
-    C::decode(partner, z);
-    const bool first = c < ra.half_vecs;
-    const int j0 = (first ? c : c - ra.half_vecs) * VE;
-    const float sg = first ? -1.0f : 1.0f;
-#pragma unroll
-    for (int e = 0; e < VE; ++e) {
-      const float2 cs = tab[j0 + e];
-      const float xo = kScaled ? x[e] * scale : x[e];
-      const float xp = kScaled ? z[e] * scale : z[e];
-      // first half: x c - p s; second half: x c + p s
-      const float y = xo * cs.x + sg * (xp * cs.y);
-      x[e] = kScaled ? y * inv_scale : y;
-    }
-  } else {
-    const int j0 = c * (VE / 2);
-#pragma unroll
-    for (int e = 0; e < VE / 2; ++e) {
-      const float2 cs = tab[j0 + e];
-      const float x1 = kScaled ? x[2 * e] * scale : x[2 * e];
-      const float x2 = kScaled ? x[2 * e + 1] * scale : x[2 * e + 1];
-      const float y1 = x1 * cs.x - x2 * cs.y;
-      const float y2 = x2 * cs.x + x1 * cs.y;
-      x[2 * e] = kScaled ? y1 * inv_scale : y1;
-      x[2 * e + 1] = kScaled ? y2 * inv_scale : y2;
-    }
-  }
-  return C::encode(x);
-}
+// The re-rotation in the flat form (kv_flat.h): each wave moves one piece of
+// a unit, V as it is, K rotated, one 16-byte vector of each per lane. A piece
+// is 64 vectors where neox partners sit a power of two of at most 32 vectors
+// apart inside a row (and for gptj, whose pairs sit inside one vector), else
+// the whole rows that fit in 64 vectors (head_dim 80, 96, 192: 48 to 60 of the
+// 64 lanes), so that a vector's partner is always another lane of its wave.
+// The page's (cos, sin) table goes through the wave's own part of LDS: no
+// barrier, and a wave that copies leaves at once. In LDS every column of pairs
+// is followed by 16 bytes, so that the columns a wave reads start in different
+// banks (unpadded they are 64 or 128 bytes apart).
+// LAYOUT: token-major; split-x K (kx_phys on both sides, partners lane ^ 32);
+// head-major cache pages (records token-major, cache vector hnd_vec(i)).
+constexpr int kRotNhd = 0, kRotKx = 1, kRotHnd = 2;
 
-// Contiguous variant: lane-consecutive 16-byte vectors over the whole K page
-// (every load instruction of a wave covers 1 KiB of contiguous page), with
-// the neox partner vector fetched from lane ^ half_vecs by a cross-lane
-// shuffle. Valid when half_vecs is a power of two <= 32 dividing the row
-// evenly (rows then start on 2*half_vecs lane boundaries), and always for
-// gptj, whose pairs sit inside one vector.
-template <int DT, int STYLE, int U, bool KX, bool HND = false>
-__device__ __forceinline__ void rotate_contig_round(const RotArgs& ra, VRound<U>& kk,
-                                                    int base, int nvec, rsrc_t kd,
-                                                    const float2* tab, float scale,
-                                                    float inv_scale) {
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    const int i = base + k * kThreads;
-    u32x4 q = kk.r[k];
-    if (STYLE == DSR_ROPE_NEOX) {  // whole wave takes part in the shuffle
-      const int dist = KX ? 32 : ra.half_vecs;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) q[w] = (unsigned)__shfl_xor((int)kk.r[k][w], dist);
-    }
-    if (i >= nvec) continue;
-    // split-x: both sides move vector kx_phys(i); head-major: the record
-    // row order is token-major (the table column follows i), the cache's not
-    const int p = KX ? kx_phys(ra, i) : i;
-    bstore(kd, (HND ? hnd_vec(ra.u, i) : p) << 4,
-           rotate_vec<DT, STYLE>(ra, kk.r[k], q, k_column<KX>(ra, p), tab, scale, inv_scale));
-  }
-}
-
-// K and V vectors per lane per round: one round covers a 32 KiB bf16 or a
-// 16 KiB e4m3 Llama page.
-template <int DT>
-constexpr int rot_contig_unroll() {
-  return is_fp8<DT>() ? 4 : 8;
-}
-
-template <int DT, int STYLE, bool KX, bool HND = false>
-__global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_contig_kernel(RotArgs ra) {
-  __shared__ float2 tab[kMaxRotHalf];
-  uint8_t *cache, *rec;
-  int l;
-  const int64_t u = layer_major_unit(ra.u.n_units, ra.u.n_layers);
-  if (u < 0 || !unit_addresses(ra.u, u, &cache, &rec, &l)) return;
-  const int64_t p = udiv32(u, ra.u.n_layers);
-  const int ti = rope_table(ra, p, l);
-  const int64_t pb = ra.u.page_bytes;
-  if (ti < 0) {
-    if (HND)
-      copy_halves_hnd<kRotCopyUnroll, false>(ra.u, cache, rec);
-    else
-      copy_halves<kRotCopyUnroll>(rec, rec + pb, cache, cache + ra.u.kv_stride, pb);
-    return;
-  }
-  constexpr int U = rot_contig_unroll<DT>();
-  const rsrc_t ks = make_rsrc(rec, pb), kd = make_rsrc(cache, pb);
-  const rsrc_t vs = make_rsrc(rec + pb, pb), vd = make_rsrc(cache + ra.u.kv_stride, pb);
-  const int nvec = (int)(pb >> 4);
-  VRound<U> v, kk;
-  v.load(vs, threadIdx.x, nvec);
-  if (KX)
-    kk.load_kx(ra, ks, threadIdx.x, nvec);
-  else
-    kk.load(ks, threadIdx.x, nvec);
-  const float2* src_tab = ra.cos_sin + (int64_t)ti * ra.rot_half;
-  for (int j = threadIdx.x; j < ra.rot_half; j += kThreads) tab[j] = src_tab[j];
-  float scale = 1.0f, inv_scale = 1.0f;
-  if (is_fp8<DT>()) {
-    scale = ra.k_scale[ra.u.layer0 + l];
-    inv_scale = 1.0f / scale;
-  }
-  __syncthreads();
-  const int rounds = (nvec + kThreads * U - 1) / (kThreads * U);
-  for (int r = 0; r < rounds; ++r) {  // uniform trip count: shuffles stay converged
-    const int base = r * kThreads * U + threadIdx.x;
-    if (r > 0) {
-      v.load(vs, base, nvec);
-      if (KX)
-        kk.load_kx(ra, ks, base, nvec);
-      else
-        kk.load(ks, base, nvec);
-    }
-    if (HND)
-      v.store_hnd(ra.u, vd, base, nvec);
-    else
-      v.store(vd, base, nvec);
-    rotate_contig_round<DT, STYLE, U, KX, HND>(ra, kk, base, nvec, kd, tab, scale, inv_scale);
-  }
-}
-
-// neox rows whose partner distance is not a power of two (head_dim 80, 96,
-// 192, ...): each wave takes rpw = 64 / row_vecs whole rows (lanes past
-// rpw * row_vecs idle), so a vector's partner half a rotation away lies in
-// the same wave and comes from lane +- half_vecs by an arbitrary-lane
-// shuffle. Idle lanes and rows past the page get an offset beyond the
-// descriptor: their loads read 0 and their stores are dropped. One unit per
-// workgroup, layer-major; V is copied in flat rounds alongside. Replaced the
-// pair-task kernel for these shapes (3.5-4.2 TB/s, 35-45% behind a plain
-// scatter of the same pages).
-template <int DT>
-__global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_rows_kernel(RotArgs ra) {
-  constexpr int U = rot_contig_unroll<DT>();
-  __shared__ float2 tab[kMaxRotHalf];
-  uint8_t *cache, *rec;
-  int l;
-  // ra.u.parts consecutive workgroups share a unit (large pages), each
-  // moving a part of whole rows of both runs
-  const int parts = ra.u.parts;
-  const int64_t w = xcd_unit(ra.u.n_units * parts);
-  if (w < 0) return;
-  const int64_t vu = parts > 1 ? udiv32(w, parts) : w;
-  const int64_t u = layer_major_of(vu, ra.u.n_units, ra.u.n_layers);
-  if (!unit_addresses(ra.u, u, &cache, &rec, &l)) return;
-  const int64_t p = udiv32(u, ra.u.n_layers);
-  const int ti = rope_table(ra, p, l);
-  const int64_t pb = ra.u.page_bytes / parts;
-  const int64_t po = pb * (w - vu * parts);
-  uint8_t* const vrec = rec + ra.u.page_bytes + po;
-  uint8_t* const vcache = cache + ra.u.kv_stride + po;
-  rec += po;
-  cache += po;
-  if (ti < 0) {
-    copy_halves<kRotCopyUnroll>(rec, vrec, cache, vcache, pb);
-    return;
-  }
-  const rsrc_t ks = make_rsrc(rec, pb), kd = make_rsrc(cache, pb);
-  const rsrc_t vs = make_rsrc(vrec, pb), vd = make_rsrc(vcache, pb);
-  const int nvec = (int)(pb >> 4);
-  const int rv = ra.row_vecs;
-  const int rpw = kWave / rv;
-  const int rows = nvec / rv;
-  const int slots = (rows + rpw - 1) / rpw;  // wave-sized groups of rows
+template <int DT, int STYLE, int LAYOUT, int POLICY>
+__global__ __launch_bounds__(kThreads) void kv_flat_rerotate_kernel(RotArgs ra, FlatMap m,
+                                                                    FastDiv row, int piece_vecs) {
+  extern __shared__ float2 lds_tab[];
+  const UnitArgs& a = ra.u;
+  FlatPos u;
+  if (!flat_pos<false>(a, m, &u)) return;
   const int lane = (int)threadIdx.x % kWave;
-  const int wave = (int)threadIdx.x / kWave;
-  const int r_in = lane / rv;
-  const int c = lane - r_in * rv;
-  const int h = ra.half_vecs;
-  const int partner = c < h ? lane + h : c < 2 * h ? lane - h : lane;
-  const int waves = kThreads / kWave;
-  const int rounds_k = (slots + waves * U - 1) / (waves * U);
-  const int rounds_v = (nvec + kThreads * U - 1) / (kThreads * U);
-  const int rounds = rounds_k > rounds_v ? rounds_k : rounds_v;
-  auto k_off = [&](int r, int k) {
-    const int row = ((r * U + k) * waves + wave) * rpw + r_in;
-    return r_in < rpw && row < rows ? (row * rv + c) << 4 : (int)pb;
-  };
-  VRound<U> v;
-  u32x4 x[U];
-  v.load(vs, threadIdx.x, nvec);
-#pragma unroll
-  for (int k = 0; k < U; ++k) x[k] = bload(ks, k_off(0, k));
-  const float2* src_tab = ra.cos_sin + (int64_t)ti * ra.rot_half;
-  for (int j = threadIdx.x; j < ra.rot_half; j += kThreads) tab[j] = src_tab[j];
+  const int first = (int)u.part * piece_vecs;
+  const int nvec = (int)(a.page_bytes >> 4);
+  const int i = first + lane;
+  const bool whole = LAYOUT != kRotNhd;  // descriptors of the whole page
+  const int64_t po = whole ? 0 : (int64_t)first << 4;
+  const int64_t left = a.page_bytes - po;
+  const int64_t n = whole || left < ((int64_t)piece_vecs << 4) ? left : (int64_t)piece_vecs << 4;
+  const bool in = i < nvec && lane < piece_vecs;
+  const int out = (int)n;  // an offset outside the descriptors: reads 0, dropped
+  const int p = LAYOUT == kRotKx ? kx_phys(ra, i) : i;  // the K vector of the record
+  int kr = lane << 4, vr = kr, kc = kr, vc = kr;
+  if (whole) {
+    kr = in ? p << 4 : out;
+    vr = in ? i << 4 : out;
+    kc = LAYOUT == kRotHnd ? (in ? hnd_vec(a, i) << 4 : out) : kr;
+    vc = LAYOUT == kRotHnd ? kc : vr;
+  }
+  const u32x4 v = bload(make_rsrc(u.rec + po + a.page_bytes, n), vr);
+  const u32x4 k = bload(make_rsrc(u.rec + po, n), kr);
+  const rsrc_t kd = make_rsrc(u.cache + po, n), vd = make_rsrc(u.cache + po + a.kv_stride, n);
+  const int ti = rope_table(ra, u.page, u.layer);
+  if (ti < 0) {
+    bstore_as<POLICY>(vd, vc, v);
+    bstore_as<POLICY>(kd, kc, k);
+    return;
+  }
+  constexpr int kCol = STYLE == DSR_ROPE_NEOX ? Codec<DT>::VE : Codec<DT>::VE / 2;
+  float2* const tab = lds_tab + (threadIdx.x / kWave) * (ra.rot_half + ra.rot_half / kCol * 2);
+  const float2* const src_tab = ra.cos_sin + (int64_t)ti * ra.rot_half;
   float scale = 1.0f, inv_scale = 1.0f;
   if (is_fp8<DT>()) {
-    scale = ra.k_scale[ra.u.layer0 + l];
+    scale = ra.k_scale[a.layer0 + u.layer];
     inv_scale = 1.0f / scale;
   }
-  __syncthreads();
-  for (int r = 0; r < rounds; ++r) {  // uniform trip count: shuffles stay converged
-    const int base = r * kThreads * U + threadIdx.x;
-    if (r > 0) {
-      v.load(vs, base, nvec);
+  for (int j = lane; j < ra.rot_half; j += kWave) tab[j + j / kCol * 2] = src_tab[j];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  bstore_as<POLICY>(vd, vc, v);
+  int c;
+  if (LAYOUT == kRotKx)
+    c = k_column<true>(ra, p);
+  else
+    c = i - (int)(div_by((uint32_t)i, row) * row.d);
+  u32x4 q = k;
+  if (STYLE == DSR_ROPE_NEOX) {
+    const int h = ra.half_vecs;
+    const int from = LAYOUT == kRotKx ? lane ^ 32 : c < h ? lane + h : c < 2 * h ? lane - h : lane;
 #pragma unroll
-      for (int k = 0; k < U; ++k) x[k] = bload(ks, k_off(r, k));
-    }
-    v.store(vd, base, nvec);
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      u32x4 q;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) q[w] = (unsigned)__shfl((int)x[k][w], partner);
-      bstore(kd, k_off(r, k),
-             rotate_vec<DT, DSR_ROPE_NEOX>(ra, x[k], q, c, tab, scale, inv_scale));
-    }
+    for (int w = 0; w < 4; ++w) q[w] = (unsigned)__shfl((int)k[w], from);
   }
+  const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
+  bstore_as<POLICY>(kd, kc, rotate_vec<DT, STYLE>(ra, k, q, c, tab + j0 + j0 / kCol * 2, scale,
+                                                  inv_scale));
 }
 
 // Any even rot_dim and either style, for rotary widths that do not fill
@@ -672,22 +616,13 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_lds_kernel(RotAr
   __shared__ float2 tab[kMaxRotHalf];
   uint8_t *cache, *rec;
   int l;
-  // ra.u.parts consecutive workgroups share a unit (large pages), each
-  // moving a part of whole rows of both runs
-  const int parts = ra.u.parts;
-  const int64_t w = xcd_unit(ra.u.n_units * parts);
-  if (w < 0) return;
-  const int64_t vu = parts > 1 ? udiv32(w, parts) : w;
-  const int64_t u = layer_major_of(vu, ra.u.n_units, ra.u.n_layers);
-  if (!unit_addresses(ra.u, u, &cache, &rec, &l)) return;
+  const int64_t u = layer_major_unit(ra.u.n_units, ra.u.n_layers);
+  if (u < 0 || !unit_addresses(ra.u, u, &cache, &rec, &l)) return;
   const int64_t p = udiv32(u, ra.u.n_layers);
   const int ti = rope_table(ra, p, l);
-  const int64_t pb = ra.u.page_bytes / parts;
-  const int64_t po = pb * (w - vu * parts);
-  uint8_t* const vrec = rec + ra.u.page_bytes + po;
-  uint8_t* const vcache = cache + ra.u.kv_stride + po;
-  rec += po;
-  cache += po;
+  const int64_t pb = ra.u.page_bytes;
+  uint8_t* const vrec = rec + pb;
+  uint8_t* const vcache = cache + ra.u.kv_stride;
   if (ti < 0) {
     copy_halves<kRotCopyUnroll>(rec, vrec, cache, vcache, pb);
     return;
@@ -708,6 +643,7 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_lds_kernel(RotAr
   if (kScaled) {
     scale = ra.k_scale[ra.u.layer0 + l];
     inv_scale = 1.0f / scale;
+    if (scale_cancels(scale)) scale = inv_scale = 1.0f;
   }
   const uint32_t* bw = reinterpret_cast<const uint32_t*>(buf);
   const int rv = ra.row_vecs, half = ra.rot_half, rot = 2 * ra.rot_half;
@@ -745,89 +681,13 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_lds_kernel(RotAr
         const float2 cs = tab[jj];
         const float xo = kScaled ? x[e] * scale : x[e];
         const float xp = kScaled ? pv * scale : pv;
-        const float y = xo * cs.x + sg * (xp * cs.y);
+        const float y = __builtin_fmaf(sg * xp, cs.y, xo * cs.x);
         x[e] = kScaled ? y * inv_scale : y;
         mask[e / PER] |= ((1u << EB) - 1u) << (EB * (e % PER));
       }
       const u32x4 enc = C::encode(x);
       bstore(kd, (r0 * rv + i) << 4, (enc & mask) | (own & ~mask));
     }
-  }
-}
-
-// Re-rotation over G units per workgroup (layer-major order, as the one-unit
-// kernel). The group's (cos, sin) tables are staged in LDS, one rot_half
-// stretch per unit; G * rot_half <= kMaxRotHalf. K of an un-rotated unit is
-// stored as loaded.
-template <int DT, int STYLE, bool KX, bool HND = false>
-__global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_grouped_kernel(RotArgs ra,
-                                                                               int G) {
-  constexpr int U = rot_contig_unroll<DT>();
-  __shared__ float2 tab[kMaxRotHalf];
-  const UnitArgs& a = ra.u;
-  // a.parts > 1 (with G = 1, token-major pages): a.parts consecutive
-  // workgroups share a unit, each moving one part of its K and V runs
-  const int64_t ng = udiv32(a.n_units * a.parts + G - 1, G);
-  const int64_t gw = ra.hw_order ? ((int64_t)blockIdx.x < ng ? (int64_t)blockIdx.x : -1)
-                                 : xcd_unit(ng);
-  if (gw < 0) return;
-  const int64_t g = a.parts > 1 ? udiv32(gw, a.parts) : gw;
-  const int64_t pbytes = a.parts > 1 ? a.page_bytes / a.parts : a.page_bytes;
-  const int64_t pofs = a.parts > 1 ? pbytes * (gw - g * a.parts) : 0;
-  const int64_t n_pages = udiv32(a.n_units, a.n_layers);
-  const int nvec = (int)(pbytes >> 4);
-  int64_t p0;
-  int l0;
-  const int64_t n_here = group_start<false>(a, g, G, n_pages, &p0, &l0);
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-  const int lane = (int)threadIdx.x % kWave;
-  rsrc_t kd[U], vd[U];
-  u32x4 rk[U], rv[U];
-  int tj[U];    // LDS table slot of the vector's unit (-1: copy)
-  float sc[U];  // its layer's K scale (e4m3)
-  int off[U];
-  int koff[U];  // K: split-x pages move vector kx_phys(i) in lane slot i
-  int coff[U];  // cache-side offset of record vector i (head-major: hnd_vec)
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    const int fw = k * kThreads + wave * kWave;
-    const int j = fw / nvec;
-    off[k] = (fw - j * nvec + lane) << 4;
-    koff[k] = KX ? kx_phys(ra, off[k] >> 4) << 4 : off[k];
-    coff[k] = HND ? hnd_vec(a, off[k] >> 4) << 4 : koff[k];
-    const UnitRsrc u = unit_rsrc<false>(a, n_pages, p0, l0, j, n_here);
-    const int64_t un = u.n ? pbytes : 0;
-    rk[k] = bload(make_rsrc(u.rec + pofs, un), koff[k]);
-    rv[k] = bload(make_rsrc(u.rec + a.page_bytes + pofs, un), off[k]);
-    kd[k] = make_rsrc(u.cache + pofs, un);
-    vd[k] = make_rsrc(u.cache + a.kv_stride + pofs, un);
-    tj[k] = u.n && rope_table(ra, u.p, u.l) >= 0 ? j : -1;
-    sc[k] = is_fp8<DT>() && u.n ? ra.k_scale[a.layer0 + u.l] : 1.0f;
-  }
-  // tables of the group's units, fetched while the page loads are in flight
-  for (int e = threadIdx.x; e < (int)n_here * ra.rot_half; e += kThreads) {
-    const int jj = e / ra.rot_half;
-    int64_t p;
-    int l;
-    unit_at<false>(a, n_pages, p0, l0, jj, &p, &l);
-    const int ti = rope_table(ra, p, l);
-    if (ti >= 0) tab[e] = ra.cos_sin[(int64_t)ti * ra.rot_half + (e - jj * ra.rot_half)];
-  }
-#pragma unroll
-  for (int k = 0; k < U; ++k) bstore(vd[k], HND ? coff[k] : off[k], rv[k]);
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    u32x4 q = rk[k];
-    if (STYLE == DSR_ROPE_NEOX) {
-      const int dist = KX ? 32 : ra.half_vecs;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) q[x] = (unsigned)__shfl_xor((int)rk[k][x], dist);
-    }
-    const int t = tj[k] < 0 ? 0 : tj[k];
-    const u32x4 r = rotate_vec<DT, STYLE>(ra, rk[k], q, k_column<KX>(ra, koff[k] >> 4),
-                                          tab + t * ra.rot_half, sc[k], 1.0f / sc[k]);
-    bstore(kd[k], coff[k], tj[k] < 0 ? rk[k] : r);
   }
 }
 

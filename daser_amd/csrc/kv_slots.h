@@ -358,8 +358,10 @@ void kv_slots_rerotate_kernel(SlotArgs a, RotArgs ra) {
 #pragma unroll
           for (int x = 0; x < 4; ++x) q[x] = (unsigned)__shfl((int)xk[j][m][x], src);
         }
-        const u32x4 r = rotate_vec<DT, STYLE>(ra, xk[j][m], q, v & (hv - 1),
-                                              tab[wave * kTokPerWave + j], scale, inv_scale);
+        const int c = v & (hv - 1);
+        const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
+        const u32x4 r = rotate_vec<DT, STYLE>(ra, xk[j][m], q, c,
+                                              tab[wave * kTokPerWave + j] + j0, scale, inv_scale);
         bstore(ck[j], v << 4, ti[j] >= 0 ? r : xk[j][m]);
       }
     }

@@ -92,3 +92,94 @@ def test_flat_copy_launch_classes(gpu, n_pages, layers):
     assert torch.equal(staging, want) and torch.equal(single, want)
     sel = torch.from_numpy(ids).to(gpu)
     assert torch.equal(back[:, :, sel].view(torch.int16), whole[:, :, sel].view(torch.int16))
+
+
+@pytest.mark.parametrize("block,heads,dim,layout,rot,style", [
+    (16, 8, 128, "nhd", 128, "neox"), (16, 1, 128, "nhd", 64, "gptj"), (1, 1, 64, "nhd", 64, "neox"),
+    (16, 3, 96, "nhd", 96, "neox"), (5, 2, 80, "nhd", 80, "neox"), (16, 2, 192, "nhd", 192, "neox"),
+    (16, 2, 256, "nhd", 256, "neox"), (2, 1, 1024, "nhd", 64, "neox"), (7, 3, 64, "hnd", 32, "neox"),
+    (16, 4, 128, "kx", 128, "neox"), (16, 2, 64, "kx", 64, "gptj")])
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "e4m3", "e5m2"])
+@pytest.mark.parametrize("stores,max_wg", [(0, 0), (3, 24)])
+def test_flat_rerotate(gpu, tuning, block, heads, dim, layout, rot, style, dt, stores, max_wg):
+    """Rotated K within one rounding of float64 from the stored bits (the
+    8-bit formats with their layer's scale, one of them zero: NaN codes as by
+    multiplication), V and un-rotated pages unchanged; launches cut inside a
+    unit, both store policies."""
+    print(f"case: flat rotate bs{block} H{heads} D{dim} {layout} {rot} {style} {dt} {stores}",
+          flush=True)
+    tuning("scatter_kernel", stores)
+    tuning("max_wg_per_launch", max_wg)
+    dtype = {"bf16": torch.bfloat16, "fp16": torch.float16, "e4m3": torch.float8_e4m3fn,
+             "e5m2": torch.float8_e5m2}[dt]
+    fp8 = dt in ("e4m3", "e5m2")
+    esize = 1 if fp8 else 2
+    if layout == "hnd" and rot // 2 * esize % 16:
+        pytest.skip("HND pages take whole-vector rotary widths")
+    x_el = 16 // esize
+    if layout == "kx" and (rot // 2 % x_el if style == "neox" else rot % x_el):
+        pytest.skip("split-x pages take whole-vector rotary widths")
+    n, layers = 9, 3
+    g = torch.Generator(device=gpu).manual_seed(dim + rot)
+    rng = np.random.default_rng(dim)
+    logical = torch.randn((layers, n, 2, block, heads, dim), generator=g, device=gpu)
+    scales = torch.tensor([0.03, 1.7, 0.0], device=gpu)
+    stored = (logical * 20).to(dtype) if fp8 else logical.to(dtype)  # record order, token-major
+    recs = stored.clone()
+    if layout == "kx":  # records hold K split-x; V as it is
+        k = stored[:, :, 0].reshape(layers, n, block, heads, dim // x_el, x_el)
+        recs[:, :, 0] = k.permute(0, 1, 3, 4, 2, 5).reshape(layers, n, block, heads, dim)
+    staging = recs.transpose(0, 1).contiguous().view(-1).view(torch.uint8)
+    nb = n + 4
+    inner = {"nhd": (block, heads, dim), "hnd": (heads, block, dim),
+             "kx": (block * heads * dim,)}[layout]
+    whole = torch.zeros((layers, 2, nb, *inner), dtype=dtype, device=gpu)
+    views = [w.transpose(2, 3) if layout == "hnd" else w for w in whole.unbind(0)]
+    geo = dict(block_size=block, head_dim=dim) if layout == "kx" else {}
+    table = ops.LayerTable(views, **geo)
+    ids = rng.permutation(nb)[:n].astype(np.int64)
+    ridx = (np.arange(n) % 3 - 1).astype(np.int64)  # every third page keeps its K
+    ang = torch.rand((2, rot // 2), generator=g, device=gpu, dtype=torch.float64) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    ops.scatter_rerotate(table, ids, np.arange(n, dtype=np.int64) * table.layout.slot_bytes,
+                         staging, tabs, ridx, rot_dim=rot, style=style,
+                         k_scale=scales if fp8 else None)
+    torch.cuda.synchronize()
+    got = whole[:, :, torch.from_numpy(ids).to(gpu)].transpose(1, 2)  # [l, p, 2, ...]
+    if layout == "hnd":
+        got = got.transpose(3, 4)
+    elif layout == "kx":
+        kk = got[:, :, 0].reshape(layers, n, heads, dim // x_el, block, x_el)
+        kk = kk.permute(0, 1, 4, 2, 3, 5).reshape(layers, n, block, heads, dim)
+        got = torch.stack([kk.view(torch.uint8), got[:, :, 1].reshape(kk.shape).view(torch.uint8)],
+                          2).view(dtype)
+    else:
+        got = got.reshape(stored.shape)
+    as_bytes = lambda t: t.contiguous().view(torch.uint8)  # noqa: E731
+    assert torch.equal(as_bytes(got[:, :, 1]), as_bytes(stored[:, :, 1]))
+    keep = torch.from_numpy(ridx < 0).to(gpu)
+    assert torch.equal(as_bytes(got[:, keep]), as_bytes(stored[:, keep]))
+    moved = torch.from_numpy(np.nonzero(ridx >= 0)[0]).to(gpu)
+    t = tabs.double()[torch.from_numpy(ridx[ridx >= 0]).to(gpu)][None, :, None, None]
+    x = stored[:, moved, 0].double()
+    ref = x.clone()
+    lo, hi = (x[..., :rot // 2], x[..., rot // 2:rot]) if style == "neox" else \
+        (x[..., 0:rot:2], x[..., 1:rot:2])
+    a, b = lo * t[..., 0] - hi * t[..., 1], hi * t[..., 0] + lo * t[..., 1]
+    if style == "neox":
+        ref[..., :rot // 2], ref[..., rot // 2:rot] = a, b
+    else:
+        ref[..., 0:rot:2], ref[..., 1:rot:2] = a, b
+    top = {"e4m3": 448.0, "e5m2": 57344.0}.get(dt, float("inf"))
+    ref = ref.clamp(-top, top)
+    k = got[:, moved, 0].double()
+    if fp8:  # a zero scale: 0 * inf in every rotated value
+        assert torch.isnan(k[2][..., :rot]).all() and torch.equal(k[2][..., rot:], x[2][..., rot:])
+        k, ref, x = k[:2], ref[:2], x[:2]
+    # half a unit in the last place of the result, plus fp32's share of the inputs
+    mant, least = {"bf16": (8, 2.0 ** -133), "fp16": (11, 2.0 ** -24), "e4m3": (4, 2.0 ** -9),
+                   "e5m2": (3, 2.0 ** -16)}[dt]
+    ulp = torch.maximum(torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(1e-300))) + 1 - mant),
+                        torch.full_like(ref, least))
+    bound = 0.5 * ulp + x.abs().amax(-1, keepdim=True) * 2.0 ** -21
+    assert ((k - ref).abs() <= bound).all()

@@ -46,12 +46,13 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) {
 
 constexpr int kPiece = kWave * 16;  // bytes of one wave instruction
 
-// Consecutive workgroups of a large launch that stay on one XCD: 32 (128 KiB
+// Consecutive workgroups of a large launch that stay on one XCD: 128 (512 KiB
 // of K). Dealt one by one, every XCD translates every page's addresses and
 // the same page's lines meet in 8 L2s; in XCD-contiguous eighths, 8 windows
-// are written at once. Chunks of 32 were within 1-2% of the better of those two
-// everywhere and 1-4% ahead of both at 32 KiB pages.
-constexpr uint32_t kChunkLog2 = 5;
+// are written at once. Against chunks of 32, 128 were 0-1% ahead at 4 and 32 KiB
+// pages and 1-3% at 64 and 96 KiB ones and at 80 layers of e4m3; of 16, 1-6%;
+// of 1,024 and 16,384, 0-2%.
+constexpr uint32_t kChunkLog2 = 7;
 
 // The waves of one launch: wave w of it moves piece wave0 + w, counted from
 // the first piece of unit unit0.
@@ -70,19 +71,24 @@ struct FlatPos {
   uint32_t part;  // piece of the unit
 };
 
+// This wave's number in the launch, in the order of the chunks.
+__device__ __forceinline__ uint32_t flat_wave(const FlatMap& m) {
+  uint32_t b = blockIdx.x;
+  if (b < m.chunked) {
+    const uint32_t x = b % kXcds, j = b / kXcds;
+    b = (((j >> kChunkLog2) * kXcds + x) << kChunkLog2) + (j & ((1u << kChunkLog2) - 1));
+  }
+  return b * (kThreads / kWave) +
+         (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+}
+
 // This wave's piece; false past the end of the launch and where the unit's
 // block id or record range is out of bounds (it is then skipped). Page-major:
 // the records are written in sequence; layer-major: the destination-ordered
 // pages of one layer are. Everything here is uniform over the wave.
 template <bool kPageMajor>
 __device__ __forceinline__ bool flat_pos(const UnitArgs& a, const FlatMap& m, FlatPos* o) {
-  uint32_t b = blockIdx.x;
-  if (b < m.chunked) {
-    const uint32_t x = b % kXcds, j = b / kXcds;
-    b = (((j >> kChunkLog2) * kXcds + x) << kChunkLog2) + (j & ((1u << kChunkLog2) - 1));
-  }
-  const uint32_t w = b * (kThreads / kWave) +
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const uint32_t w = flat_wave(m);
   if (w >= m.n_waves) return false;
   const uint32_t g = m.wave0 + w;
   const uint32_t q = div_by(g, m.per_unit);

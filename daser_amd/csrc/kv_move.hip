@@ -24,9 +24,7 @@
 //     and for other neox rows of <= 64 vectors; the pair-task
 //     kv_scatter_rerotate_kernel otherwise; rotary widths that are not whole
 //     16-byte vectors: kv_scatter_rerotate_lds_kernel.
-//   token form (dsr_gather_slots / dsr_scatter_slots): kv_slots_packed_kernel
-//     for power-of-two rows of <= 8 vectors, kv_slots_small_kernel for other
-//     rows of <= 32 vectors, kv_slots_kernel above.
+//   token form (dsr_*_slots): the flat kernels over tokens (kv_slots.h).
 //   split-x K pages (dsr_scatter_rerotate_kx): the flat kernel with the
 //     split-x vector map, or the pair-task kernel.
 //   head-major cache pages (dsr_*_hnd): the same kernels as token-major
@@ -143,13 +141,13 @@ int launch_page_ranges(const UnitArgs& a, int n_pages, F launch) {
   return DSR_OK;
 }
 
-// Launches of a flat kernel over every piece of `a` (one launch unless the
-// workgroups exceed max_wg_per_launch()), `minor` the inner extent of its unit
-// order: launch(map, grid).
+// Launches of a flat kernel over every piece of n_units units (one launch
+// unless the workgroups exceed max_wg_per_launch()), `minor` the inner extent
+// of the unit order: launch(map, grid).
 template <class F>
-int launch_flat(const UnitArgs& a, int64_t pieces_per_unit, int64_t minor, bool chunked, F launch) {
+int launch_flat(int64_t n_units, int64_t pieces_per_unit, int64_t minor, bool chunked, F launch) {
   constexpr int kWaves = kThreads / kWave;
-  const int64_t total = a.n_units * pieces_per_unit;
+  const int64_t total = n_units * pieces_per_unit;
   const int64_t per = max_wg_per_launch() * kWaves;
   for (int64_t g0 = 0; g0 < total; g0 += per) {
     const int64_t n = total - g0 < per ? total - g0 : per;
@@ -240,7 +238,7 @@ int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s) {
   const int64_t pieces = c.whole ? a.page_bytes / (8 * kPiece) : (a.page_bytes + kPiece - 1) / kPiece;
   const int64_t t = tune(DSR_TUNE_COPY_WG_PER_CU);
   const size_t dyn = occupancy_lds(t ? (int)t : kCopyWgPerCu, 0);
-  return launch_flat(a, pieces, kGather ? a.n_layers : n_pages, c.chunked,
+  return launch_flat(a.n_units, pieces, kGather ? a.n_layers : n_pages, c.chunked,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_COPY(HND, POLICY, U) \
   kv_flat_copy_kernel<kGather, HND, POLICY, U><<<grid, kThreads, dyn, s>>>(a, m)
@@ -294,7 +292,7 @@ int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_ve
   const size_t tabs = sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave);
   const size_t lds = occupancy_lds(wg, 0);
   const size_t dyn = lds > tabs ? lds : tabs;
-  return launch_flat(ra.u, (nvec + piece_vecs - 1) / piece_vecs, n_pages, c.chunked,
+  return launch_flat(ra.u.n_units, (nvec + piece_vecs - 1) / piece_vecs, n_pages, c.chunked,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_ROT(STYLE, POLICY)                                                          \
   kv_flat_rerotate_kernel<DT, STYLE, LAYOUT, POLICY><<<grid, kThreads, dyn, s>>>(ra, m, row, \
@@ -684,14 +682,36 @@ int dsr_scatter_hnd(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
 
 namespace {
 
-// Unit order and workgroups per CU of the large-row token scatters
-// (kv_slots_kernel, kv_slots_rerotate_kernel); DSR_TUNE_SLOTS_ORDER (1 per-XCD
-// layer-major, 2 hardware dispatch order) and DSR_TUNE_SLOTS_WG_PER_CU
-// override them.
-bool slots_hw_order() { return tune(DSR_TUNE_SLOTS_ORDER) == 2; }
-int slots_wg_per_cu(int dflt) {
+// The token form's pieces: rows of 64 vectors and more are cut by themselves,
+// 16 tokens to a unit; of shorter rows a unit holds at least 256 vectors, one
+// workgroup's.
+struct SlotShape {
+  bool wide;
+  int64_t pieces;  // per unit
+  int64_t units;   // per layer
+};
+SlotShape slot_shape(SlotArgs* a) {
+  const int64_t vpr = a->row_bytes >> 4;
+  SlotShape h{vpr >= kWave, 0, 0};
+  a->unit_tokens = (int32_t)(vpr >= 16 ? 16 : 16 * ((16 + vpr - 1) / vpr));
+  const int64_t per_row = h.wide ? (vpr + kWave - 1) / kWave : vpr;
+  a->row = fast_div((uint32_t)per_row);
+  h.pieces = h.wide ? a->unit_tokens * per_row : (a->unit_tokens * vpr + kWave - 1) / kWave;
+  h.units = ((int64_t)a->n_tokens + a->unit_tokens - 1) / a->unit_tokens;
+  return h;
+}
+
+// Stores and order of a token-form launch, by the bytes it moves, as for the
+// page copies (copy_shape).
+bool slots_large(const SlotArgs& a) {
+  return 4 * a.row_bytes * a.n_tokens * a.n_layers > (200 << 20);
+}
+
+// Workgroups per CU: 6, wide rows' scatters 4 (8B bf16 rows 5.92 TB/s at 4, 5.78 at
+// 6; one-head e4m3 rows 5.78 at 4, 5.88 at 6, gathers 5.75 and 5.89).
+int slots_wg_per_cu(bool gather, bool wide) {
   const int64_t t = tune(DSR_TUNE_SLOTS_WG_PER_CU);
-  return t > 0 ? (int)t : dflt;
+  return t ? (int)t : wide && !gather ? 4 : 6;
 }
 
 int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t kv_stride,
@@ -710,24 +730,6 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   if (!aligned16(kv_stride) || !aligned16(page_stride) || !aligned16(page_bytes) ||
       !aligned16(row_bytes) || !aligned16(layer_bytes) || !aligned16p(staging))
     return DSR_ERR_ALIGN;
-  const int64_t vpr = row_bytes >> 4;
-  // Tokens per wave for small rows, measured in-process (ragged requests,
-  // 80 layers): 8 at 16-vector rows (4.34 ms gather vs 4.39 at 4 and 16),
-  // 4 at 32-vector rows (8.19 ms vs 8.35-8.45). 0: the large-row kernel.
-  int tpw = vpr <= 16 ? 8 : vpr <= 32 ? 4 : 0;
-  if (const int64_t t = tune(DSR_TUNE_SLOTS_TPW))  // override for small rows
-    if (tpw && (t == 4 || t == 8 || t == 16)) tpw = (int)t;
-  // power-of-two rows of <= 8 vectors: the packed kernel, U instructions
-  // per wave (4 and 8 measured alike; 16 spills)
-  int pk_u = vpr <= 8 && (vpr & (vpr - 1)) == 0 && (block_size & (block_size - 1)) == 0 ? 8 : 0;
-  if (tune(DSR_TUNE_SLOTS_KERNEL) == 1) pk_u = 0;
-  if (const int64_t t = tune(DSR_TUNE_SLOTS_UNROLL))
-    if (pk_u && (t == 4 || t == 8)) pk_u = (int)t;
-  const int pk_s = pk_u ? __builtin_ctzll((unsigned long long)vpr) : 0;
-  const int tok_wg = pk_u ? (kWave >> pk_s) * pk_u * (kThreads / kWave)
-                     : tpw ? tpw * (kThreads / kWave) : kTokPerWg;
-  const int64_t blocks = ((int64_t)n_tokens + tok_wg - 1) / tok_wg;
-  if (blocks * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   SlotArgs a{};
   a.layer_base = layer_base;
   a.kv_stride = kv_stride;
@@ -745,57 +747,24 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   a.layer0 = layer0;
   a.block_size = block_size;
   a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
-  hipStream_t s = (hipStream_t)stream;
-  // token ranges whose launches stay within max_wg_per_launch()
-  const int64_t per = items_per_launch(n_layers, tok_wg) / tok_wg * tok_wg;
-  if (per <= 0) return DSR_ERR_ARG;
-  for (int64_t t0 = 0; t0 < n_tokens; t0 += per) {
-    SlotArgs b = a;
-    b.slot_mapping += t0;
-    b.row_offsets += t0;
-    b.n_tokens = (int32_t)(n_tokens - t0 < per ? n_tokens - t0 : per);
-    const int64_t units = ((int64_t)b.n_tokens + tok_wg - 1) / tok_wg * n_layers;
-    const unsigned grid = (unsigned)(gather ? units : (units + kXcds - 1) / kXcds * kXcds);
-    if (pk_u == 8) {
-      if (gather)
-        kv_slots_packed_kernel<true, 8><<<grid, kThreads, 0, s>>>(b, pk_s);
-      else
-        kv_slots_packed_kernel<false, 8><<<grid, kThreads, 0, s>>>(b, pk_s);
-    } else if (pk_u == 4) {
-      if (gather)
-        kv_slots_packed_kernel<true, 4><<<grid, kThreads, 0, s>>>(b, pk_s);
-      else
-        kv_slots_packed_kernel<false, 4><<<grid, kThreads, 0, s>>>(b, pk_s);
-    } else if (tpw == 16) {
-      if (gather)
-        kv_slots_small_kernel<true, 16><<<grid, kThreads, 0, s>>>(b);
-      else
-        kv_slots_small_kernel<false, 16><<<grid, kThreads, 0, s>>>(b);
-    } else if (tpw == 8) {
-      if (gather)
-        kv_slots_small_kernel<true, 8><<<grid, kThreads, 0, s>>>(b);
-      else
-        kv_slots_small_kernel<false, 8><<<grid, kThreads, 0, s>>>(b);
-    } else if (tpw == 4) {
-      if (gather)
-        kv_slots_small_kernel<true, 4><<<grid, kThreads, 0, s>>>(b);
-      else
-        kv_slots_small_kernel<false, 4><<<grid, kThreads, 0, s>>>(b);
-    } else if (gather) {
-      kv_slots_kernel<true><<<grid, kThreads, occupancy_lds(3, 0), s>>>(b);
-    } else if (slots_hw_order()) {
-      kv_slots_kernel<false, true><<<grid, kThreads, occupancy_lds(slots_wg_per_cu(3), 0), s>>>(b);
-    } else {
-      kv_slots_kernel<false><<<grid, kThreads, occupancy_lds(slots_wg_per_cu(3), 0), s>>>(b);
-    }
-    const int rc = (int)hipGetLastError();
-    if (rc != 0) return rc;
-  }
-  return DSR_OK;
+  const SlotShape h = slot_shape(&a);
+  if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
+  const bool large = slots_large(a);
+  const hipStream_t s = (hipStream_t)stream;
+  const size_t dyn = occupancy_lds(slots_wg_per_cu(gather, h.wide), 0);
+  return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units, large,
+                     [&](const FlatMap& m, unsigned grid) {
+#define DSR_SLOTS(WIDE, POLICY)                                                              \
+  (gather ? kv_slots_flat_kernel<true, WIDE, POLICY><<<grid, kThreads, dyn, s>>>(a, m)       \
+          : kv_slots_flat_kernel<false, WIDE, POLICY><<<grid, kThreads, dyn, s>>>(a, m))
+    if (!h.wide) DSR_SLOTS(false, kStoreNt);
+    else if (large) DSR_SLOTS(true, kStoreNtSc);
+    else DSR_SLOTS(true, kStoreNt);
+#undef DSR_SLOTS
+  });
 }
 
-// Token-form scatter with re-rotation: argument checks, then
-// kv_slots_rerotate_kernel over token ranges that fit one launch each.
+// Token-form scatter with re-rotation: argument checks, then the flat kernel.
 int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
                           int64_t page_stride, int64_t page_bytes, int64_t num_blocks,
                           int block_size, int64_t row_bytes, const int64_t* slot_mapping,
@@ -832,8 +801,6 @@ int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_s
   if (!aligned16(kv_stride) || !aligned16(page_stride) || !aligned16(page_bytes) ||
       !aligned16(row_bytes) || !aligned16(layer_bytes) || !aligned16p(staging))
     return DSR_ERR_ALIGN;
-  const int64_t blocks = ((int64_t)n_tokens + kTokPerWg - 1) / kTokPerWg;
-  if (blocks * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   SlotArgs a{};
   a.layer_base = layer_base;
   a.kv_stride = kv_stride;
@@ -863,26 +830,27 @@ int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_s
   ra.rot_vecs = rot_dim * esize / 16;
   ra.half_vecs = rope_style == DSR_ROPE_NEOX ? rot_dim / 2 * esize / 16 : 0;
   ra.k_scale = k_scale;
-  hipStream_t s = (hipStream_t)stream;
-  const int64_t per = items_per_launch(n_layers, kTokPerWg) / kTokPerWg * kTokPerWg;
-  if (per <= 0) return DSR_ERR_ARG;
-  for (int64_t t0 = 0; t0 < n_tokens; t0 += per) {
-    SlotArgs b = a;
-    b.slot_mapping += t0;
-    b.row_offsets += t0;
-    b.n_tokens = (int32_t)(n_tokens - t0 < per ? n_tokens - t0 : per);
-    RotArgs rb = ra;
-    rb.rope_idx = rope_idx + t0;
-    const int64_t units = ((int64_t)b.n_tokens + kTokPerWg - 1) / kTokPerWg * n_layers;
-    const unsigned grid = (unsigned)((units + kXcds - 1) / kXcds * kXcds);
-    const size_t dyn =
-        occupancy_lds(slots_wg_per_cu(3), sizeof(float2) * kTokPerWg * kSlotRotMaxHalf);
-    const bool neox = rope_style == DSR_ROPE_NEOX, hw = slots_hw_order();
-#define DSR_SLOT_ROT(DT)                                                                      \
-  (hw ? (neox ? kv_slots_rerotate_kernel<DT, DSR_ROPE_NEOX, true><<<grid, kThreads, dyn, s>>>(b, rb) \
-              : kv_slots_rerotate_kernel<DT, DSR_ROPE_GPTJ, true><<<grid, kThreads, dyn, s>>>(b, rb)) \
-      : (neox ? kv_slots_rerotate_kernel<DT, DSR_ROPE_NEOX><<<grid, kThreads, dyn, s>>>(b, rb)       \
-              : kv_slots_rerotate_kernel<DT, DSR_ROPE_GPTJ><<<grid, kThreads, dyn, s>>>(b, rb)))
+  const SlotShape h = slot_shape(&a);
+  if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
+  const bool large = slots_large(a);
+  const hipStream_t s = (hipStream_t)stream;
+  const int64_t t = tune(DSR_TUNE_SLOTS_WG_PER_CU);
+  const int col = (esize == 1 ? 16 : 8) / (rope_style == DSR_ROPE_NEOX ? 1 : 2);  // pairs
+  const size_t tabs = sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave);
+  const size_t lds = occupancy_lds(t ? (int)t : kRotFlatWgPerCu, 0);
+  const size_t dyn = lds > tabs ? lds : tabs;
+  return launch_flat(h.units * n_layers, h.pieces, h.units, large,
+                     [&](const FlatMap& m, unsigned grid) {
+    const bool neox = rope_style == DSR_ROPE_NEOX;
+#define DSR_SLOT_ROT_P(DT, WIDE, POLICY)                                                     \
+  (neox ? kv_slots_flat_rerotate_kernel<DT, DSR_ROPE_NEOX, WIDE, POLICY>                     \
+          <<<grid, kThreads, dyn, s>>>(a, ra, m)                                             \
+        : kv_slots_flat_rerotate_kernel<DT, DSR_ROPE_GPTJ, WIDE, POLICY>                     \
+          <<<grid, kThreads, dyn, s>>>(a, ra, m))
+#define DSR_SLOT_ROT(DT)                                     \
+  (!h.wide ? DSR_SLOT_ROT_P(DT, false, kStoreNt)             \
+   : large ? DSR_SLOT_ROT_P(DT, true, kStoreNtSc)            \
+           : DSR_SLOT_ROT_P(DT, true, kStoreNt))
     switch (dtype) {
       case DSR_DTYPE_BF16: DSR_SLOT_ROT(DSR_DTYPE_BF16); break;
       case DSR_DTYPE_FP16: DSR_SLOT_ROT(DSR_DTYPE_FP16); break;
@@ -890,10 +858,8 @@ int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_s
       default: DSR_SLOT_ROT(DSR_DTYPE_FP8_E5M2); break;
     }
 #undef DSR_SLOT_ROT
-    const int rc = (int)hipGetLastError();
-    if (rc != 0) return rc;
-  }
-  return DSR_OK;
+#undef DSR_SLOT_ROT_P
+  });
 }
 
 }  // namespace

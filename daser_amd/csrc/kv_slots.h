@@ -1,15 +1,21 @@
 // kv_slots.h -- token-granular (slot_mapping-driven) gather and scatter.
 // Part of libdaser_kv: included by kv_move.hip, one translation unit.
+//
+// The flat form of the page kernels (kv_flat.h) over tokens: the unit is a run
+// of tokens of one layer, cut into pieces of one wave instruction. Rows of 64
+// vectors (1 KiB) and more are cut by themselves, so a wave's token is uniform,
+// its table entries come by scalar loads and its addresses go into buffer
+// descriptors. Shorter rows follow each other in the lanes, 64 vectors of
+// whatever tokens come next, each lane with its token's entries and its own
+// 64-bit addresses; every row length fills the wave. Invalid tokens (padding,
+// out-of-range slots or records) are left out.
 
 #pragma once
 
-#include "kv_common.h"
+#include "kv_flat.h"
 #include "kv_rotate.h"
 
 namespace {
-
-// ---------------------------------------------------------------------------
-// Token-granular (slot_mapping-driven) gather / scatter.
 
 struct SlotArgs {
   const uint64_t* layer_base;
@@ -28,6 +34,8 @@ struct SlotArgs {
   int32_t layer0;
   int32_t block_size;
   int32_t block_shift;  // log2(block_size) when a power of two, else -1
+  int32_t unit_tokens;  // tokens per unit
+  FastDiv row;          // wide rows: pieces per row; others: vectors per row
 };
 
 // Block of a non-negative slot: a shift for power-of-two block sizes (all
@@ -37,334 +45,159 @@ __device__ __forceinline__ int64_t slot_block(const SlotArgs& a, int64_t slot) {
   return slot < (int64_t)0xffffffffLL ? udiv32(slot, a.block_size) : slot / a.block_size;
 }
 
-constexpr int kTokPerWave = 4;  // tokens whose rows a wave has in flight at once
-constexpr int kTokPerWg = kTokPerWave * (kThreads / kWave);
-constexpr int kRowUnroll = 2;   // 64-vector slices of a row per round
+// One lane's (short rows) or wave's (wide rows) place: token t, vector v of
+// its row, the row's addresses.
+struct SlotPos {
+  uint8_t* cache;
+  uint8_t* rec;
+  int64_t t;
+  int layer;
+  int v;  // wide rows: first vector of the piece
+};
 
-// One workgroup per (16 consecutive tokens, layer); each wave owns 4 of the
-// tokens. Token addresses are wave-uniform (scalar loads of slot_mapping and
-// row_offsets); the lanes cover a row's 16-byte vectors, so a wave moves a
-// token's whole K and V rows, and 4 tokens' rows are in flight together.
-// Branch-free over the rows: a padding or out-of-range token goes through
-// zero-size descriptors (loads read 0, stores are dropped), and so do the
-// vectors past a row, so each store is issued as soon as its own load has
-// arrived (with a branch per vector the compiler waited for all 16 loads).
-// Launched with dynamic LDS sized for three workgroups per CU, the
-// registers' own limit: measured in-process at config 2, gather 12.04 ->
-// 11.58 ms and scatter 12.63 -> 12.38 ms against the branching kernel
-// without LDS (the branch-free kernel without LDS: 12.38 / 12.55; at one or
-// two workgroups per CU: 13.8-14.3 ms).
-template <bool kGather, bool kHwOrder = false>
-__global__ __launch_bounds__(kThreads) void kv_slots_kernel(SlotArgs a) {
-  // the scatter writes the paged cache: layer-major per XCD, as the page
-  // scatter (-2.4% in-process), or layer-major in hardware dispatch order
-  // (kHwOrder); the gather keeps the identity order
-  int64_t unit = blockIdx.x;
-  if (!kGather) {
-    const int64_t nu = ((int64_t)a.n_tokens + kTokPerWg - 1) / kTokPerWg * a.n_layers;
-    unit = kHwOrder ? layer_major_unit_hw(nu, a.n_layers) : layer_major_unit(nu, a.n_layers);
-    if (unit < 0) return;
+// False past the end of the launch or the unit and for invalid tokens. Gather:
+// the layers of a run of tokens follow each other (the records are written in
+// sequence); scatter: the runs of a layer.
+template <bool kGather, bool WIDE>
+__device__ __forceinline__ bool slot_pos(const SlotArgs& a, const FlatMap& m, SlotPos* o) {
+  const uint32_t w = flat_wave(m);
+  if (w >= m.n_waves) return false;
+  const uint32_t g = m.wave0 + w;
+  const uint32_t q = div_by(g, m.per_unit);
+  const uint32_t part = g - q * m.per_unit.d;
+  const uint32_t u = m.unit0 + q;
+  const uint32_t hi = div_by(u, m.minor);
+  const uint32_t lo = u - hi * m.minor.d;
+  const uint32_t tb = kGather ? hi : lo, l = kGather ? lo : hi;
+  uint32_t in_unit;
+  if (WIDE) {
+    in_unit = div_by(part, a.row);
+    o->v = (int)((part - in_unit * a.row.d) * kWave);
+  } else {
+    const uint32_t f = part * kWave + (uint32_t)threadIdx.x % kWave;
+    in_unit = div_by(f, a.row);
+    o->v = (int)(f - in_unit * a.row.d);
+    if (in_unit >= (uint32_t)a.unit_tokens) return false;
   }
-  const int64_t tb = udiv32(unit, a.n_layers);
-  const int l = (int)(unit - tb * a.n_layers);
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int vpr = (int)(a.row_bytes >> 4);
-  rsrc_t ck[kTokPerWave], cv[kTokPerWave], rk[kTokPerWave], rv[kTokPerWave];
-#pragma unroll
-  for (int j = 0; j < kTokPerWave; ++j) {
-    const int64_t t = tb * kTokPerWg + wave * kTokPerWave + j;
-    ck[j] = cv[j] = rk[j] = rv[j] = make_rsrc(a.staging, 0);
-    if (t < a.n_tokens) {
-      const int64_t slot = a.slot_mapping[t];
-      const int64_t blk = slot >= 0 ? slot_block(a, slot) : -1;
-      const int64_t off = a.row_offsets[t] + (int64_t)(a.layer0 + l) * a.layer_bytes;
-      if (blk >= 0 && blk < a.num_blocks && off >= 0 &&
-          off + a.page_bytes + a.row_bytes <= a.staging_bytes) {
-        const uint8_t* row = reinterpret_cast<const uint8_t*>(a.layer_base[l]) +
-                             blk * a.page_stride + (slot - blk * a.block_size) * a.row_bytes;
-        ck[j] = make_rsrc(row, a.row_bytes);
-        cv[j] = make_rsrc(row + a.kv_stride, a.row_bytes);
-        rk[j] = make_rsrc(a.staging + off, a.row_bytes);
-        rv[j] = make_rsrc(a.staging + off + a.page_bytes, a.row_bytes);
-      }
-    }
-  }
-  for (int vb = 0; vb < vpr; vb += kWave * kRowUnroll) {
-    u32x4 xk[kTokPerWave][kRowUnroll], xv[kTokPerWave][kRowUnroll];
-#pragma unroll
-    for (int j = 0; j < kTokPerWave; ++j) {
-#pragma unroll
-      for (int m = 0; m < kRowUnroll; ++m) {
-        const int v = vb + m * kWave + lane;
-        xk[j][m] = bload(kGather ? ck[j] : rk[j], v << 4);
-        xv[j][m] = bload(kGather ? cv[j] : rv[j], v << 4);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kTokPerWave; ++j) {
-#pragma unroll
-      for (int m = 0; m < kRowUnroll; ++m) {
-        const int v = vb + m * kWave + lane;
-        bstore(kGather ? rk[j] : ck[j], v << 4, xk[j][m]);
-        bstore(kGather ? rv[j] : cv[j], v << 4, xv[j][m]);
-      }
-    }
+  const int64_t t = (int64_t)tb * a.unit_tokens + in_unit;
+  if (t >= a.n_tokens) return false;
+  const int64_t slot = a.slot_mapping[t];
+  const int64_t off = a.row_offsets[t] + (int64_t)(a.layer0 + (int)l) * a.layer_bytes;
+  const int64_t blk = slot >= 0 ? slot_block(a, slot) : -1;
+  if (blk < 0 || blk >= a.num_blocks) return false;
+  if (off < 0 || off + a.page_bytes + a.row_bytes > a.staging_bytes) return false;
+  o->cache = reinterpret_cast<uint8_t*>(a.layer_base[l]) + blk * a.page_stride +
+             (slot - blk * a.block_size) * a.row_bytes;
+  o->rec = a.staging + off;
+  o->t = t;
+  o->layer = (int)l;
+  return true;
+}
+
+__device__ __forceinline__ u32x4 gload(const uint8_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+__device__ __forceinline__ void gstore(uint8_t* p, u32x4 v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+}
+
+template <bool kGather, bool WIDE, int POLICY>
+__global__ __launch_bounds__(kThreads) void kv_slots_flat_kernel(SlotArgs a, FlatMap m) {
+  SlotPos u;
+  if (!slot_pos<kGather, WIDE>(a, m, &u)) return;
+  const int64_t po = (int64_t)u.v << 4;
+  uint8_t* const src = (kGather ? u.cache : u.rec) + po;
+  uint8_t* const dst = (kGather ? u.rec : u.cache) + po;
+  const int64_t sv = kGather ? a.kv_stride : a.page_bytes;
+  const int64_t dv = kGather ? a.page_bytes : a.kv_stride;
+  if (WIDE) {
+    const int64_t left = a.row_bytes - po;
+    const int64_t n = left < kPiece ? left : kPiece;
+    const int o = ((int)threadIdx.x % kWave) << 4;
+    const u32x4 k = bload(make_rsrc(src, n), o), v = bload(make_rsrc(src + sv, n), o);
+    bstore_as<POLICY>(make_rsrc(dst, n), o, k);
+    bstore_as<POLICY>(make_rsrc(dst + dv, n), o, v);
+  } else {
+    const u32x4 k = gload(src), v = gload(src + sv);
+    gstore(dst, k);
+    gstore(dst + dv, v);
   }
 }
 
-// Rows of at most 32 vectors (512 B: one KV head at head_dim 128 bf16, or
-// two at head_dim 64). The kernel above resolves each token with dependent
-// scalar loads and a 64-bit division, and keeps 4 tokens per wave in flight
-// with a quarter or half of the lanes active: at one and two KV heads it
-// measured 1.9 and 3.5 TB/s, against 6.2 for the page kernels of the same
-// caches. Here lane j of a wave resolves the wave's token j (one vector load
-// of the tables for all of them, a shift for power-of-two block sizes) and
-// the wave reads each token's addresses back with readlane; TPW tokens' rows
-// are in flight per wave. Branch-free: an invalid token goes through
-// zero-size descriptors and lanes past the row end fall outside the
-// descriptor, so their loads read 0 and their stores are dropped. Measured
-// 5.3 (one head) and 5.7 TB/s (two heads) for the gather.
-template <bool kGather, int TPW>
-__global__ __launch_bounds__(kThreads) void kv_slots_small_kernel(SlotArgs a) {
-  constexpr int kTokWg = TPW * (kThreads / kWave);
-  int64_t unit = blockIdx.x;
-  if (!kGather) {
-    const int64_t nu = ((int64_t)a.n_tokens + kTokWg - 1) / kTokWg * a.n_layers;
-    unit = layer_major_unit(nu, a.n_layers);
-    if (unit < 0) return;
-  }
-  const int64_t tb = udiv32(unit, a.n_layers);
-  const int l = (int)(unit - tb * a.n_layers);
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-  const int lane = (int)threadIdx.x % kWave;
-  // Lane j < TPW resolves token j of the wave (one vector load of the
-  // tables for all of them); the wave then reads each token's addresses
-  // from its lane.
-  const int64_t t0 = tb * kTokWg + (int64_t)wave * TPW;
-  const int64_t t = t0 + lane;
-  const bool live = lane < TPW && t < a.n_tokens;
-  const int64_t slot = live ? a.slot_mapping[t] : -1;
-  const int64_t blk = slot < 0 ? -1 : slot_block(a, slot);
-  const int64_t in_blk = slot - blk * a.block_size;
-  const int64_t off = live ? a.row_offsets[t] + (int64_t)(a.layer0 + l) * a.layer_bytes : -1;
-  const bool ok = blk >= 0 && blk < a.num_blocks && off >= 0 &&
-                  off + a.page_bytes + a.row_bytes <= a.staging_bytes;
-  const uint64_t row = reinterpret_cast<uint64_t>(a.layer_base[l]) +
-                       (ok ? blk * a.page_stride + in_blk * a.row_bytes : 0);
-  const uint64_t rec = reinterpret_cast<uint64_t>(a.staging) + (ok ? off : 0);
-  const int n_lane = ok ? (int)a.row_bytes : 0;
-  rsrc_t dk[TPW], dv[TPW];
-  u32x4 xk[TPW], xv[TPW];
-#pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    const int n = __builtin_amdgcn_readlane(n_lane, j);
-    const uint8_t* rj = reinterpret_cast<const uint8_t*>(
-        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(row >> 32), j) << 32) |
-        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)row, j));
-    const uint8_t* cj = reinterpret_cast<const uint8_t*>(
-        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(rec >> 32), j) << 32) |
-        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rec, j));
-    const rsrc_t ck = make_rsrc(rj, n), cv = make_rsrc(rj + a.kv_stride, n);
-    const rsrc_t rk = make_rsrc(cj, n), rv = make_rsrc(cj + a.page_bytes, n);
-    xk[j] = bload(kGather ? ck : rk, lane << 4);
-    xv[j] = bload(kGather ? cv : rv, lane << 4);
-    dk[j] = kGather ? rk : ck;
-    dv[j] = kGather ? rv : cv;
-  }
-#pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    bstore(dk[j], lane << 4, xk[j]);
-    bstore(dv[j], lane << 4, xv[j]);
-  }
-}
-
-// Rows of 2^s <= 8 vectors (128 B: one e4m3 KV head of 128 dims, one bf16
-// head of 64), packed 64 >> s tokens to a wave instruction: lane = (token
-// sub-slot << s) | vector, so each load and store instruction moves a whole
-// KiB (a token's row is contiguous on both sides), where the kernel above
-// leaves 7/8 of its lanes idle on such rows. Measured on the e4m3 TP8 share
-// (80 layers, 1 KV head, 2 KiB pages), two boxes: 5.2-5.3 / 5.1-5.9 TB/s
-// gather / scatter against 3.6-3.8 / 3.5-3.7. At 16- and 32-vector rows it
-// measured equal or slower than the kernel above (5.1-5.6 vs 5.3-5.7 TB/s
-// gather), which keeps those. Each lane resolves
-// its own token (the 2^s lanes of a token read the same table entries) and
-// uses its own 64-bit global address; U instructions per wave are in flight
-// for K and for V. Invalid tokens' lanes are masked off. Block sizes are
-// powers of two here (vLLM's always are).
-template <bool kGather, int U>
-__global__ __launch_bounds__(kThreads, 4) void kv_slots_packed_kernel(SlotArgs a, int s) {
-  const int tpi = kWave >> s;
-  const int64_t tok_wg = (int64_t)tpi * U * (kThreads / kWave);
-  int64_t unit = blockIdx.x;
-  if (!kGather) {
-    const int64_t nu = ((int64_t)a.n_tokens + tok_wg - 1) / tok_wg * a.n_layers;
-    unit = layer_major_unit(nu, a.n_layers);
-    if (unit < 0) return;
-  }
-  const int64_t tb = udiv32(unit, a.n_layers);
-  const int l = (int)(unit - tb * a.n_layers);
-  const int wave = (int)threadIdx.x / kWave, lane = (int)threadIdx.x % kWave;
-  const int64_t vo = (int64_t)(lane & ((1 << s) - 1)) << 4;
-  const int64_t t0 = tb * tok_wg + (int64_t)wave * tpi * U + (lane >> s);
-  const uint8_t* base = reinterpret_cast<const uint8_t*>(a.layer_base[l]);
-  const int64_t lofs = (int64_t)(a.layer0 + l) * a.layer_bytes;
-  int64_t slot[U], roff[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) {  // every table load first
-    const int64_t t = t0 + (int64_t)k * tpi;
-    const bool live = t < a.n_tokens;
-    slot[k] = live ? a.slot_mapping[t] : -1;
-    roff[k] = live ? a.row_offsets[t] : -1;
-  }
-  const int64_t sv = kGather ? a.kv_stride : a.page_bytes;  // K -> V, source side
-  const int64_t dvs = kGather ? a.page_bytes : a.kv_stride;  // K -> V, destination side
-  const uint8_t* src[U];
-  uint8_t* dst[U];
-  bool ok[U];
-  u32x4 xk[U], xv[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    // power-of-two block sizes only (the launcher checks): a shift and a mask
-    const int64_t blk = slot[k] >> a.block_shift;  // -1 for padding slots
-    const int64_t off = roff[k] + lofs;
-    ok[k] = slot[k] >= 0 && blk < a.num_blocks && roff[k] >= 0 &&
-            off + a.page_bytes + a.row_bytes <= a.staging_bytes;
-    uint8_t* cache = const_cast<uint8_t*>(base) + blk * a.page_stride +
-                     (slot[k] & (a.block_size - 1)) * a.row_bytes + vo;
-    uint8_t* rec = a.staging + off + vo;
-    src[k] = kGather ? cache : rec;
-    dst[k] = kGather ? rec : cache;
-    if (ok[k]) {
-      xk[k] = *reinterpret_cast<const u32x4*>(src[k]);
-      xv[k] = *reinterpret_cast<const u32x4*>(src[k] + sv);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    if (ok[k]) {
-      *reinterpret_cast<u32x4*>(dst[k]) = xk[k];
-      *reinterpret_cast<u32x4*>(dst[k] + dvs) = xv[k];
-    }
-  }
-}
-
-// Token-form load scatter with the fused re-rotation: kv_slots_kernel's
-// scatter (16 tokens per workgroup, 4 per wave, lanes across the row,
-// branch-free) where the K vectors of a token with rope_idx[t] >= 0 go
-// through rotate_vec with that token's (cos, sin) table. Each wave stages
-// its own 4 tokens' tables in its slice of LDS with loads that write LDS
-// directly (no registers), issued before the rows; one wait for all of the
-// wave's loads then covers them. Heads are row_vecs (a power of two <= 64)
-// vectors, so a head never straddles a 64-vector slice of the row and its
-// neox partner sits half_vecs lanes away in the same load. At most 168
-// VGPRs keep 3 waves per SIMD.
+// The load scatter with K re-rotated by each token's own (cos, sin) table.
+// Heads are a power-of-two number of vectors (<= 64), so a head never leaves
+// its piece and its neox partner sits half_vecs lanes away. Where all tokens of
+// a wave use one table (always in wide rows, nearly always in a load of whole
+// chunks) it goes through the wave's part of LDS, as in the page kernel; other
+// lanes read their token's pairs themselves, 64 or 128 bytes for each 16 that
+// they move (one-head e4m3 rows: 2.9 TB/s, 4.2 through LDS). Lanes without a valid
+// token take part in the shuffles and move nothing.
 constexpr int kSlotRotMaxHalf = 128;  // rot_dim <= 256
-// s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima
-constexpr int kWaitVmcnt0 = 0x0F70;
 
-template <int DT, int STYLE, bool kHwOrder = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
-void kv_slots_rerotate_kernel(SlotArgs a, RotArgs ra) {
-  __shared__ float2 tab[kTokPerWg][kSlotRotMaxHalf];
-  const int64_t nu = ((int64_t)a.n_tokens + kTokPerWg - 1) / kTokPerWg * a.n_layers;
-  const int64_t unit =
-      kHwOrder ? layer_major_unit_hw(nu, a.n_layers) : layer_major_unit(nu, a.n_layers);
-  if (unit < 0) return;
-  const int64_t tb = udiv32(unit, a.n_layers);
-  const int l = (int)(unit - tb * a.n_layers);
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int vpr = (int)(a.row_bytes >> 4);
-  // layer l's group block of tables (-1: no RoPE in this layer)
-  int gbase = 0;
-  if (ra.layer_group) {
-    const int g = ra.layer_group[ra.u.layer0 + l];
-    gbase = g < 0 || g >= ra.n_groups ? -1 : g * ra.n_tables;
-  }
-  rsrc_t ck[kTokPerWave], cv[kTokPerWave], rk[kTokPerWave], rv[kTokPerWave];
-  int ti[kTokPerWave];
-#pragma unroll
-  for (int j = 0; j < kTokPerWave; ++j) {
-    const int64_t t = tb * kTokPerWg + wave * kTokPerWave + j;
-    ck[j] = cv[j] = rk[j] = rv[j] = make_rsrc(a.staging, 0);
-    ti[j] = -1;
-    if (t < a.n_tokens) {
-      const int64_t slot = a.slot_mapping[t];
-      const int64_t ro = a.row_offsets[t];
-      const int r = ra.rope_idx[t];
-      const int64_t blk = slot >= 0 ? slot_block(a, slot) : -1;
-      const int64_t off = ro + (int64_t)(a.layer0 + l) * a.layer_bytes;
-      if (blk >= 0 && blk < a.num_blocks && off >= 0 &&
-          off + a.page_bytes + a.row_bytes <= a.staging_bytes) {
-        const uint8_t* row = reinterpret_cast<const uint8_t*>(a.layer_base[l]) +
-                             blk * a.page_stride + (slot - blk * a.block_size) * a.row_bytes;
-        ck[j] = make_rsrc(row, a.row_bytes);
-        cv[j] = make_rsrc(row + a.kv_stride, a.row_bytes);
-        rk[j] = make_rsrc(a.staging + off, a.row_bytes);
-        rv[j] = make_rsrc(a.staging + off + a.page_bytes, a.row_bytes);
-        ti[j] = r < 0 || r >= ra.n_tables || gbase < 0 ? -1 : gbase + r;
-      }
+template <int DT, int STYLE, bool WIDE, int POLICY>
+__global__ __launch_bounds__(kThreads) void kv_slots_flat_rerotate_kernel(SlotArgs a, RotArgs ra,
+                                                                          FlatMap m) {
+  extern __shared__ float2 lds_tab[];
+  SlotPos u{};
+  const bool ok = slot_pos<false, WIDE>(a, m, &u);
+  if (WIDE && !ok) return;
+  const int lane = (int)threadIdx.x % kWave;
+  int ti = -1;
+  u32x4 k = {0u, 0u, 0u, 0u}, v = k;
+  uint8_t* dst = nullptr;
+  int64_t n = 0;
+  if (ok) {
+    const int64_t po = (int64_t)u.v << 4;
+    const uint8_t* const src = u.rec + po;
+    dst = u.cache + po;
+    if (WIDE) {
+      const int64_t left = a.row_bytes - po;
+      n = left < kPiece ? left : kPiece;
+      v = bload(make_rsrc(src + a.page_bytes, n), lane << 4);
+      k = bload(make_rsrc(src, n), lane << 4);
+    } else {
+      v = gload(src + a.page_bytes);
+      k = gload(src);
     }
-  }
-  // this wave's tables straight into its LDS slice (16 bytes = 2 pairs per
-  // lane: one load covers 128 pairs); zero-size descriptors for tokens that
-  // keep their K
-#pragma unroll
-  for (int j = 0; j < kTokPerWave; ++j) {
-    const uint8_t* tp = reinterpret_cast<const uint8_t*>(ra.cos_sin);
-    const rsrc_t tr = ti[j] >= 0 ? make_rsrc(tp + (int64_t)ti[j] * ra.rot_half * sizeof(float2),
-                                             ra.rot_half * (int64_t)sizeof(float2))
-                                 : make_rsrc(tp, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        tr, (__attribute__((address_space(3))) void*)&tab[wave * kTokPerWave + j][0], 16,
-        lane * 16, 0, 0, 0);
+    ti = rope_table(ra, u.t, u.layer);
   }
   float scale = 1.0f, inv_scale = 1.0f;
-  if (is_fp8<DT>()) {
-    scale = ra.k_scale[a.layer0 + l];
+  if (is_fp8<DT>() && ok) {
+    scale = ra.k_scale[a.layer0 + u.layer];
     inv_scale = 1.0f / scale;
   }
-  const int hv = ra.row_vecs;  // vectors per head
-  // 64-vector slices per round: fp8 rows of up to 1 KiB fit one
-  constexpr int RU = is_fp8<DT>() ? 1 : kRowUnroll;
-  for (int vb = 0; vb < vpr; vb += kWave * RU) {
-    u32x4 xk[kTokPerWave][RU], xv[kTokPerWave][RU];
+  constexpr int kCol = STYLE == DSR_ROPE_NEOX ? Codec<DT>::VE : Codec<DT>::VE / 2;
+  const int c = (WIDE ? lane : u.v) & (ra.row_vecs - 1);
+  const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
+  u32x4 q = k;
+  if (STYLE == DSR_ROPE_NEOX) {
+    const int from = c < ra.half_vecs ? lane + ra.half_vecs : lane - ra.half_vecs;
 #pragma unroll
-    for (int j = 0; j < kTokPerWave; ++j) {
-#pragma unroll
-      for (int m = 0; m < RU; ++m) {
-        const int v = vb + m * kWave + lane;
-        xk[j][m] = bload(rk[j], v << 4);
-        xv[j][m] = bload(rv[j], v << 4);
-      }
-    }
-    if (vb == 0) {  // the tables (loaded first) and this round's rows have landed
-      __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    for (int w = 0; w < 4; ++w) q[w] = (unsigned)__shfl((int)k[w], from);
+  }
+  const uint64_t valid = __ballot(ok);
+  if (valid == 0) return;
+  const int ti0 = __builtin_amdgcn_readlane(ti, __builtin_ctzll(valid));
+  if (WIDE || __ballot(ok && ti != ti0) == 0) {
+    if (ti0 >= 0) {
+      float2* const tab = lds_tab + (threadIdx.x / kWave) * (ra.rot_half + ra.rot_half / kCol * 2);
+      const float2* const src_tab = ra.cos_sin + (int64_t)ti0 * ra.rot_half;
+      for (int j = lane; j < ra.rot_half; j += kWave) tab[j + j / kCol * 2] = src_tab[j];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);  // no LDS read moves above the wait
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      k = rotate_vec<DT, STYLE>(ra, k, q, c, tab + j0 + j0 / kCol * 2, scale, inv_scale);
     }
-#pragma unroll
-    for (int j = 0; j < kTokPerWave; ++j)
-#pragma unroll
-      for (int m = 0; m < RU; ++m) bstore(cv[j], (vb + m * kWave + lane) << 4, xv[j][m]);
-#pragma unroll
-    for (int j = 0; j < kTokPerWave; ++j) {
-#pragma unroll
-      for (int m = 0; m < RU; ++m) {
-        const int v = vb + m * kWave + lane;
-        u32x4 q = xk[j][m];
-        if (STYLE == DSR_ROPE_NEOX) {  // the partner half_vecs away inside the same head
-          const int c = v & (hv - 1);
-          const int src = c < ra.half_vecs ? lane + ra.half_vecs : lane - ra.half_vecs;
-#pragma unroll
-          for (int x = 0; x < 4; ++x) q[x] = (unsigned)__shfl((int)xk[j][m][x], src);
-        }
-        const int c = v & (hv - 1);
-        const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
-        const u32x4 r = rotate_vec<DT, STYLE>(ra, xk[j][m], q, c,
-                                              tab[wave * kTokPerWave + j] + j0, scale, inv_scale);
-        bstore(ck[j], v << 4, ti[j] >= 0 ? r : xk[j][m]);
-      }
-    }
+  } else if (ti >= 0) {
+    k = rotate_vec<DT, STYLE>(ra, k, q, c, ra.cos_sin + (int64_t)ti * ra.rot_half + j0, scale,
+                              inv_scale);
+  }
+  if (WIDE) {
+    bstore_as<POLICY>(make_rsrc(dst + a.kv_stride, n), lane << 4, v);
+    bstore_as<POLICY>(make_rsrc(dst, n), lane << 4, k);
+  } else if (ok) {
+    gstore(dst + a.kv_stride, v);
+    gstore(dst, k);
   }
 }
 

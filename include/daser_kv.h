@@ -59,35 +59,21 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  * overrides them for measurements and tests only (results are the same
  * bytes); the library reads no environment variables. Knobs (value 0 = the
  * geometry's own choice):
- *   DSR_TUNE_UNITS_PER_GROUP      cap the (page, layer) units per workgroup
- *                                 of the small-page kernels (1: off)
  *   DSR_TUNE_MAX_WG_PER_LAUNCH    split calls into launches of <= n workgroups
- *   DSR_TUNE_ROT_KERNEL           re-rotation kernel where several apply:
- *                                 1 pairs, 2 contig, 3 grouped
- *   DSR_TUNE_ROT_WG_PER_CU, DSR_TUNE_ROT_GROUPED_WG_PER_CU
- *                                 re-rotation occupancy
- *   DSR_TUNE_SLOTS_TPW            4|8|16 tokens per wave of the small-row
- *                                 token kernels
- *   DSR_TUNE_SLOTS_KERNEL         1: rows of <= 8 vectors take the small-row
- *                                 kernel instead of the packed one
- *   DSR_TUNE_SLOTS_UNROLL         4|8 instructions per wave of the packed kernel
+ *   DSR_TUNE_ROT_KERNEL           1: the pair-task re-rotation kernel where
+ *                                 the flat one applies too
+ *   DSR_TUNE_ROT_WG_PER_CU        workgroups per CU of the re-rotation
  *   DSR_TUNE_COPY_WG_PER_CU       workgroups per CU of the page gather / scatter
  *   DSR_TUNE_COPY_STORES          (DSR_TUNE_SCATTER_KERNEL) store policy of the
  *                                 page gather / scatter: 1 nt, else nt sc0 sc1
  *   DSR_TUNE_COPY_PIECES          (DSR_TUNE_GATHER_SPLIT) 1 KiB pieces per wave
  *                                 of the page gather / scatter: 8, else 1
- *   DSR_TUNE_PAGE_PARTS           parts (one workgroup each) of a page in the
- *                                 re-rotation (1: whole pages; default: 32 KiB
- *                                 parts of larger pages)
- *   DSR_TUNE_SLOTS_ORDER          unit order of the large-row token scatters
- *                                 (plain and re-rotating): 1 per-XCD
- *                                 layer-major, 2 layer-major in hardware
- *                                 dispatch order
- *   DSR_TUNE_SLOTS_WG_PER_CU      workgroups per CU of those kernels
+ *   DSR_TUNE_SLOTS_WG_PER_CU      workgroups per CU of the token kernels
  *   DSR_TUNE_FANOUT_WG_PER_CU     workgroups per CU of dsr_scatter_fanout
  *   DSR_TUNE_FANOUT_PARTS         workgroups per (record, layer) unit of
  *                                 dsr_scatter_fanout (1, 2, 4: parts of
  *                                 whole rows)
+ * The other numbers have no effect; they keep the rest in their places.
  */
 #define DSR_TUNE_UNITS_PER_GROUP 0
 #define DSR_TUNE_MAX_WG_PER_LAUNCH 1

@@ -183,3 +183,70 @@ def test_flat_rerotate(gpu, tuning, block, heads, dim, layout, rot, style, dt, s
                         torch.full_like(ref, least))
     bound = 0.5 * ulp + x.abs().amax(-1, keepdim=True) * 2.0 ** -21
     assert ((k - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("heads,dim,dt", [(1, 64, "e4m3"), (1, 128, "bf16"), (3, 32, "bf16"),
+                                          (5, 128, "fp16"), (4, 128, "bf16"), (9, 128, "bf16"),
+                                          (2, 256, "e5m2")])
+@pytest.mark.parametrize("block,max_wg", [(16, 0), (6, 24)])
+def test_flat_slots(gpu, tuning, heads, dim, dt, block, max_wg):
+    """Token form on device tables, rows of 4 to 144 vectors: padding, slots
+    and records out of range, tokens of one wave with one table, several
+    and none; gathers and copies byte for byte, rotated tokens bit for bit as
+    the page form rotates them."""
+    print(f"case: flat slots H{heads} D{dim} {dt} bs{block} {max_wg}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    dtype = {"bf16": torch.bfloat16, "fp16": torch.float16, "e4m3": torch.float8_e4m3fn,
+             "e5m2": torch.float8_e5m2}[dt]
+    layers, n = 2, 7
+    nb = n + 2
+    g = torch.Generator(device=gpu).manual_seed(dim + heads)
+    rng = np.random.default_rng(heads)
+    whole = torch.randn((layers, 2, nb, block, heads, dim), generator=g, device=gpu).to(dtype)
+    table = ops.LayerTable(list(whole.unbind(0)))
+    lay = table.layout
+    row = heads * dim * lay.elem_bytes
+    ids = rng.permutation(nb)[:n]
+    tokens = n * block - 3
+    slots = ops.slot_mapping_for([ids], [tokens], block)
+    rows = ops.token_row_offsets([tokens], lay.slot_bytes, block, row)
+    drop = rng.random(tokens) < 0.2
+    slots[drop] = -1
+    slots[1], rows[2] = nb * block, n * lay.slot_bytes  # out of range
+    slots_d, rows_d = torch.from_numpy(slots).to(gpu), torch.from_numpy(rows).to(gpu)
+    ok = np.nonzero(~drop)[0]
+    ok = ok[(ok != 1) & (ok != 2)]
+    want = torch.zeros((n, layers, 2, block, heads, dim), dtype=dtype, device=gpu)
+    for t in ok:
+        want[t // block, :, :, t % block] = whole[:, :, int(ids[t // block]), t % block]
+    staging = torch.zeros(n * lay.slot_bytes, dtype=torch.uint8, device=gpu)
+    ops.gather_slots(table, slots_d, rows_d, staging)
+    torch.cuda.synchronize()
+    assert torch.equal(staging, want.view(-1).view(torch.uint8))
+    back = torch.zeros_like(whole)
+    ops.scatter_slots(ops.LayerTable(list(back.unbind(0))), slots_d, rows_d, staging)
+    ref = torch.zeros_like(whole)
+    for t in ok:
+        ref[:, :, int(ids[t // block]), t % block] = whole[:, :, int(ids[t // block]), t % block]
+    torch.cuda.synchronize()
+    assert torch.equal(back.view(torch.uint8), ref.view(torch.uint8))
+    if (dim * lay.elem_bytes // 16) & (dim * lay.elem_bytes // 16 - 1) or dim // 2 % (16 // lay.elem_bytes):
+        return
+    # rotated: runs of tokens with one table, then a table per token
+    ang = torch.rand((3, dim // 2), generator=g, device=gpu, dtype=torch.float64) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    scales = torch.tensor([0.5, 3.0], device=gpu) if lay.elem_bytes == 1 else None
+    ridx = np.where(np.arange(tokens) < 3 * block, 1, np.arange(tokens) % 4 - 1)
+    rot = torch.zeros_like(whole)
+    ops.scatter_slots_rerotate(ops.LayerTable(list(rot.unbind(0))), slots_d, rows_d, staging, tabs,
+                               torch.from_numpy(ridx.astype(np.int32)).to(gpu), k_scale=scales)
+    exp = torch.zeros_like(whole)
+    offs = np.arange(n, dtype=np.int64) * lay.slot_bytes
+    for r in (-1, 0, 1, 2):  # the page form with one table for every page
+        tmp = torch.zeros_like(whole)
+        ops.scatter_rerotate(ops.LayerTable(list(tmp.unbind(0))), ids, offs, staging, tabs,
+                             np.full(n, r), k_scale=scales)
+        for t in ok[ridx[ok] == r]:
+            exp[:, :, int(ids[t // block]), t % block] = tmp[:, :, int(ids[t // block]), t % block]
+    torch.cuda.synchronize()
+    assert torch.equal(rot.view(torch.uint8), exp.view(torch.uint8))

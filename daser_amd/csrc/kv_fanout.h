@@ -5,10 +5,10 @@
 //
 // The per-page scatter reads a shared record once per destination page, so a
 // chunk placed in 16 requests is read 16 times (partly from the memory-side
-// cache). Here the unit is one (source record, layer): the workgroup loads
-// the record's K and V pages into registers once, then for each destination
-// stores V as is and K rotated by that destination's delta table. Reads drop
-// to one pass over the distinct records; the writes are the same.
+// cache). Here a wave holds one piece (kv_flat.h) of a source's K and V of one
+// layer and writes it to each destination, V as is and K rotated by that
+// destination's delta table. Reads drop to one pass over the distinct records;
+// the writes are the same.
 
 #pragma once
 
@@ -23,120 +23,120 @@ struct FanArgs {
   const int32_t* dst_pages;    // block id of each destination
   const int32_t* dst_rope;     // table index of each destination (-1: K copied); null: no rotation
   int32_t n_src;
-  int32_t batch;  // destinations whose tables are staged in LDS at once
-  int32_t parts;  // workgroups per unit, each a 1/parts share of whole rows of the page
 };
 
-constexpr int kFanLdsFloat2 = 2048;  // 16 KiB of staged (cos, sin) pairs
-constexpr int kFanMaxBatch = 16;
-
-// One workgroup per (source, layer), source-major (a source's layers are
-// consecutive units) with each XCD taking one contiguous share of the units:
-// an XCD reads its sources' records front to back, and the chip's writes at
-// any moment spread over every layer's cache instead of one (config 5:
-// 28.1 ms against 33.5 ms layer-major in hardware order, 28.5 ms source-major
-// in hardware order). Pages of at most U * 4 KiB: the whole page sits in registers, U vectors per
-// lane of K and of V. K rotation as in the contig kernel (neox partner from
-// lane ^ half_vecs, fetched once per source since every destination rotates
-// the same stored vectors).
-// Cache layouts (LAYOUT): kFanNhd token-major pages; kFanKx split-x K pages
-// of vLLM's 3-D PagedAttention caches (K vector i of the record is physical
-// vector kx_phys(i) on both sides, neox partners lane ^ 32); kFanHnd
-// head-major pages (records token-major: cache vector hnd_vec(i) for K and V,
-// rotation columns in record order). kx and hnd units are whole pages.
-constexpr int kFanNhd = 0, kFanKx = 1, kFanHnd = 2;
-
-template <int DT, int STYLE, int U, int LAYOUT = kFanNhd>
-__global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa) {
-  __shared__ float2 tabs[kFanLdsFloat2];
-  __shared__ int32_t s_blk[kFanMaxBatch];
-  __shared__ int32_t s_ti[kFanMaxBatch];
+// A destination's table is fetched while the one before is being written (the
+// first 128 pairs; wider tables read the rest when they are needed). ROT false:
+// a plain copy. Cache layouts (LAYOUT) as in kv_flat_rerotate_kernel.
+template <int DT, int STYLE, int LAYOUT, bool ROT>
+__global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa, FlatMap m, FastDiv row,
+                                                             bool layer_major) {
+  extern __shared__ float2 lds_tab[];
   const RotArgs& ra = fa.ra;
   const UnitArgs& a = ra.u;
-  const int64_t w = xcd_unit(a.n_units * fa.parts);
-  if (w < 0) return;
-  // consecutive units take the parts of one (source, layer)
-  const uint32_t b = (uint32_t)w / (uint32_t)fa.parts;
-  const uint32_t part = (uint32_t)w - b * (uint32_t)fa.parts;
-  const uint32_t s = b / (uint32_t)a.n_layers;
-  const uint32_t l = b - s * (uint32_t)a.n_layers;
+  const uint32_t w = flat_wave(m);
+  if (w >= m.n_waves) return;
+  const uint32_t g = m.wave0 + w;
+  const uint32_t qu = div_by(g, m.per_unit);
+  const uint32_t part = g - qu * m.per_unit.d;
+  const uint32_t un = m.unit0 + qu;
+  const uint32_t hi = div_by(un, m.minor);
+  const uint32_t lo = un - hi * m.minor.d;
+  const uint32_t s = layer_major ? lo : hi, l = layer_major ? hi : lo;
   const int64_t off = fa.src_offsets[s] + (int64_t)(a.layer0 + (int)l) * a.layer_bytes;
   const int d0 = fa.dst_start[s], d1 = fa.dst_start[s + 1];
   if (off < 0 || off + 2 * a.page_bytes > a.staging_bytes || d1 <= d0) return;
-  const int64_t pb = a.page_bytes;
-  // this part: whole rows, so a vector's rotation column is its index
-  // modulo the row as in the whole page
-  const int64_t sb = pb / fa.parts;
-  const int64_t po = sb * part;
-  const uint8_t* rec = a.staging + off + po;
+  const int lane = (int)threadIdx.x % kWave;
+  const int first = (int)part * kWave;
+  const int nvec = (int)(a.page_bytes >> 4);
+  const int i = first + lane;
+  const bool whole = LAYOUT != kRotNhd;
+  const int64_t po = whole ? 0 : (int64_t)first << 4;
+  const int64_t left = a.page_bytes - po;
+  const int64_t n = whole || left < kPiece ? left : kPiece;
+  const bool in = i < nvec;
+  const int out = (int)n;
+  const int p = LAYOUT == kRotKx ? kx_phys(ra, i) : i;
+  int kr = lane << 4, vr = kr, kc = kr, vc = kr;
+  if (whole) {
+    kr = in ? p << 4 : out;
+    vr = in ? i << 4 : out;
+    kc = LAYOUT == kRotHnd ? (in ? hnd_vec(a, i) << 4 : out) : kr;
+    vc = LAYOUT == kRotHnd ? kc : vr;
+  }
+  const uint8_t* const rec = a.staging + off + po;
+  const u32x4 k = bload(make_rsrc(rec, n), kr);
+  const u32x4 v = bload(make_rsrc(rec + a.page_bytes, n), vr);
   uint8_t* const lbase = reinterpret_cast<uint8_t*>(a.layer_base[l]) + po;
-  const int nvec = (int)(sb >> 4);
-  VRound<U> v, kk;
-  v.load(make_rsrc(rec + pb, sb), threadIdx.x, nvec);
-  if (LAYOUT == kFanKx)
-    kk.load_kx(ra, make_rsrc(rec, sb), threadIdx.x, nvec);
-  else
-    kk.load(make_rsrc(rec, sb), threadIdx.x, nvec);
-  // this layer's table block, or no rotation at all
-  const int grp = ra.layer_group ? ra.layer_group[a.layer0 + (int)l] : 0;
-  const bool rot_layer = fa.dst_rope != nullptr && grp >= 0 && grp < ra.n_groups;
+  const int grp = ROT && ra.layer_group ? ra.layer_group[a.layer0 + (int)l] : 0;
+  const bool rot_layer = ROT && grp >= 0 && grp < ra.n_groups;
   float scale = 1.0f, inv_scale = 1.0f;
   if (is_fp8<DT>() && rot_layer) {
     scale = ra.k_scale[a.layer0 + (int)l];
     inv_scale = 1.0f / scale;
   }
-  u32x4 q[U];
+  constexpr int kCol = STYLE == DSR_ROPE_NEOX ? Codec<DT>::VE : Codec<DT>::VE / 2;
+  const int rh = ra.rot_half;
+  float2* const tab = lds_tab + (threadIdx.x / kWave) * (rh + rh / kCol * 2);
+  int c = 0, j0 = 0;
+  u32x4 q = k;
+  if (ROT) {
+    c = LAYOUT == kRotKx ? k_column<true>(ra, p) : i - (int)(div_by((uint32_t)i, row) * row.d);
+    j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
+    if (STYLE == DSR_ROPE_NEOX) {
+      const int from = LAYOUT == kRotKx ? lane ^ 32 : lane ^ ra.half_vecs;
 #pragma unroll
-  for (int k = 0; k < U; ++k) {
-    q[k] = kk.r[k];
-    if (STYLE == DSR_ROPE_NEOX && rot_layer) {  // uniform: the whole wave shuffles
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        q[k][c] = (unsigned)__shfl_xor((int)kk.r[k][c], LAYOUT == kFanKx ? 32 : ra.half_vecs);
+      for (int x = 0; x < 4; ++x) q[x] = (unsigned)__shfl((int)k[x], from);
     }
   }
-  const int rh = ra.rot_half;
-  for (int db = d0; db < d1; db += fa.batch) {
-    const int nb = d1 - db < fa.batch ? d1 - db : fa.batch;
-    __syncthreads();  // the previous batch's tables and ids are no longer read
-    if ((int)threadIdx.x < nb) {
-      const int d = db + (int)threadIdx.x;
-      s_blk[threadIdx.x] = fa.dst_pages[d];
-      const int ti = rot_layer ? fa.dst_rope[d] : -1;
-      s_ti[threadIdx.x] = ti >= 0 && ti < ra.n_tables ? grp * ra.n_tables + ti : -1;
+  // 64 destinations at a time: lane d holds the d-th one's block and table
+  for (int db = d0; db < d1; db += kWave) {
+    const int nb = d1 - db < kWave ? d1 - db : kWave;
+    const int my_blk = lane < nb ? fa.dst_pages[db + lane] : -1;
+    int my_ti = -1;
+    if (rot_layer && lane < nb) {
+      my_ti = fa.dst_rope[db + lane];
+      my_ti = my_ti >= 0 && my_ti < ra.n_tables ? grp * ra.n_tables + my_ti : -1;
     }
-    __syncthreads();
-    if (rot_layer) {
-      for (int j = threadIdx.x; j < nb * rh; j += kThreads) {
-        const int t = j / rh;
-        const int ti = s_ti[t];
-        tabs[j] = ti >= 0 ? ra.cos_sin[(int64_t)ti * rh + (j - t * rh)] : make_float2(1.0f, 0.0f);
+    float2 next[ROT ? 2 : 1];  // the next destination's table, this lane's pairs
+    auto fetch = [&](int t) {
+      const int ti = __builtin_amdgcn_readlane(my_ti, t);
+      if (ti >= 0) {
+        const float2* src = ra.cos_sin + (int64_t)ti * rh;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+          if (lane + x * kWave < rh) next[x] = src[lane + x * kWave];
       }
-      __syncthreads();
-    }
+    };
+    if (ROT) fetch(0);
     for (int t = 0; t < nb; ++t) {
-      const int64_t blk = s_blk[t];
+      const int64_t blk = __builtin_amdgcn_readlane(my_blk, t);
+      const int ti = ROT ? __builtin_amdgcn_readlane(my_ti, t) : -1;
+      u32x4 kk = k;
+      if (ROT) {
+        if (ti >= 0) {
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const int j = lane + x * kWave;
+            if (j < rh) tab[j + j / kCol * 2] = next[x];
+          }
+          for (int j = lane + 2 * kWave; j < rh; j += kWave)
+            tab[j + j / kCol * 2] = ra.cos_sin[(int64_t)ti * rh + j];
+        }
+        if (t + 1 < nb) fetch(t + 1);
+        if (ti >= 0) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          kk = rotate_vec<DT, STYLE>(ra, k, q, c, tab + j0 + j0 / kCol * 2, scale, inv_scale);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
       if (blk < 0 || blk >= a.num_blocks) continue;  // skipped, as by the page scatter
       uint8_t* const cache = lbase + blk * a.page_stride;
-      const rsrc_t kd = make_rsrc(cache, sb), vd = make_rsrc(cache + a.kv_stride, sb);
-      if (LAYOUT == kFanHnd)
-        v.store_hnd(a, vd, threadIdx.x, nvec);
-      else
-        v.store(vd, threadIdx.x, nvec);
-      const int ti = s_ti[t];
-      const float2* tab = tabs + t * rh;
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int i = (int)threadIdx.x + k * kThreads;
-        if (i >= nvec) continue;
-        const int p = LAYOUT == kFanKx ? kx_phys(ra, i) : i;  // record-side vector
-        const int o = LAYOUT == kFanHnd ? hnd_vec(a, i) : p;  // cache-side vector
-        const int c = k_column<LAYOUT == kFanKx>(ra, p);
-        const int j0 = c < ra.rot_vecs ? table_column<DT, STYLE>(ra, c) : 0;
-        bstore(kd, o << 4,
-               ti < 0 ? kk.r[k]
-                      : rotate_vec<DT, STYLE>(ra, kk.r[k], q[k], c, tab + j0, scale, inv_scale));
-      }
+      bstore_as<kStoreNtSc>(make_rsrc(cache + a.kv_stride, n), vc, v);
+      bstore_as<kStoreNtSc>(make_rsrc(cache, n), kc, kk);
     }
   }
 }

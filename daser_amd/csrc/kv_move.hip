@@ -1026,61 +1026,53 @@ int dsr_scatter_rerotate_static(const uint64_t* layer_base, int n_layers,
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// Loads of shared records (dsr_scatter_fanout): one workgroup per (source
-// record, layer), written to all of that record's destination pages.
+// Loads of shared records (dsr_scatter_fanout): each piece of a source record
+// read once and written to all of that record's destination pages.
 
 namespace {
 
-// Workgroups per CU of the fan-out kernel (DSR_TUNE_FANOUT_WG_PER_CU
-// overrides): pages of 16 KiB and up at 2 (config 5's 32 KiB pages measured
-// 33.58-33.64 ms from 2 to 8 per CU, 34.23 at 1), smaller ones at 8 (config
-// 6's 4 KiB pages: 4.53 ms at 8, 4.55 at 4, 4.74 at 2, 6.54 at 1).
-int fanout_wg_per_cu(int U) { return U >= 4 ? 2 : 8; }
+// Unit order and workgroups per CU of the fan-out, whose destinations lie
+// anywhere: that bounds it (5.0-5.3 TB/s where ordered pages take 6.4 or more).
+// Few sources: layer-major in dispatch order, 6 per CU; the chip then writes one
+// layer's pages, and every wave its source's in block order. From 512 sources
+// up that span (all of a layer's pages) is too wide, and source-major, 4 per CU,
+// in chunks of workgroups is ahead. Measured, per-unit workgroups -> layer-major
+// / source-major: 8B bf16, 256 sources 657 -> 585 / 609 us, 640 sources 2,420 ->
+// 2,320 / 2,327; 7B bf16, 640 sources 1,054 -> 1,083 / 1,033; 8B e4m3, 256 sources
+// 388 -> 288 / 308, 640 sources 1,421 -> 1,176 / 1,153; 70B bf16, 512 sources 4,806 ->
+// 4,703 / 4,657. DSR_TUNE_FANOUT_WG_PER_CU overrides the workgroups.
+constexpr int64_t kFanManySources = 512;
 
-template <int DT, int STYLE, int LAYOUT>
-int launch_fanout_u(FanArgs fa, int U, int64_t n_src, hipStream_t s) {
-  int wpc = fanout_wg_per_cu(U);
-  if (const int64_t t = tune(DSR_TUNE_FANOUT_WG_PER_CU)) wpc = (int)t;
-  const size_t dyn = occupancy_lds(
-      wpc, (int64_t)sizeof(float2) * kFanLdsFloat2 + 2 * sizeof(int32_t) * kFanMaxBatch);
-  // source ranges of at most max_wg_per_launch() workgroups each
-  // (one source's layers and parts always fit HIP's limit; a tuning limit
-  // below them still launches one source at a time)
-  int64_t per = (max_wg_per_launch() - kXcds) / (fa.ra.u.n_layers * fa.parts);
-  if (per <= 0) per = 1;
-  for (int64_t s0 = 0; s0 < n_src; s0 += per) {
-    FanArgs f = fa;
-    const int64_t n = n_src - s0 < per ? n_src - s0 : per;
-    f.src_offsets += s0;
-    f.dst_start += s0;
-    f.n_src = (int32_t)n;
-    f.ra.u.n_units = n * fa.ra.u.n_layers;
-    const unsigned grid = (unsigned)((f.ra.u.n_units * fa.parts + kXcds - 1) / kXcds * kXcds);
-    switch (U) {
-      case 1: kv_fanout_kernel<DT, STYLE, 1, LAYOUT><<<grid, kThreads, dyn, s>>>(f); break;
-      case 2: kv_fanout_kernel<DT, STYLE, 2, LAYOUT><<<grid, kThreads, dyn, s>>>(f); break;
-      case 4: kv_fanout_kernel<DT, STYLE, 4, LAYOUT><<<grid, kThreads, dyn, s>>>(f); break;
-      default: kv_fanout_kernel<DT, STYLE, 8, LAYOUT><<<grid, kThreads, dyn, s>>>(f); break;
-    }
-    const int rc = (int)hipGetLastError();
-    if (rc != 0) return rc;
-  }
-  return DSR_OK;
+template <int DT, int STYLE, int LAYOUT, bool ROT>
+int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
+  const RotArgs& ra = fa.ra;
+  const int col = (is_fp8<DT>() ? 16 : 8) / (STYLE == DSR_ROPE_NEOX ? 1 : 2);  // pairs
+  const size_t tabs =
+      ROT ? sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave) : 0;
+  const bool many = fa.n_src >= kFanManySources;
+  const int64_t t = tune(DSR_TUNE_FANOUT_WG_PER_CU);
+  const size_t lds = occupancy_lds(t ? (int)t : many ? 4 : 6, 0);
+  const size_t dyn = lds > tabs ? lds : tabs;
+  const FastDiv row = fast_div((uint32_t)(ROT ? ra.row_vecs : 1));
+  return launch_flat((int64_t)fa.n_src * ra.u.n_layers, (ra.u.page_bytes + kPiece - 1) / kPiece,
+                     many ? ra.u.n_layers : fa.n_src, many, [&](const FlatMap& m, unsigned grid) {
+    kv_fanout_kernel<DT, STYLE, LAYOUT, ROT><<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
+  });
 }
 
 template <int DT, int LAYOUT>
-int launch_fanout_l(const FanArgs& fa, int U, int64_t n_src, int style, hipStream_t s) {
-  return style == DSR_ROPE_GPTJ ? launch_fanout_u<DT, DSR_ROPE_GPTJ, LAYOUT>(fa, U, n_src, s)
-                                : launch_fanout_u<DT, DSR_ROPE_NEOX, LAYOUT>(fa, U, n_src, s);
+int launch_fanout_l(const FanArgs& fa, int style, hipStream_t s) {
+  if (!fa.dst_rope) return launch_fanout_s<DSR_DTYPE_BF16, DSR_ROPE_NEOX, LAYOUT, false>(fa, s);
+  return style == DSR_ROPE_GPTJ ? launch_fanout_s<DT, DSR_ROPE_GPTJ, LAYOUT, true>(fa, s)
+                                : launch_fanout_s<DT, DSR_ROPE_NEOX, LAYOUT, true>(fa, s);
 }
 
 template <int DT>
-int launch_fanout(const FanArgs& fa, int U, int64_t n_src, int style, int layout,
-                  hipStream_t s) {
+int launch_fanout(const FanArgs& fa, int style, int layout, hipStream_t s) {
   switch (layout) {
-    case kFanKx: return launch_fanout_l<DT, kFanKx>(fa, U, n_src, style, s);
-    case kFanHnd: return launch_fanout_l<DT, kFanHnd>(fa, U, n_src, style, s);
-    default: return launch_fanout_l<DT, kFanNhd>(fa, U, n_src, style, s);
+    case kRotKx: return launch_fanout_l<DT, kRotKx>(fa, style, s);
+    case kRotHnd: return launch_fanout_l<DT, kRotHnd>(fa, style, s);
+    default: return launch_fanout_l<DT, kRotNhd>(fa, style, s);
   }
 }
 
@@ -1108,9 +1100,8 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
   if (rc != DSR_OK) return rc;
   // the geometry is checked before the empty-work return below, so that a
   // call with n_dst = 0 tells whether the fan-out takes a geometry
-  // the page (or its part) in registers: at most 8 vectors per lane
-  const int64_t nvec = page_bytes >> 4;
-  if (nvec > 8 * kThreads) return DSR_ERR_SHAPE;
+  // pages of at most 32 KiB
+  if (page_bytes > (32 << 10)) return DSR_ERR_SHAPE;
   RotArgs ra{};
   ra.u = make_unit(layer_base, n_layers, kv_stride, page_stride, page_bytes, num_blocks,
                    nullptr, nullptr, 0, staging, staging_bytes, layer_bytes, layer0);
@@ -1192,19 +1183,9 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
     ra.u.hnd_row_vecs = (int)(page_bytes / ((int64_t)block_size * num_heads) / 16);
   }
   // a plain copy of split-x pages moves raw bytes: the token-major kernel
-  const int layout = k_layout == DSR_K_HND ? kFanHnd
-                     : k_layout == DSR_K_KX && dst_rope_idx ? kFanKx : kFanNhd;
-  // parts of whole rows (the rotation columns stay those of the page), at
-  // least one vector per lane each
-  int parts = 1;
-  if (const int64_t t = tune(DSR_TUNE_FANOUT_PARTS)) parts = layout == kFanNhd ? (int)t : 1;
-  const int64_t row_vecs = dst_rope_idx ? ra.row_vecs : 1;
-  while (parts > 1 && (nvec % parts || (nvec / parts) % row_vecs || nvec / parts < kThreads))
-    parts /= 2;
-  if (parts < 1) parts = 1;
-  if ((int64_t)n_src * n_layers * parts > 0x7fffffffLL) return DSR_ERR_ARG;
-  const int64_t pv = nvec / parts;
-  const int U = pv <= kThreads ? 1 : pv <= 2 * kThreads ? 2 : pv <= 4 * kThreads ? 4 : 8;
+  const int layout = k_layout == DSR_K_HND ? kRotHnd
+                     : k_layout == DSR_K_KX && dst_rope_idx ? kRotKx : kRotNhd;
+  if ((int64_t)n_src * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   if (n_src == 0 || n_dst == 0 || n_layers == 0) return DSR_OK;
   if (!dst_start) return DSR_ERR_ARG;
   FanArgs fa{};
@@ -1214,15 +1195,12 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
   fa.dst_pages = dst_page_ids;
   fa.dst_rope = dst_rope_idx;
   fa.n_src = n_src;
-  fa.parts = parts;
-  const int b = kFanLdsFloat2 / ra.rot_half;
-  fa.batch = b < kFanMaxBatch ? b : kFanMaxBatch;
   hipStream_t s = (hipStream_t)stream;
   switch (dt) {
-    case DSR_DTYPE_BF16: return launch_fanout<DSR_DTYPE_BF16>(fa, U, n_src, style, layout, s);
-    case DSR_DTYPE_FP16: return launch_fanout<DSR_DTYPE_FP16>(fa, U, n_src, style, layout, s);
-    case DSR_DTYPE_FP8_E4M3: return launch_fanout<DSR_DTYPE_FP8_E4M3>(fa, U, n_src, style, layout, s);
-    default: return launch_fanout<DSR_DTYPE_FP8_E5M2>(fa, U, n_src, style, layout, s);
+    case DSR_DTYPE_BF16: return launch_fanout<DSR_DTYPE_BF16>(fa, style, layout, s);
+    case DSR_DTYPE_FP16: return launch_fanout<DSR_DTYPE_FP16>(fa, style, layout, s);
+    case DSR_DTYPE_FP8_E4M3: return launch_fanout<DSR_DTYPE_FP8_E4M3>(fa, style, layout, s);
+    default: return launch_fanout<DSR_DTYPE_FP8_E5M2>(fa, style, layout, s);
   }
 }
 

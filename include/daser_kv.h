@@ -70,9 +70,6 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  *                                 of the page gather / scatter: 8, else 1
  *   DSR_TUNE_SLOTS_WG_PER_CU      workgroups per CU of the token kernels
  *   DSR_TUNE_FANOUT_WG_PER_CU     workgroups per CU of dsr_scatter_fanout
- *   DSR_TUNE_FANOUT_PARTS         workgroups per (record, layer) unit of
- *                                 dsr_scatter_fanout (1, 2, 4: parts of
- *                                 whole rows)
  * The other numbers have no effect; they keep the rest in their places.
  */
 #define DSR_TUNE_UNITS_PER_GROUP 0

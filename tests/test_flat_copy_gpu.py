@@ -250,3 +250,47 @@ def test_flat_slots(gpu, tuning, heads, dim, dt, block, max_wg):
             exp[:, :, int(ids[t // block]), t % block] = tmp[:, :, int(ids[t // block]), t % block]
     torch.cuda.synchronize()
     assert torch.equal(rot.view(torch.uint8), exp.view(torch.uint8))
+
+
+@pytest.mark.parametrize("n_src,n_dst,heads,dim,dt,layout,rot", [
+    (3, 300, 1, 64, "bf16", "nhd", 64), (511, 1100, 1, 128, "e4m3", "nhd", 128),
+    (512, 1100, 1, 128, "bf16", "nhd", 64), (600, 1300, 2, 64, "e5m2", "hnd", 64),
+    (5, 200, 2, 512, "fp16", "nhd", 512)])
+def test_flat_fanout(gpu, n_src, n_dst, heads, dim, dt, layout, rot):
+    """Both unit orders of the fan-out (few and many sources), more
+    destinations of a source than a wave holds at once, tables of up to 256
+    pairs: bit for bit the per-page load, K rotated or not."""
+    print(f"case: flat fanout {n_src}->{n_dst} H{heads} D{dim} {dt} {layout}", flush=True)
+    dtype = {"bf16": torch.bfloat16, "fp16": torch.float16, "e4m3": torch.float8_e4m3fn,
+             "e5m2": torch.float8_e5m2}[dt]
+    layers, block, nb = 2, 4, n_dst + 9
+    g = torch.Generator(device=gpu).manual_seed(n_src)
+    rng = np.random.default_rng(n_src)
+    recs = torch.randn((n_src, layers, 2, block, heads, dim), generator=g, device=gpu).to(dtype)
+    staging = recs.view(-1).view(torch.uint8)
+    inner = (heads, block, dim) if layout == "hnd" else (block, heads, dim)
+    caches = [torch.zeros((layers, 2, nb, *inner), dtype=dtype, device=gpu) for _ in range(2)]
+    tables = [ops.LayerTable([w.transpose(2, 3) if layout == "hnd" else w for w in c.unbind(0)])
+              for c in caches]
+    slot = tables[0].layout.slot_bytes
+    ids = rng.permutation(nb)[:n_dst].astype(np.int64)
+    src = np.concatenate([np.arange(n_src), rng.integers(0, n_src, n_dst - n_src)])
+    offs = rng.permutation(src).astype(np.int64) * slot
+    ang = torch.rand((5, rot // 2), generator=g, device=gpu, dtype=torch.float64) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    ridx = rng.integers(-1, 5, n_dst)
+    scales = torch.tensor([0.02, 1.5], device=gpu) if dt in ("e4m3", "e5m2") else None
+    assert ops.fanout_supported(tables[0].layout, rot)
+    ops.PreparedFanout(tables[0], ids, offs, staging,
+                       rope=(ridx, tabs, rot, "neox", scales, None))()
+    ops.scatter_rerotate(tables[1], ids, offs, staging, tabs, ridx, rot_dim=rot, k_scale=scales,
+                         shared_records=False)
+    torch.cuda.synchronize()
+    assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
+    assert caches[0].view(torch.uint8).any()
+    for c in caches:
+        c.zero_()
+    ops.PreparedFanout(tables[0], ids, offs, staging)()
+    ops.scatter(tables[1], ids, offs, staging, shared_records=False)
+    torch.cuda.synchronize()
+    assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))

@@ -14,7 +14,8 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-SRCS = [os.path.join(HERE, "csrc", "kv_move.hip"), os.path.join(HERE, "csrc", "store_ring.cpp")]
+SRCS = [os.path.join(HERE, "csrc", n)
+        for n in ("kv_move.hip", "store_ring.cpp", "load_plan.cpp")]
 INCLUDE = os.path.join(ROOT, "include")
 OUT = os.path.join(HERE, "libdaser_kv.so")
 ABI_TEST_SRC = os.path.join(ROOT, "tests", "c", "abi_roundtrip.cpp")

@@ -20,7 +20,7 @@ LIB_PATH = os.environ.get("DASER_KV_LIB") or os.path.join(
     os.path.dirname(os.path.abspath(__file__)), "libdaser_kv.so"
 )
 
-DSR_ABI_VERSION = 11
+DSR_ABI_VERSION = 12
 DSR_OK = 0
 DSR_ERR_ARG = -1
 DSR_ERR_ALIGN = -2
@@ -29,6 +29,15 @@ DSR_ERR_IO = -4
 DSR_ERR_NOFILE = -5
 DSR_ERR_TOO_LARGE = -6
 DSR_STATIC_TABLE_BYTES = 4 << 20
+DSR_PLAN_ERR_BLOCK = -20
+DSR_PLAN_ERR_RECORD = -21
+DSR_PLAN_ERR_ALIGN = -22
+DSR_PLAN_ERR_ROPE = -23
+DSR_PLAN_ERR_OVERLAP = -24
+DSR_PLAN_ERR_SLOT = -25
+DSR_PLAN_ERR_ROW = -26
+DSR_PLAN_ERR_ROWALIGN = -27
+DSR_PUT_BYTES = 3584
 
 DSR_RING_HOST = 1
 DSR_RING_DIRECT = 2
@@ -59,6 +68,43 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _I64 = ctypes.c_int64
 
+
+def plan_bytes(n: int) -> int:
+    """DSR_PLAN_BYTES."""
+    return 20 * n + 128
+
+
+class Plan(ctypes.Structure):
+    """dsr_plan."""
+
+    _fields_ = [("n_pages", ctypes.c_int32), ("n_src", ctypes.c_int32), ("off_start", _I64),
+                ("off_ids", _I64), ("off_rope", _I64), ("bytes", _I64)]
+
+
+def slot_plan_bytes(n: int) -> int:
+    """DSR_SLOT_PLAN_BYTES."""
+    return 44 * n + 256
+
+
+class SlotPlan(ctypes.Structure):
+    """dsr_slot_plan."""
+
+    _fields_ = [("n_pages", ctypes.c_int32), ("n_tokens", ctypes.c_int32)] + [
+        (n, _I64) for n in ("off_ids", "off_offsets", "off_page_rope", "off_slots", "off_rows",
+                            "off_rope", "bytes")]
+
+
+class GatherArgs(ctypes.Structure):
+    """dsr_gather_args."""
+
+    _fields_ = [("layer_base", _P), ("kv_stride", _I64), ("page_stride", _I64),
+                ("page_bytes", _I64), ("num_blocks", _I64), ("page_ids", _P),
+                ("slot_offsets", _P), ("staging", _P), ("staging_bytes", _I64),
+                ("layer_bytes", _I64)] + [
+        (n, ctypes.c_int32) for n in ("n_layers", "layer0", "n_pages", "block_size",
+                                      "num_heads", "reserved")]
+
+
 # Argument lists, one per exported entry point, in header order.
 _COPY_ARGS = [_P, _I, _I64, _I64, _I64, _I64, _P, _P, _I, _P, _I64, _I64, _I, _P]
 _SLOT_ARGS = [_P, _I, _I64, _I64, _I64, _I64, _I, _I64, _P, _P, _I, _P, _I64, _I64, _I, _P]
@@ -73,6 +119,14 @@ SIGNATURES = {
     "dsr_scatter_slots": (_SLOT_ARGS, _I),
     "dsr_scatter_slots_rerotate": (
         _SLOT_ARGS[:-1] + [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _P], _I),
+    "dsr_plan_shared": ([_P, _I], _I),
+    "dsr_plan_load": ([_P, _P, _P, _I, _I64, _I64, _I64, _I, _I, _P, _I64, _P], _I),
+    "dsr_plan_gather": ([_P, _P, _I, _I64, _I64, _I64, _I64, _P, _I64, _P], _I),
+    "dsr_plan_slots": (
+        [_P, _P, _P, _I, _I64, _I, _I64, _I64, _I64, _I, _I, _P, _I64, _P], _I),
+    "dsr_put": ([_P, _P, _I64, _P], _I),
+    "dsr_delta_tables": ([_P, _I, _I, _P, _P], _I),
+    "dsr_gather_layers": ([_P, _I, _I, _P], _I),
     "dsr_ring_open": ([ctypes.c_char_p, _I64, _I, _I, ctypes.POINTER(_P)], _I),
     "dsr_ring_write": ([_P, _P, _I64, _I64, _P], _I),
     "dsr_ring_read": ([_P, _P, _I64, _I64, _P], _I),

@@ -313,11 +313,7 @@ class KVDataPlane:
 
         arena = torch.empty(max(plan.arena_bytes, 16), dtype=torch.uint8, device=self.device)
         if plan.page_ids.size:
-            ops._validate(self.table.layout, plan.page_ids, plan.slot_offsets, arena, 0,
-                          self.table.layout.num_layers, True)
-            plan.gather = ops.PreparedGather(
-                self.table, torch.from_numpy(plan.page_ids).to(self.device),
-                torch.from_numpy(plan.slot_offsets).to(self.device), arena)
+            plan.gather = ops.PreparedGather(self.table, plan.page_ids, plan.slot_offsets, arena)
             per_layer = plan.page_ids.size * self.table.layout.layer_bytes
             plan.on_side = self._side is not None and (
                 self.save_stream == "side" or per_layer >= SIDE_STREAM_MIN_LAYER_BYTES)

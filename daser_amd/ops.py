@@ -15,6 +15,7 @@ Reference semantics restated here:
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 from typing import Optional, Sequence
@@ -281,6 +282,120 @@ def dest_order(page_ids, slot_offsets, extra=None):
     return sids, offs[order], ex
 
 
+_PLAN_ERRORS = {
+    _lib.DSR_PLAN_ERR_RECORD: (IndexError, "slot record outside the staging buffer"),
+    _lib.DSR_PLAN_ERR_ALIGN: (ValueError, "slot offsets must be multiples of 16 bytes"),
+    _lib.DSR_PLAN_ERR_ROPE: (IndexError, "rope_idx outside [-1, n_tables)"),
+    _lib.DSR_PLAN_ERR_OVERLAP: (ValueError, "slot records of two pages overlap"),
+    _lib.DSR_PLAN_ERR_SLOT: (IndexError, "slot outside the block pool"),
+    _lib.DSR_PLAN_ERR_ROW: (IndexError, "token row outside the staging buffer"),
+    _lib.DSR_PLAN_ERR_ROWALIGN: (ValueError, "row offsets must be multiples of 16 bytes"),
+}
+
+
+def _plan_check(name: str, rc: int, num_blocks: int) -> None:
+    if rc == _lib.DSR_PLAN_ERR_BLOCK:
+        raise IndexError(f"block id out of range [0, {num_blocks})")
+    if rc in _PLAN_ERRORS:
+        kind, text = _PLAN_ERRORS[rc]
+        raise kind(text)
+    _lib.check(name, rc)
+
+
+def _host_list(x) -> Optional[np.ndarray]:
+    """A host table as a contiguous int64 vector; None for device tensors and
+    for anything that is no vector."""
+    a = _host_array(x, np.int64)
+    return np.ascontiguousarray(a) if a is not None and a.ndim == 1 else None
+
+
+def _addr(a: Optional[np.ndarray]) -> Optional[int]:
+    return None if a is None else a.__array_interface__["data"][0]
+
+
+_BLIT_BYTES = 16 << 10
+
+
+def _plan_room(size: int) -> torch.Tensor:
+    """Host memory for a plan: pinned where its upload is a copy."""
+    return torch.empty(size, dtype=torch.uint8, pin_memory=size > _lib.DSR_PUT_BYTES)
+
+
+def _upload_plan(host: torch.Tensor, at: int, nbytes: int, device: torch.device,
+                 stream: int) -> torch.Tensor:
+    """``nbytes`` of the plan at ``at``, in stream order. Copies of up to 16 KiB
+    run as a kernel on the stream; larger ones go to a copy engine, which holds
+    the stream up by some 10 us (a load of 2,000 pages 139 against 152 us), so two
+    of the former are taken before one of the latter."""
+    if host.numel() > _lib.DSR_PUT_BYTES and nbytes > 2 * _BLIT_BYTES:
+        return host[at:at + nbytes].to(device, non_blocking=True)
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if host.numel() > _lib.DSR_PUT_BYTES:
+        for i in range(0, nbytes, _BLIT_BYTES):
+            k = min(_BLIT_BYTES, nbytes - i)
+            buf[i:i + k].copy_(host[at + i:at + i + k], non_blocking=True)
+        return buf
+    _lib.check("dsr_put", _lib.lib().dsr_put(buf.data_ptr(), host.data_ptr() + at, nbytes, stream))
+    return buf
+
+
+class _HostPlan:
+    """Host tables of one call, planned by the library (dsr_plan_load,
+    dsr_plan_gather) into one buffer and uploaded with one kernel (up to
+    DSR_PUT_BYTES) or one asynchronous copy from pinned memory. ``ptr`` holds
+    the device addresses of its sections."""
+
+    def __init__(self, n: int, device: torch.device, fill) -> None:
+        """``fill(address, size, plan)`` has the library write the tables."""
+        if torch.cuda.is_current_stream_capturing():
+            raise ValueError("host index tables cannot be used under graph capture: pass "
+                             "device tensors")
+        size = _lib.plan_bytes(n)
+        host = _plan_room(size)
+        self.plan = plan = _lib.Plan()
+        fill(host.data_ptr(), size, ctypes.addressof(plan))
+        self.stream = _stream_handle(device)
+        self.buf = _upload_plan(host, 0, plan.bytes, device, self.stream)
+        base = self.buf.data_ptr()
+        self.offsets, self.start = base, base + plan.off_start
+        self.ids, self.rope = base + plan.off_ids, base + plan.off_rope
+
+    def table(self, at: int, count: int, dtype: torch.dtype) -> torch.Tensor:
+        """A section as a tensor (a view that keeps the buffer)."""
+        width = torch.empty(0, dtype=dtype).element_size()
+        return self.buf[at:at + count * width].view(dtype)
+
+
+def _layer_range(lay: PagedKVLayout, layers) -> tuple[int, int]:
+    first, count = (0, lay.num_layers) if layers is None else layers
+    if first < 0 or count < 0 or first + count > lay.num_layers:
+        raise IndexError("layer range outside the registered caches")
+    return first, count
+
+
+def _check_staging(lay: PagedKVLayout, staging: torch.Tensor) -> int:
+    if staging.device != lay.device:
+        raise ValueError("staging must live on the KV caches' device")
+    if not staging.is_contiguous():
+        raise ValueError("staging must be contiguous")
+    return staging.numel() * staging.element_size()
+
+
+def _load_plan(lay: PagedKVLayout, ids, offs, ridx, n_tables: int, staging_bytes: int,
+               rec_layers: int, fanout: bool) -> _HostPlan:
+    """The tables of a load (host vectors), in destination order or grouped by
+    record."""
+    rec_end = (rec_layers - 1) * lay.layer_bytes + 2 * lay.page_bytes
+    lib = _lib.lib()
+
+    def fill(out: int, size: int, plan: int) -> None:
+        _plan_check("dsr_plan_load", lib.dsr_plan_load(
+            _addr(ids), _addr(offs), _addr(ridx), ids.size, lay.num_blocks, max(rec_end, 0),
+            staging_bytes, n_tables, int(fanout), out, size, plan), lay.num_blocks)
+
+    return _HostPlan(ids.size, lay.device, fill)
+
+
 def _copy_args(table: LayerTable, page_ids, slot_offsets, staging, layer0, layers,
                records_written: bool = False):
     lay = table.layout
@@ -328,10 +443,14 @@ def gather(
     ``layers=(first, count)`` restricts the launch to a layer range; the
     record index of table layer ``first + i`` is ``layer0 + first + i``.
     """
-    args, _tables = _copy_args(table, page_ids, slot_offsets, staging, layer0, layers,
-                            records_written=True)
-    fn, name, extra = _copy_entry(table.layout, "dsr_gather")
-    rc = fn(*args, *extra, _stream_handle(table.layout.device))
+    lay = table.layout
+    (ids, offs), _plan = _gather_tables(table, page_ids, slot_offsets, staging, layer0, layers)
+    first, count = _layer_range(lay, layers)
+    fn, name, extra = _copy_entry(lay, "dsr_gather")
+    rc = fn(table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
+            lay.num_blocks, ids.data_ptr(), offs.data_ptr(), ids.numel(), staging.data_ptr(),
+            staging.numel() * staging.element_size(), lay.layer_bytes, layer0 + first, *extra,
+            _stream_handle(lay.device))
     _lib.check(name, rc)
 
 
@@ -353,25 +472,54 @@ class PreparedGather:
 
     def __init__(self, table: LayerTable, page_ids, slot_offsets, staging: torch.Tensor,
                  *, layer0: int = 0) -> None:
-        args, self._keep = _copy_args(table, page_ids, slot_offsets, staging, layer0, None,
-                                      records_written=True)
-        self.tables = self._keep  # (page_ids, slot_offsets) as device tensors
-        self._table = table
-        self._staging = staging
-        self._mid = args[2:12]  # strides, page geometry, tables, staging
-        self._layer0 = layer0
-        self._n_layers = table.layout.num_layers
-        self._fn, self._name, self._extra = _copy_entry(table.layout, "dsr_gather")
+        lay = table.layout
+        self.tables, plan = _gather_tables(table, page_ids, slot_offsets, staging, layer0, None)
+        ids, offs = self.tables  # (page_ids, slot_offsets) as device tensors
+        self._keep = (table, staging, plan)
+        hnd = lay.k_layout == "hnd"
+        self._args = _lib.GatherArgs(
+            table.ptr(), lay.kv_stride, lay.page_stride, lay.page_bytes, lay.num_blocks,
+            ids.data_ptr(), offs.data_ptr(), staging.data_ptr(),
+            staging.numel() * staging.element_size(), lay.layer_bytes, lay.num_layers, layer0,
+            ids.numel(), lay.block_size if hnd else 0, lay.num_heads if hnd else 0, 0)
+        self._args_ptr = ctypes.addressof(self._args)
+        self._n_layers = lay.num_layers
+        self._fn = _lib.lib().dsr_gather_layers
 
     def __call__(self, first: int, count: int, stream: int) -> None:
         """Gathers table layers [first, first + count) on ``stream`` (a HIP
         stream handle, e.g. ``torch.cuda.current_stream().cuda_stream``)."""
         if first < 0 or count < 0 or first + count > self._n_layers:
             raise IndexError("layer range outside the registered caches")
-        rc = self._fn(self._table.ptr(first), count, *self._mid, self._layer0 + first,
-                      *self._extra, stream)
+        rc = self._fn(self._args_ptr, first, count, stream)
         if rc:
-            _lib.check(self._name, rc)
+            _lib.check("dsr_gather_layers", rc)
+
+
+def _gather_tables(table: LayerTable, page_ids, slot_offsets, staging, layer0, layers):
+    """Checked device tables (page_ids, slot_offsets) of a gather and, of host
+    tables, the plan that holds them."""
+    lay = table.layout
+    ids, offs = _host_list(page_ids), _host_list(slot_offsets)
+    if ids is None or offs is None or not ids.size or lay.device.type != "cuda":
+        return _copy_args(table, page_ids, slot_offsets, staging, layer0, layers,
+                          records_written=True)[1], None
+    first, count = _layer_range(lay, layers)
+    nbytes = _check_staging(lay, staging)
+    if ids.shape != offs.shape:
+        raise ValueError("page_ids and slot_offsets differ in length")
+    span = (count - 1) * lay.layer_bytes + 2 * lay.page_bytes
+    end = span + (layer0 + first) * lay.layer_bytes
+    lib = _lib.lib()
+
+    def fill(out: int, size: int, plan: int) -> None:
+        _plan_check("dsr_plan_gather", lib.dsr_plan_gather(
+            _addr(ids), _addr(offs), ids.size, lay.num_blocks, max(end, 0), max(span, 0),
+            nbytes, out, size, plan), lay.num_blocks)
+
+    h = _HostPlan(ids.size, lay.device, fill)
+    return (h.table(h.plan.off_ids, ids.size, torch.int32),
+            h.table(0, ids.size, torch.int64)), h
 
 
 def scatter(
@@ -392,12 +540,13 @@ def scatter(
     tables a launch shaped for cache-served reads. None: inferred from host
     ``slot_offsets`` (at most half of them distinct), False for device
     tables. Results do not depend on it."""
+    host = _host_tables(table, page_ids, slot_offsets)
+    if host is not None:
+        _load_host(table, *host, staging, layer0, layers, shared_records)
+        return
     if shared_records is None:
         shared_records = _shared_offsets(slot_offsets)
     page_ids, slot_offsets, _ = dest_order(page_ids, slot_offsets)
-    if shared_records and _scatter_fanout(table, page_ids, slot_offsets, staging, layer0,
-                                          layers):
-        return
     args, _tables = _copy_args(table, page_ids, slot_offsets, staging, layer0, layers)
     stream = _stream_handle(table.layout.device)
     if shared_records and table.layout.k_layout != "hnd":
@@ -407,6 +556,73 @@ def scatter(
     fn, name, extra = _copy_entry(table.layout, "dsr_scatter")
     rc = fn(*args, *extra, stream)
     _lib.check(name, rc)
+
+
+def _host_tables(table: LayerTable, page_ids, slot_offsets):
+    """(page_ids, slot_offsets) as host vectors if the library can plan them:
+    both on the host, not empty, of one length."""
+    ids, offs = _host_list(page_ids), _host_list(slot_offsets)
+    if ids is None or offs is None or not ids.size or ids.size != offs.size or \
+            table.layout.device.type != "cuda":
+        return None
+    return ids, offs
+
+
+def _load_host(table: LayerTable, ids: np.ndarray, offs: np.ndarray, staging: torch.Tensor,
+               layer0: int, layers, shared: Optional[bool], rope=None) -> None:
+    """A load of host tables: planned, uploaded once, launched. ``rope``: None,
+    or (rope_idx, cos_sin, rot_dim, style, n_tables, n_groups, layer_group on the
+    device or None, k_scale pointer)."""
+    lay = table.layout
+    lib = _lib.lib()
+    if shared is None:
+        shared = lib.dsr_plan_shared(_addr(offs), ids.size) == 1
+    fan = shared and (fanout_supported(lay, rope[2], rope[3]) if rope else fanout_supported(lay))
+    first, count = _layer_range(lay, layers)
+    nbytes = _check_staging(lay, staging)
+    ridx, n_tables = (rope[0], rope[4]) if rope else (None, 0)
+    p = _load_plan(lay, ids, offs, ridx, n_tables, nbytes, layer0 + first + count, fan)
+    plan = p.plan
+    if fan:
+        tail = (None, 0, None, 0, 0, 0, 0, 0, None) if rope is None else _fan_tail(lay, rope)
+        _lib.check("dsr_scatter_fanout", lib.dsr_scatter_fanout(
+            table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
+            lay.num_blocks, p.offsets, plan.n_src, p.start, p.ids, p.rope if rope else None,
+            plan.n_pages, staging.data_ptr(), nbytes, lay.layer_bytes, layer0 + first, *tail,
+            _K_LAYOUTS[lay.k_layout], lay.block_size, lay.num_heads, p.stream))
+        return
+    args = (table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
+            lay.num_blocks, p.ids, p.offsets, plan.n_pages, staging.data_ptr(), nbytes,
+            lay.layer_bytes, layer0 + first)
+    if rope is None:
+        fn, name, extra = _copy_entry(lay, "dsr_scatter")
+        _lib.check(name, fn(*args, *extra, p.stream))
+        return
+    _, cos_sin, rot_dim, style, n_tables, n_groups, lg_d, ks_ptr = rope
+    _rerotate(lay, args, cos_sin.data_ptr(), p.rope, n_tables, n_groups, lg_d, rot_dim, style,
+              ks_ptr, shared, p.stream)
+
+
+def _fan_tail(lay: PagedKVLayout, rope):
+    _, cos_sin, rot_dim, style, n_tables, n_groups, lg_d, ks_ptr = rope
+    return (cos_sin.data_ptr(), n_tables, None if lg_d is None else lg_d.data_ptr(), n_groups,
+            lay.head_dim, rot_dim, ROPE_STYLES[style], _DTYPE_CODES[lay.dtype], ks_ptr)
+
+
+def _rerotate(lay: PagedKVLayout, args, cos_sin: int, rope_idx: int, n_tables: int,
+              n_groups: int, lg_d, rot_dim: int, style: str, ks_ptr, shared: bool,
+              stream: int) -> None:
+    """The layout's re-rotation entry point on device tables."""
+    common = (*args, cos_sin, rope_idx, n_tables, None if lg_d is None else lg_d.data_ptr(),
+              n_groups, lay.head_dim, rot_dim, ROPE_STYLES[style], _DTYPE_CODES[lay.dtype],
+              ks_ptr)
+    flags = _lib.DSR_REROTATE_SHARED_RECORDS if shared else 0
+    if lay.k_layout in ("kx", "hnd"):
+        name = "dsr_scatter_rerotate_" + lay.k_layout
+        _lib.check(name, getattr(_lib.lib(), name)(*common, lay.block_size, flags, stream))
+    else:
+        _lib.check("dsr_scatter_rerotate",
+                   _lib.lib().dsr_scatter_rerotate(*common, flags, stream))
 
 
 def _shared_offsets(slot_offsets) -> bool:
@@ -470,85 +686,52 @@ class PreparedFanout:
     def __init__(self, table: LayerTable, page_ids, slot_offsets, staging: torch.Tensor, *,
                  rope=None, layer0: int = 0, layers: Optional[tuple[int, int]] = None) -> None:
         lay = table.layout
-        ids = _host_array(page_ids, np.int64)
-        offs = _host_array(slot_offsets, np.int64)
+        ids, offs = _host_list(page_ids), _host_list(slot_offsets)
         if ids is None or offs is None:
             raise ValueError("PreparedFanout takes host tables")
-        first, count = (0, lay.num_layers) if layers is None else layers
-        if first < 0 or count < 0 or first + count > lay.num_layers:
-            raise IndexError("layer range outside the registered caches")
+        first, count = _layer_range(lay, layers)
         if staging.device != lay.device or not staging.is_contiguous():
             raise ValueError("staging must be a contiguous tensor on the KV caches' device")
+        if ids.shape != offs.shape:
+            raise ValueError("page_ids and slot_offsets differ in length")
         tail = (None, 0, None, 0, 0, 0, 0, 0, None)
-        ridx = None
-        keep = []
+        ridx, n_tables, keep = None, 0, []
         if rope is not None:
             rope_idx, cos_sin, rot_dim, style, k_scale, layer_group = rope
             rot_dim, n_tables, n_groups, lg_d, ks_ptr = _rope_args(
                 lay, cos_sin, rope_idx, rot_dim, k_scale, layer0, layer_group)
-            ridx = _host_array(rope_idx, np.int64)
+            ridx = _host_list(rope_idx)
             if ridx is None:
                 raise ValueError("PreparedFanout takes host tables")
             if ridx.shape != ids.shape:
                 raise ValueError("rope_idx and page_ids differ in length")
             if not fanout_supported(lay, rot_dim, style):
                 raise ValueError("these pages need the per-page re-rotation kernels")
-            tail = (cos_sin.data_ptr(), n_tables, None if lg_d is None else lg_d.data_ptr(),
-                    n_groups, lay.head_dim, rot_dim, ROPE_STYLES[style],
-                    _DTYPE_CODES[lay.dtype], ks_ptr)
+            tail = _fan_tail(lay, (ridx, cos_sin, rot_dim, style, n_tables, n_groups, lg_d,
+                                   ks_ptr))
             keep += [cos_sin, lg_d, k_scale]
         elif not fanout_supported(lay):
             raise ValueError("these pages need the per-page scatter kernels")
-        ids, offs, ridx = dest_order(ids, offs, ridx)
-        _validate(lay, ids, offs, staging, layer0 + first, count, False)
-        src, start, dpages, drope = fanout_tables(ids, offs, ridx)
-        dev = lay.device
-        self._tables = [_upload(torch.from_numpy(src), dev),
-                        _upload(torch.from_numpy(start), dev),
-                        _upload(torch.from_numpy(dpages.astype(np.int32)), dev),
-                        None if drope is None else
-                        _upload(torch.from_numpy(drope.astype(np.int32)), dev)]
-        self._keep = keep + [table, staging]
-        self.n_src, self.n_dst = int(src.size), int(dpages.size)
-        src_d, start_d, pages_d, rope_d = self._tables
+        nbytes = staging.numel() * staging.element_size()
+        p = _load_plan(lay, ids, offs, ridx, n_tables, nbytes, layer0 + first + count, True)
+        self._keep = keep + [table, staging, p]
+        self.n_src, self.n_dst = p.plan.n_src, p.plan.n_pages
         self._args = (table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
-                      lay.num_blocks, src_d.data_ptr(), self.n_src, start_d.data_ptr(),
-                      pages_d.data_ptr(), None if rope_d is None else rope_d.data_ptr(),
-                      self.n_dst, staging.data_ptr(), staging.numel() * staging.element_size(),
+                      lay.num_blocks, p.offsets, self.n_src, p.start, p.ids,
+                      None if ridx is None else p.rope, self.n_dst, staging.data_ptr(), nbytes,
                       lay.layer_bytes, layer0 + first, *tail, _K_LAYOUTS[lay.k_layout],
                       lay.block_size, lay.num_heads)
-        self._device = dev
+        self._device = lay.device
 
     def __call__(self) -> None:
         rc = _lib.lib().dsr_scatter_fanout(*self._args, _stream_handle(self._device))
         _lib.check("dsr_scatter_fanout", rc)
 
 
-def _scatter_fanout(table: LayerTable, page_ids, slot_offsets, staging: torch.Tensor,
-                    layer0: int, layers, rope=None) -> bool:
-    """The load of host tables whose pages share records, each record read
-    once (:class:`PreparedFanout`, prepared and launched once). Returns
-    False, having launched nothing, for device tables and for pages that
-    need the per-page kernels (:func:`fanout_supported`)."""
-    lay = table.layout
-    if _host_array(page_ids, np.int64) is None or _host_array(slot_offsets, np.int64) is None:
-        return False
-    if rope is not None:
-        if _host_array(rope[0], np.int64) is None:
-            return False
-        rot_dim = lay.head_dim if rope[2] is None else rope[2]
-        if not fanout_supported(lay, rot_dim, rope[3]):
-            return False
-    elif not fanout_supported(lay):
-        return False
-    PreparedFanout(table, page_ids, slot_offsets, staging, rope=rope, layer0=layer0,
-                   layers=layers)()
-    return True
-
-
 def _rope_args(lay: PagedKVLayout, cos_sin: torch.Tensor, rope_idx, rot_dim, k_scale,
                layer0: int, layer_group):
-    """Checks the re-rotation inputs shared by the page and token forms;
+    """Checks the re-rotation inputs shared by the page and token forms
+    (rope_idx None: its entries are checked elsewhere);
     returns (rot_dim, n_tables, n_groups or 0, device layer_group or None,
     k_scale pointer or None)."""
     if lay.dtype not in _DTYPE_CODES:
@@ -566,7 +749,7 @@ def _rope_args(lay: PagedKVLayout, cos_sin: torch.Tensor, rope_idx, rot_dim, k_s
         raise ValueError("cos_sin must be a contiguous device tensor")
     n_groups = cos_sin.shape[0] if grouped else 1
     n_tables = cos_sin.shape[-3]
-    ridx = _host_array(rope_idx, np.int64)
+    ridx = None if rope_idx is None else _host_array(rope_idx, np.int64)
     if ridx is not None and ridx.size and (ridx.max() >= n_tables or ridx.min() < -1):
         raise IndexError("rope_idx outside [-1, n_tables)")
     lg_d = None
@@ -623,31 +806,23 @@ def scatter_rerotate(
     tables. Results do not depend on it.
     """
     lay = table.layout
+    host, ridx = _host_tables(table, page_ids, slot_offsets), _host_list(rope_idx)
+    planned = host is not None and ridx is not None and ridx.size == host[0].size
     rot_dim, n_tables, n_groups, lg_d, ks_ptr = _rope_args(
-        lay, cos_sin, rope_idx, rot_dim, k_scale, layer0, layer_group)
+        lay, cos_sin, None if planned else rope_idx, rot_dim, k_scale, layer0, layer_group)
+    if planned:
+        _load_host(table, *host, staging, layer0, layers, shared_records,
+                   (ridx, cos_sin, rot_dim, style, n_tables, n_groups, lg_d, ks_ptr))
+        return
     if shared_records is None:
         shared_records = _shared_offsets(slot_offsets)
     page_ids, slot_offsets, rope_idx = dest_order(page_ids, slot_offsets, rope_idx)
-    if shared_records and _scatter_fanout(
-            table, page_ids, slot_offsets, staging, layer0, layers,
-            (rope_idx, cos_sin, rot_dim, style, k_scale, layer_group)):
-        return
     args, _tables = _copy_args(table, page_ids, slot_offsets, staging, layer0, layers)
     ridx_d = _as_device_table(rope_idx, torch.int32, lay.device, "rope_idx")
     if ridx_d.numel() != _tables[0].numel():
         raise ValueError("rope_idx and page_ids differ in length")
-    common = (*args, cos_sin.data_ptr(), ridx_d.data_ptr(), n_tables,
-              None if lg_d is None else lg_d.data_ptr(), n_groups,
-              lay.head_dim, rot_dim, ROPE_STYLES[style], _DTYPE_CODES[lay.dtype], ks_ptr)
-    flags = _lib.DSR_REROTATE_SHARED_RECORDS if shared_records else 0
-    if lay.k_layout in ("kx", "hnd"):
-        name = "dsr_scatter_rerotate_" + lay.k_layout
-        rc = getattr(_lib.lib(), name)(*common, lay.block_size, flags,
-                                       _stream_handle(lay.device))
-        _lib.check(name, rc)
-    else:
-        rc = _lib.lib().dsr_scatter_rerotate(*common, flags, _stream_handle(lay.device))
-        _lib.check("dsr_scatter_rerotate", rc)
+    _rerotate(lay, args, cos_sin.data_ptr(), ridx_d.data_ptr(), n_tables, n_groups, lg_d, rot_dim,
+              style, ks_ptr, shared_records, _stream_handle(lay.device))
 
 
 def _slots_args(table: LayerTable, slot_mapping, row_offsets, staging, layer0, layers,
@@ -703,11 +878,71 @@ def _slots_args(table: LayerTable, slot_mapping, row_offsets, staging, layer0, l
             lay.layer_bytes, layer0 + first), (sm_d, ro_d)
 
 
+def _slots_host(table: LayerTable, slot_mapping, row_offsets, staging: torch.Tensor, layer0: int,
+                layers, mode: int, rope=None) -> bool:
+    """A token-form call with host tables: planned by the library, its whole
+    pages (loads) through the page form, the other tokens through the token
+    kernels. ``rope`` as for :func:`_load_host`. False, having done nothing, for
+    tables that the library cannot plan (device tables, empty or odd ones)."""
+    lay = table.layout
+    sm, ro = _host_list(slot_mapping), _host_list(row_offsets)
+    if sm is None or ro is None or not sm.size or sm.size != ro.size or \
+            lay.device.type != "cuda" or not lay.has_geometry or lay.k_layout != "nhd":
+        return False
+    ridx, n_tables = (rope[0], rope[4]) if rope else (None, 0)
+    if rope and (ridx is None or ridx.size != sm.size):
+        return False
+    first, count = _layer_range(lay, layers)
+    if staging.device != lay.device or not staging.is_contiguous():
+        raise ValueError("staging must be a contiguous tensor on the caches' device")
+    if torch.cuda.is_current_stream_capturing():
+        raise ValueError("host index tables cannot be used under graph capture: pass "
+                         "device tensors")
+    nbytes = staging.numel() * staging.element_size()
+    row = lay.num_heads * lay.head_dim * lay.elem_bytes
+    end = (layer0 + first + count - 1) * lay.layer_bytes + lay.page_bytes + row
+    size = _lib.slot_plan_bytes(sm.size)
+    host = _plan_room(size)
+    plan = _lib.SlotPlan()
+    lib = _lib.lib()
+    _plan_check("dsr_plan_slots", lib.dsr_plan_slots(
+        _addr(sm), _addr(ro), _addr(ridx), sm.size, lay.num_blocks, lay.block_size, row,
+        max(end, 0), nbytes, n_tables, mode, host.data_ptr(), size, ctypes.addressof(plan)),
+        lay.num_blocks)
+    if plan.n_pages:
+        at = host.numpy()
+        ids, offs, prope = (at[o:o + 8 * plan.n_pages].view(np.int64) for o in
+                            (plan.off_ids, plan.off_offsets,
+                             plan.off_page_rope if rope else plan.off_ids))
+        _load_host(table, ids, offs, staging, layer0, layers, None,
+                   (prope, *rope[1:]) if rope else None)
+    if not plan.n_tokens:
+        return True
+    stream = _stream_handle(lay.device)
+    buf = _upload_plan(host, plan.off_slots, plan.bytes, lay.device, stream)
+    base = buf.data_ptr() - plan.off_slots
+    args = (table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
+            lay.num_blocks, lay.block_size, row, base + plan.off_slots, base + plan.off_rows,
+            plan.n_tokens, staging.data_ptr(), nbytes, lay.layer_bytes, layer0 + first)
+    if rope:
+        _, cos_sin, rot_dim, style, n_tables, n_groups, lg_d, ks_ptr = rope
+        _lib.check("dsr_scatter_slots_rerotate", lib.dsr_scatter_slots_rerotate(
+            *args, cos_sin.data_ptr(), base + plan.off_rope, n_tables,
+            None if lg_d is None else lg_d.data_ptr(), n_groups, lay.head_dim, rot_dim,
+            ROPE_STYLES[style], _DTYPE_CODES[lay.dtype], ks_ptr, stream))
+    else:
+        name = "dsr_gather_slots" if mode else "dsr_scatter_slots"
+        _lib.check(name, getattr(lib, name)(*args, stream))
+    return True
+
+
 def gather_slots(table: LayerTable, slot_mapping, row_offsets, staging: torch.Tensor, *,
                  layer0: int = 0, layers: Optional[tuple[int, int]] = None) -> None:
     """Token-granular gather driven by vLLM's slot_mapping (-1 = padding):
     each valid token's K and V rows of every layer go to its record rows at
     ``row_offsets[t]`` (see :func:`token_row_offsets`)."""
+    if _slots_host(table, slot_mapping, row_offsets, staging, layer0, layers, 1):
+        return
     args, _tables = _slots_args(table, slot_mapping, row_offsets, staging, layer0, layers, True)
     rc = _lib.lib().dsr_gather_slots(*args, _stream_handle(table.layout.device))
     _lib.check("dsr_gather_slots", rc)
@@ -787,20 +1022,11 @@ def scatter_slots(table: LayerTable, slot_mapping, row_offsets, staging: torch.T
     tokens (the ragged edges of requests) go through the token kernel;
     whole pages that share records load through :class:`PreparedFanout`,
     as in :func:`scatter`. Device tables go to the token kernel as given."""
+    if _slots_host(table, slot_mapping, row_offsets, staging, layer0, layers, 0):
+        return
     host = slot_order(slot_mapping, row_offsets)
     if host is not None:
-        sm, ro, _ = host
-        lay = table.layout
-        if lay.has_geometry and lay.k_layout == "nhd":
-            row = lay.num_heads * lay.head_dim * lay.elem_bytes
-            pages, offs, _, rest = whole_pages(sm, ro, lay.block_size, row)
-            if pages.size:
-                scatter(table, pages, offs, staging, layer0=layer0, layers=layers,
-                        shared_records=None)
-                sm, ro = sm[rest], ro[rest]
-                if not np.any(sm >= 0):
-                    return
-        slot_mapping, row_offsets = sm, ro
+        slot_mapping, row_offsets, _ = host
     args, _tables = _slots_args(table, slot_mapping, row_offsets, staging, layer0, layers, False)
     rc = _lib.lib().dsr_scatter_slots(*args, _stream_handle(table.layout.device))
     _lib.check("dsr_scatter_slots", rc)
@@ -821,20 +1047,13 @@ def scatter_slots_rerotate(table: LayerTable, slot_mapping, row_offsets,
     lay = table.layout
     rot_dim, n_tables, n_groups, lg_d, ks_ptr = _rope_args(
         lay, cos_sin, rope_idx, rot_dim, k_scale, layer0, layer_group)
+    if _slots_host(table, slot_mapping, row_offsets, staging, layer0, layers, 0,
+                   (_host_list(rope_idx), cos_sin, rot_dim, style, n_tables, n_groups, lg_d,
+                    ks_ptr)):
+        return
     host = slot_order(slot_mapping, row_offsets, rope_idx)
     if host is not None:
-        sm, ro, ri = host
-        if lay.has_geometry and lay.k_layout == "nhd":
-            row = lay.num_heads * lay.head_dim * lay.elem_bytes
-            pages, offs, pri, rest = whole_pages(sm, ro, lay.block_size, row, ri)
-            if pages.size:
-                scatter_rerotate(table, pages, offs, staging, cos_sin, pri, rot_dim=rot_dim,
-                                 style=style, k_scale=k_scale, layer0=layer0, layers=layers,
-                                 layer_group=layer_group, shared_records=None)
-                sm, ro, ri = sm[rest], ro[rest], ri[rest]
-                if not np.any(sm >= 0):
-                    return
-        slot_mapping, row_offsets, rope_idx = sm, ro, ri
+        slot_mapping, row_offsets, rope_idx = host
     args, _tables = _slots_args(table, slot_mapping, row_offsets, staging, layer0, layers, False)
     ridx_d = _as_device_table(rope_idx, torch.int32, lay.device, "rope_idx")
     if ridx_d.numel() != _tables[0].numel():

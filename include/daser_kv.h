@@ -52,7 +52,7 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  * dsr_set_tuning, 7 dsr_scatter_ex, 8 dsr_scatter_slots_rerotate, 9
  * DSR_RING_MMAP and dsr_ring_is_mapped, 10 dsr_scatter_rerotate_static, 11
  * dsr_scatter_fanout. Callers check dsr_abi_version() against it. */
-#define DSR_ABI_VERSION 11
+#define DSR_ABI_VERSION 12
 
 /*
  * Kernel choice and launch shape follow from the geometry. dsr_set_tuning()
@@ -464,6 +464,102 @@ int dsr_scatter_slots_rerotate(const uint64_t* layer_base, int n_layers, int64_t
                                const int32_t* layer_group, int n_groups, int head_dim,
                                int rot_dim, int rope_style, int dtype, const float* k_scale,
                                dsr_stream_t stream);
+
+/*
+ * Host tables of a gather or a load, checked, ordered and packed into one buffer
+ * for a single upload (host code; the entry points above take the tables from
+ * device memory). page_ids, slot_offsets and rope_idx (NULL: none) hold n
+ * entries. rec_end: bytes from a record's offset to the end of the last layer
+ * that the call moves. `out` has out_bytes >= DSR_PLAN_BYTES(n) bytes, 16-byte
+ * aligned; the sections lie at the plan's offsets, the record offsets (int64) at
+ * 0: copy plan->bytes of it to the device.
+ *
+ * dsr_plan_load: entries in destination-block order, of a block listed more than
+ * once the last one (the reference's sequential copies, daser_connector.py:
+ * 536-551, leave that one). fanout = 0: page tables (n_pages entries of offsets,
+ * ids, rope); 1: the tables of dsr_scatter_fanout (n_src offsets, n_src + 1
+ * starts, n_pages ids and rope, sources by offset).
+ * dsr_plan_gather: entries as given; records of two pages (rec_span bytes each)
+ * must not overlap.
+ * dsr_plan_shared: 1 if at most half of the n offsets are distinct (n > 1), else 0.
+ *
+ * Return 0, DSR_PLAN_ERR_* for a bad entry, or DSR_ERR_ARG / DSR_ERR_TOO_LARGE
+ * (out too small, or out of host memory).
+ */
+#define DSR_PLAN_ERR_BLOCK (-20)   /* a block id outside [0, num_blocks)        */
+#define DSR_PLAN_ERR_RECORD (-21)  /* a record outside the staging buffer        */
+#define DSR_PLAN_ERR_ALIGN (-22)   /* a record offset not a multiple of 16       */
+#define DSR_PLAN_ERR_ROPE (-23)    /* a table index outside [-1, n_tables)       */
+#define DSR_PLAN_ERR_OVERLAP (-24) /* two pages' records overlap (gather)        */
+#define DSR_PLAN_BYTES(n) (20 * (int64_t)(n) + 128)
+
+typedef struct {
+  int32_t n_pages;
+  int32_t n_src;     /* fan-out only */
+  int64_t off_start; /* fan-out only */
+  int64_t off_ids;
+  int64_t off_rope;
+  int64_t bytes;
+} dsr_plan;
+
+int dsr_plan_shared(const int64_t* slot_offsets, int n);
+int dsr_plan_load(const int64_t* page_ids, const int64_t* slot_offsets, const int64_t* rope_idx,
+                  int n, int64_t num_blocks, int64_t rec_end, int64_t staging_bytes, int n_tables,
+                  int fanout, void* out, int64_t out_bytes, dsr_plan* plan);
+int dsr_plan_gather(const int64_t* page_ids, const int64_t* slot_offsets, int n,
+                    int64_t num_blocks, int64_t rec_end, int64_t rec_span, int64_t staging_bytes,
+                    void* out, int64_t out_bytes, dsr_plan* plan);
+
+/*
+ * The same for the token form: n tokens' slots (negative: padding) and record row
+ * offsets. row_end: bytes from a row's offset to the end of the row's V in the
+ * last layer that the call moves. mode 0: a load; blocks whose every slot is
+ * listed with consecutive record rows and one table index become pages (for
+ * dsr_plan_load: ids, offsets and rope as int64), the other tokens follow in slot
+ * order; of a slot listed more than once the last one. mode 1: a save; tokens as
+ * given, of a row listed more than once the last one. The sections from
+ * off_slots on (slots and rows as int64, rope as int32) are one upload.
+ */
+#define DSR_PLAN_ERR_SLOT (-25)    /* a slot outside the block pool              */
+#define DSR_PLAN_ERR_ROW (-26)     /* a row outside the staging buffer           */
+#define DSR_PLAN_ERR_ROWALIGN (-27) /* a row offset not a multiple of 16         */
+#define DSR_SLOT_PLAN_BYTES(n) (44 * (int64_t)(n) + 256)
+
+typedef struct {
+  int32_t n_pages, n_tokens;
+  int64_t off_ids, off_offsets, off_page_rope;
+  int64_t off_slots, off_rows, off_rope, bytes; /* bytes: of the upload from off_slots */
+} dsr_slot_plan;
+
+int dsr_plan_slots(const int64_t* slots, const int64_t* rows, const int64_t* rope_idx, int n,
+                   int64_t num_blocks, int block_size, int64_t row_bytes, int64_t row_end,
+                   int64_t staging_bytes, int n_tables, int mode, void* out, int64_t out_bytes,
+                   dsr_slot_plan* plan);
+
+/* Writes up to DSR_PUT_BYTES bytes (a multiple of 4) of host memory to device
+ * memory (4-byte aligned) as a kernel's arguments, in stream order: the source
+ * may be reused at once. For small tables; a copy costs twice the host time. */
+#define DSR_PUT_BYTES 3584
+int dsr_put(void* dst, const void* src, int64_t bytes, dsr_stream_t stream);
+
+/* Rotation tables on the device: out[d][j] = (cos, sin)(x[d] * x[n + j]) in
+ * float64, rounded once to float32, for d < n deltas and j < half inverse
+ * frequencies; x holds the n deltas, then the half frequencies (device, float64). */
+int dsr_delta_tables(const double* x, int n, int half, float* out, dsr_stream_t stream);
+
+/* dsr_gather (num_heads = 0) or dsr_gather_hnd with its arguments kept by the
+ * caller, for layers [first, first + count) of the table: the record index of
+ * layer l is layer0 + l. For callers that launch one gather per layer. */
+typedef struct {
+  const uint64_t* layer_base;
+  int64_t kv_stride, page_stride, page_bytes, num_blocks;
+  const int32_t* page_ids;
+  const int64_t* slot_offsets;
+  void* staging;
+  int64_t staging_bytes, layer_bytes;
+  int32_t n_layers, layer0, n_pages, block_size, num_heads, reserved;
+} dsr_gather_args;
+int dsr_gather_layers(const dsr_gather_args* args, int first, int count, dsr_stream_t stream);
 
 /*
  * Pinned-host staging ring between device records and the store file.

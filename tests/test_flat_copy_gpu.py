@@ -294,3 +294,22 @@ def test_flat_fanout(gpu, n_src, n_dst, heads, dim, dt, layout, rot):
     ops.scatter(tables[1], ids, offs, staging, shared_records=False)
     torch.cuda.synchronize()
     assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
+
+
+@pytest.mark.parametrize("n,rot", [(1, 128), (7, 128), (8, 128), (60, 20), (1024, 128)])
+def test_delta_tables_on_the_device(gpu, n, rot):
+    """The device's float64 tables (more than a kernel's arguments hold) are the
+    host's within one float32 unit in the last place."""
+    from daser_amd import position
+
+    print(f"case: delta tables {n} x {rot}", flush=True)
+    rng = np.random.default_rng(n)
+    deltas = rng.integers(-32768, 32768, n).tolist()
+    host = position.delta_tables(deltas, rot, 500000.0)
+    dev = position.delta_tables(deltas, rot, 500000.0, device=gpu)
+    torch.cuda.synchronize()
+    assert dev.shape == host.shape and dev.dtype == torch.float32
+    diff = (dev.cpu().double() - host.double()).abs()
+    assert (diff <= host.double().abs() * 2.0 ** -23 + 2.0 ** -60).all()
+    # float64 sine and cosine of the same product, rounded once: nearly all the same bits
+    assert (diff == 0).double().mean() > 0.999

@@ -39,6 +39,7 @@ class StorePlan:
     arena_bytes: int
     gather: Optional[object] = None  # ops.PreparedGather bound to the step's arena
     on_side: bool = False  # gathers run on the plane's side stream
+    uploaded: Optional[tuple] = None  # (stream handle, event) of the page tables' upload
 
 
 @dataclass
@@ -317,8 +318,15 @@ class KVDataPlane:
             per_layer = plan.page_ids.size * self.table.layout.layer_bytes
             plan.on_side = self._side is not None and (
                 self.save_stream == "side" or per_layer >= SIDE_STREAM_MIN_LAYER_BYTES)
-            if plan.on_side:
-                arena.record_stream(self._side)  # freed only after the side stream's gathers
+            if plan.on_side:  # freed only after the side stream's gathers
+                arena.record_stream(self._side)
+                plan.gather.tables[0].record_stream(self._side)
+            if self.device.type == "cuda":
+                # the upload is asynchronous: a layer saved from another stream waits for it
+                cur = torch.cuda.current_stream(self.device)
+                ev = torch.cuda.Event()
+                ev.record(cur)
+                plan.uploaded = (cur.cuda_stream, ev)
         return arena
 
     def _save_stream(self, plan: StorePlan) -> int:
@@ -326,6 +334,8 @@ class KVDataPlane:
         ordered after the work the model's stream has enqueued so far (the
         layer's KV writes); or the current stream."""
         cur = torch.cuda.current_stream(self.device)
+        if plan.uploaded is not None and plan.uploaded[0] != cur.cuda_stream:
+            cur.wait_event(plan.uploaded[1])
         if not plan.on_side:
             return cur.cuda_stream
         if self._save_ev is None:

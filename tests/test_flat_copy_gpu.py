@@ -313,3 +313,29 @@ def test_delta_tables_on_the_device(gpu, n, rot):
     assert (diff <= host.double().abs() * 2.0 ** -23 + 2.0 ** -60).all()
     # float64 sine and cosine of the same product, rounded once: nearly all the same bits
     assert (diff == 0).double().mean() > 0.999
+
+
+@pytest.mark.parametrize("save_stream", ["current", "side"])
+def test_saves_from_another_stream_wait_for_the_tables(gpu, tmp_path, save_stream):
+    """The page tables of a step are uploaded behind the stream's earlier work
+    (here a delay); layers saved from another stream still read whole tables."""
+    from daser_amd.connector import ReqStoreSpec
+    from daser_amd.data_plane import KVDataPlane, plan_store
+
+    print(f"case: saves on another stream, {save_stream}", flush=True)
+    whole, views, ids, _ = _setup(gpu, 40, 3, 16, 2, 64, "nhd", 5)
+    plane = KVDataPlane(str(tmp_path / "s"), save_stream=save_stream, io_backend="python")
+    slot = plane.register({f"model.layers.{i}.self_attn.attn": v for i, v in enumerate(views)})
+    plan = plan_store({"r": ReqStoreSpec("k", 0, ids.size, ids.tolist(), 0, 16 * ids.size)}, slot)
+    want = _records(views, ids)
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(20_000_000)
+        arena = plane.new_store_arena(plan)
+    with torch.cuda.stream(second):
+        for name in plane.layer_idx:
+            plane.save_layer(name, plan, arena)
+    torch.cuda.synchronize()
+    assert torch.equal(arena.view(torch.int16), want.view(torch.int16).flatten())
+    plane.close()

@@ -305,9 +305,10 @@ def delta_tables(
     device = torch.device(device)
     if cuda:  # stream-ordered, without blocking the host
         out = torch.empty(t.shape, dtype=torch.float32, device=device)
-        _lib.check("dsr_put", _lib.lib().dsr_put(
-            out.data_ptr(), t.data_ptr(), 4 * t.numel(),
-            torch.cuda.current_stream(device).cuda_stream))
+        with torch.cuda.device(device):
+            _lib.check("dsr_put", _lib.lib().dsr_put(
+                out.data_ptr(), t.data_ptr(), 4 * t.numel(),
+                torch.cuda.current_stream(device).cuda_stream))
         return out
     return t.to(device)
 
@@ -322,8 +323,9 @@ def _device_tables(deltas: np.ndarray, inv: np.ndarray, device: torch.device) ->
     flat[:n], flat[n:] = deltas[:, 0], inv
     x = host.to(device, non_blocking=True)
     out = torch.empty((n, half, 2), dtype=torch.float32, device=device)
-    _lib.check("dsr_delta_tables", _lib.lib().dsr_delta_tables(
-        x.data_ptr(), n, half, out.data_ptr(), torch.cuda.current_stream(device).cuda_stream))
+    with torch.cuda.device(device):
+        _lib.check("dsr_delta_tables", _lib.lib().dsr_delta_tables(
+            x.data_ptr(), n, half, out.data_ptr(), torch.cuda.current_stream(device).cuda_stream))
     return out
 
 

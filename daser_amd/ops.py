@@ -183,10 +183,14 @@ def _stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def _on_device(x) -> bool:
+    return isinstance(x, torch.Tensor) and not x.is_cpu
+
+
 def _as_device_table(
     x, dtype: torch.dtype, device: torch.device, name: str
 ) -> torch.Tensor:
-    if isinstance(x, torch.Tensor) and x.device.type != "cpu":
+    if _on_device(x):
         if x.dtype != dtype or not x.is_contiguous():
             raise ValueError(f"{name} must be a contiguous {dtype} tensor")
         return x
@@ -211,7 +215,7 @@ def _upload(arr: torch.Tensor, device: torch.device) -> torch.Tensor:
 
 def _host_array(x, np_dtype) -> Optional[np.ndarray]:
     if isinstance(x, torch.Tensor):
-        if x.device.type != "cpu":
+        if not x.is_cpu:
             return None
         return x.numpy().astype(np_dtype, copy=False)
     return np.asarray(x, dtype=np_dtype)
@@ -500,7 +504,9 @@ def _gather_tables(table: LayerTable, page_ids, slot_offsets, staging, layer0, l
     """Checked device tables (page_ids, slot_offsets) of a gather and, of host
     tables, the plan that holds them."""
     lay = table.layout
-    ids, offs = _host_list(page_ids), _host_list(slot_offsets)
+    ids = offs = None
+    if not _on_device(page_ids):
+        ids, offs = _host_list(page_ids), _host_list(slot_offsets)
     if ids is None or offs is None or not ids.size or lay.device.type != "cuda":
         return _copy_args(table, page_ids, slot_offsets, staging, layer0, layers,
                           records_written=True)[1], None
@@ -539,7 +545,8 @@ def scatter(
     once and written to all of its pages) where the pages allow it, device
     tables a launch shaped for cache-served reads. None: inferred from host
     ``slot_offsets`` (at most half of them distinct), False for device
-    tables. Results do not depend on it."""
+    tables. Results do not depend on it. Host tables are planned by the library
+    (dsr_plan_load) and uploaded once."""
     host = _host_tables(table, page_ids, slot_offsets)
     if host is not None:
         _load_host(table, *host, staging, layer0, layers, shared_records)
@@ -561,6 +568,8 @@ def scatter(
 def _host_tables(table: LayerTable, page_ids, slot_offsets):
     """(page_ids, slot_offsets) as host vectors if the library can plan them:
     both on the host, not empty, of one length."""
+    if _on_device(page_ids):
+        return None
     ids, offs = _host_list(page_ids), _host_list(slot_offsets)
     if ids is None or offs is None or not ids.size or ids.size != offs.size or \
             table.layout.device.type != "cuda":
@@ -828,7 +837,7 @@ def scatter_rerotate(
 def _slots_args(table: LayerTable, slot_mapping, row_offsets, staging, layer0, layers,
                 records_written: bool):
     lay = table.layout
-    if not lay.has_geometry or lay.k_layout != "nhd":
+    if lay.k_layout != "nhd" or not lay.has_geometry:
         raise ValueError("the token form needs token-major pages ([block_size][H][D]) of "
                          "known geometry")
     first, count = (0, lay.num_layers) if layers is None else layers
@@ -884,6 +893,8 @@ def _slots_host(table: LayerTable, slot_mapping, row_offsets, staging: torch.Ten
     pages (loads) through the page form, the other tokens through the token
     kernels. ``rope`` as for :func:`_load_host`. False, having done nothing, for
     tables that the library cannot plan (device tables, empty or odd ones)."""
+    if _on_device(slot_mapping):
+        return False
     lay = table.layout
     sm, ro = _host_list(slot_mapping), _host_list(row_offsets)
     if sm is None or ro is None or not sm.size or sm.size != ro.size or \

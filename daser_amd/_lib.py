@@ -201,8 +201,9 @@ def check(fn: str, code: int) -> None:
 
 def set_tuning(knob: str, value) -> None:
     """Launch-shape override for measurements and tests (``TUNE`` names;
-    ``rot_kernel`` also takes "auto" / "pairs" / "contig" / "grouped",
-    ``slots_kernel`` "small"); 0 or "auto" restores the default."""
+    ``rot_kernel`` also takes "auto" / "pairs"); 0 or "auto" restores the
+    default. Names and values that no kernel uses any more are accepted and
+    have no effect."""
     if knob == "rot_kernel" and isinstance(value, str):
         value = ROT_KERNEL_CODES[value]
     elif knob == "slots_kernel" and isinstance(value, str):

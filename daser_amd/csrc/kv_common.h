@@ -14,7 +14,6 @@
 namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;     // 4 wave64 per workgroup
 constexpr int kWave = 64;
@@ -25,9 +24,9 @@ constexpr int kMaxRotHalf = 512;   // LDS table capacity: rot_dim <= 1024
 constexpr int kXcds = 8;           // MI355X: 8 XCDs, workgroups dealt round-robin
 
 // Cache-policy bits of gfx950 buffer instructions (CPol: sc0 = 1, nt = 2,
-// sc1 = 16). Loads stream through (nt); stores are written with sc0 sc1,
-// which measured fastest for these write-once streams (6.0 vs 5.2 TB/s for
-// default-policy stores at the Llama-3-8B shape).
+// sc1 = 16). Loads stream through (nt). The pair-task and LDS re-rotations, one
+// workgroup per unit, store with sc0 sc1 (6.0 vs 5.2 TB/s for default-policy
+// stores from such workgroups at the Llama-3-8B shape).
 constexpr int kLoadPolicy = 2;
 constexpr int kStorePolicy = 17;
 // The flat copies' stores: nt for launches that the caches can absorb, nt sc0
@@ -70,10 +69,9 @@ struct UnitArgs {
   int32_t hnd_row_vecs = 0;
 };
 
-// Workgroup -> unit. Hardware deals consecutive workgroup ids round-robin
+// Workgroup -> unit, for the kernels of one workgroup per unit. Hardware deals consecutive workgroup ids round-robin
 // over the 8 XCDs; remapping so that each XCD walks one contiguous eighth of
-// the unit list keeps each XCD's stream of records contiguous (measured
-// +2% over the identity mapping for the gather). Returns -1 past the end.
+// the unit list keeps each XCD's stream contiguous. Returns -1 past the end.
 __device__ __forceinline__ int64_t xcd_unit(int64_t n_units) {
   const int64_t per = (n_units + kXcds - 1) / kXcds;
   const int64_t b = blockIdx.x;
@@ -81,8 +79,7 @@ __device__ __forceinline__ int64_t xcd_unit(int64_t n_units) {
   return u < n_units ? u : -1;
 }
 
-// Workgroup -> unit for the kernels that write the paged cache (scatter and
-// re-rotation). The unit list is walked layer-major (all pages of layer 0,
+// The same, layer-major: the unit list is walked layer-major (all pages of layer 0,
 // then layer 1, ...) and each XCD takes one contiguous eighth of it, so each
 // XCD writes the (destination-ordered) pages of a few layers in sequence
 // instead of interleaving 32 layer regions. Measured in-process against the
@@ -133,10 +130,6 @@ __device__ __forceinline__ rsrc_t make_rsrc(const uint8_t* p, int64_t bytes) {
 }
 __device__ __forceinline__ u32x4 bload(rsrc_t r, int off) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kLoadPolicy);
-}
-// 8-byte load with the default (cached) policy, for small shared tables
-__device__ __forceinline__ u32x2 bload_b64(rsrc_t r, int off) {
-  return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
 }
 __device__ __forceinline__ void bstore(rsrc_t r, int off, u32x4 v) {
   __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kStorePolicy);

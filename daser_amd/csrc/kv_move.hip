@@ -109,15 +109,6 @@ int64_t max_wg_per_launch() {
   return m;
 }
 
-// Items (pages or tokens) per launch such that ceil(items * n_layers /
-// per_wg), rounded up to the XCD count, stays within max_wg_per_launch();
-// per_wg = items' units per workgroup (G pages or a block of tokens).
-int64_t items_per_launch(int n_layers, int64_t per_wg) {
-  const int64_t wg = max_wg_per_launch() - kXcds;
-  const int64_t per = wg * per_wg / n_layers;
-  return per > 0 ? per : 0;
-}
-
 // Launches over consecutive page ranges of `a` (one launch unless the pages
 // exceed max_wg_per_launch()), each range's tables offset to its first
 // page; launch(b, grid) enqueues one kernel. Grids are a whole multiple of
@@ -125,7 +116,7 @@ int64_t items_per_launch(int n_layers, int64_t per_wg) {
 // launch error.
 template <class F>
 int launch_page_ranges(const UnitArgs& a, int n_pages, F launch) {
-  const int64_t per = items_per_launch(a.n_layers, 1);
+  const int64_t per = (max_wg_per_launch() - kXcds) / a.n_layers;
   if (per <= 0) return DSR_ERR_ARG;
   for (int64_t p0 = 0; p0 < n_pages; p0 += per) {
     const int64_t n = n_pages - p0 < per ? n_pages - p0 : per;
@@ -511,8 +502,8 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
   ra.k_scale = k_scale;
   hipStream_t s = (hipStream_t)stream;
   if (hnd_block > 0) {
-    // head-major pages: the contig or grouped kernels (rows and partners
-    // stay whole in record order; the cache side goes through hnd_vec)
+    // head-major pages: rows and partners stay whole in record order, the cache
+    // side goes through hnd_vec
     const int h = ra.half_vecs;
     const bool contig = vec_ok && (rope_style == DSR_ROPE_GPTJ ||
                                    (h > 0 && h <= 32 && (h & (h - 1)) == 0 &&
@@ -1149,7 +1140,7 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
       return DSR_ERR_SHAPE;
     const int64_t row_bytes = (int64_t)head_dim * esize;
     if (row_bytes % 16 || page_bytes % row_bytes) return DSR_ERR_SHAPE;
-    // the contig kernel's vector geometry: whole-vector rotary widths, neox
+    // the vector map's geometry: whole-vector rotary widths, neox
     // partners a power of two <= 32 vectors apart inside a row
     const bool vec_ok = ((int64_t)(head_dim - rot_dim) * esize) % 16 == 0 &&
                         (rope_style == DSR_ROPE_NEOX ? (rot_dim / 2) % ve == 0 : rot_dim % ve == 0);
@@ -1171,7 +1162,7 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
     dt = dtype;
     style = rope_style;
     if (k_layout == DSR_K_KX) {
-      // the contig kernel's split-x conditions: head blocks of a power-of-two
+      // the vector map's split-x conditions: head blocks of a power-of-two
       // number (>= 64) of vectors, power-of-two block size, neox partners a
       // multiple of 32 vectors apart
       const int64_t hv = row_bytes / 16 * block_size;

@@ -437,22 +437,6 @@ struct VRound {
       if (i < nvec) bstore(rd, i << 4, r[k]);
     }
   }
-  // head-major cache page: vector i of the round goes to cache vector hnd_vec(i)
-  __device__ __forceinline__ void store_hnd(const UnitArgs& a, rsrc_t rd, int base, int nvec) {
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = base + k * kThreads;
-      if (i < nvec) bstore(rd, hnd_vec(a, i) << 4, r[k]);
-    }
-  }
-  // K of a split-x page: vector i of the round is physical vector kx_phys(i)
-  __device__ __forceinline__ void load_kx(const RotArgs& ra, rsrc_t rs, int base, int nvec) {
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = base + k * kThreads;
-      r[k] = i < nvec ? bload(rs, kx_phys(ra, i) << 4) : u32x4{0u, 0u, 0u, 0u};
-    }
-  }
 };
 
 // One workgroup per (page, layer) unit in page-list order. V, and K of pages

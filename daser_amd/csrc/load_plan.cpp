@@ -26,7 +26,7 @@ class Distinct {
  public:
   explicit Distinct(int n) {
     int log = 4;
-    while ((1 << log) < 2 * (int64_t)n && log < 30) ++log;
+    while (((int64_t)1 << log) < 2 * (int64_t)n) ++log;
     shift_ = 64 - log;
     mask_ = ((uint64_t)1 << log) - 1;
     place_.assign((size_t)mask_ + 1, -1);

@@ -1022,9 +1022,10 @@ def reference_loop(torch, dev, budget_s: float = 6.0) -> dict:
             "sample": f"{wl.n_pages} pages x 32 layers, {n} save+load rounds in {el:.1f} s"}
 
 
-# the re-rotation kernel each configuration's launch selects (by page size)
-ROT_KERNEL = {3: "kv_scatter_rerotate_grouped_kernel", 5: "kv_scatter_rerotate_grouped_kernel",
-              6: "kv_scatter_rerotate_grouped_kernel"}
+# the page copies' and the per-page re-rotation's kernels (one kernel template for
+# both directions; the traffic records name the direction)
+GATHER_KERNEL, SCATTER_KERNEL = "kv_flat_copy_kernel<gather>", "kv_flat_copy_kernel<scatter>"
+ROT_KERNEL = "kv_flat_rerotate_kernel"
 
 
 def frac_hbm(traffic, ms):
@@ -1219,8 +1220,7 @@ def main() -> int:
         })
         dom = "gather" if r["gather_ms"] >= r["scatter_ms"] else "scatter"
         achieved = r[f"{dom}_GBps"]
-        # the one-unit kernels the launch policy picks for 32 KiB pages
-        kname = "kv_gather_kernel" if dom == "gather" else "kv_scatter_stream_kernel"
+        kname = GATHER_KERNEL if dom == "gather" else SCATTER_KERNEL
         out["roofline"] = {
             "kernel": kname,
             "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
@@ -1242,11 +1242,11 @@ def main() -> int:
         out["kernels"]["scatter_slots"] = {
             "ms": round(r["slots_scatter_ms"], 4), "GBps": round(r["slots_scatter_GBps"], 1),
             "frac": round(r["slots_scatter_GBps"] / HBM_PEAK_GBS, 4),
-            "path": "kv_scatter_stream_kernel + kv_slots_kernel: " + split}
+            "path": "kv_flat_copy_kernel + kv_slots_flat_kernel: " + split}
         out["kernels"]["scatter_slots_rerotate"] = {
             "ms": round(r["slots_rerotate_ms"], 4), "GBps": round(r["slots_rerotate_GBps"], 1),
             "frac": round(r["slots_rerotate_GBps"] / HBM_PEAK_GBS, 4),
-            "path": "kv_scatter_rerotate_grouped_kernel + kv_slots_rerotate_kernel: " + split}
+            "path": "kv_flat_rerotate_kernel + kv_slots_flat_rerotate_kernel: " + split}
         out["check"] = {"round_trip_probe": r["probe_ok"]}
     for c in (3, 5, 6):
         if c in res:
@@ -1263,8 +1263,8 @@ def main() -> int:
                 **({"same_pages_slots_gather_GBps": round(r["slots_gather_GBps"], 1),
                     "same_pages_slots_scatter_GBps": round(r["slots_scatter_GBps"], 1)}
                    if "slots_gather_GBps" in r else {}),
-                "kernel": ROT_KERNEL[c],
-                "traffic": pmc_traffic(ROT_KERNEL[c], c, r["pages"]),
+                "kernel": ROT_KERNEL,
+                "traffic": pmc_traffic(ROT_KERNEL, c, r["pages"]),
                 "algorithmic_bytes": 2 * r["payload_bytes"]}
             out[f"rerotate_cfg{c}"]["frac_hbm"] = frac_hbm(
                 out[f"rerotate_cfg{c}"]["traffic"], r["kernel_ms"])
@@ -1301,14 +1301,14 @@ def main() -> int:
                            "rerotate_ms": round(r.get("rerotate_ms", 0.0), 4),
                            "rerotate_e5m2_GBps": round(r.get("rerotate_e5m2_GBps", 0.0), 1),
                            "tokens": r["tokens"], "payload_bytes": r["payload_bytes"],
-                           "traffic_rerotate": pmc_traffic("kv_scatter_rerotate_contig_kernel", 4,
+                           "traffic_rerotate": pmc_traffic(ROT_KERNEL, 4,
                                                            r["pages"])}
         f8 = out["fp8_cfg4"]
         f8["frac"] = {k: round(r[f"{k}_GBps"] / HBM_PEAK_GBS, 4)
                       for k in ("gather", "scatter", "rerotate") if r.get(f"{k}_GBps")}
         f8["frac_hbm"] = {
-            "gather": frac_hbm(pmc_traffic("kv_gather_kernel", 4, r["pages"]), r["gather_ms"]),
-            "scatter": frac_hbm(pmc_traffic("kv_scatter_kernel", 4, r["pages"]), r["scatter_ms"]),
+            "gather": frac_hbm(pmc_traffic(GATHER_KERNEL, 4, r["pages"]), r["gather_ms"]),
+            "scatter": frac_hbm(pmc_traffic(SCATTER_KERNEL, 4, r["pages"]), r["scatter_ms"]),
             "rerotate": frac_hbm(f8["traffic_rerotate"], r.get("rerotate_ms"))}
     if "value" not in out and configs:
         r = res[configs[0]]

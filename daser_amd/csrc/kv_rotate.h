@@ -25,17 +25,26 @@ __device__ __forceinline__ uint32_t f32_to_bf16(float f) {
 __device__ __forceinline__ float fp16_to_f32(uint32_t h) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
-// fp32 -> fp16 by the hardware conversion (round-to-nearest-even), of the fp32
-// value itself: a multiply-add that the compiler fuses with the conversion
-// (v_fma_mixlo_f16) rounds otherwise, here and there by kernel.
-__device__ __forceinline__ uint32_t f32_bits_fp16(float f) {
+// fp32 -> fp16 by the hardware conversion (round-to-nearest-even) of the fp32
+// value itself; NaN -> 0x7E00.
+__device__ __forceinline__ uint32_t f32_to_fp16(float f) {
+  if (__builtin_isnan(f)) return 0x7e00u;
   asm("" : "+v"(f));
   return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
 }
-// The same with NaN -> 0x7E00.
-__device__ __forceinline__ uint32_t f32_to_fp16(float f) {
-  if (__builtin_isnan(f)) return 0x7e00u;
-  return f32_bits_fp16(f);
+// a * b + t rounded once, to fp16: the vector kernels' fp16 sums. The compiler
+// fuses the conversion in some kernels and not in others; by name, every kernel
+// rounds alike, and once.
+__device__ __forceinline__ uint32_t fma_fp16(float a, float b, float t) {
+  _Float16 h;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(a), "v"(b), "v"(t));
+  return (uint32_t)__builtin_bit_cast(uint16_t, h);
+}
+// The two halves of w with NaN -> 0x7E00.
+__device__ __forceinline__ uint32_t canonical_fp16(uint32_t w) {
+  if ((w & 0x7fffu) > 0x7c00u) w = (w & 0xffff0000u) | 0x7e00u;
+  if ((w & 0x7fff0000u) > 0x7c000000u) w = (w & 0xffffu) | 0x7e000000u;
+  return w;
 }
 
 // OCP e4m3fn (bias 7, no infinities, S.1111.111 = NaN) through the gfx950
@@ -163,15 +172,22 @@ struct Codec<DSR_DTYPE_FP16> {
     return v;
   }
   static constexpr uint32_t kSigns = 0x80008000u;
-  __device__ static bool encode_quick(const float* y, u32x4* v) {
+  // the rotated sums x * c + t themselves; c: the cosine of element e is c[e / per].x
+  template <int per>
+  __device__ static u32x4 encode_sums(const float* x, const float2* c, const float* t) {
+    u32x4 v;
     uint32_t odd = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const uint32_t w = f32_bits_fp16(y[2 * k]) | f32_bits_fp16(y[2 * k + 1]) << 16;
-      odd |= (w & 0x7fff7fffu) + 0x03ff03ffu;  // past infinity: bit 15
-      (*v)[k] = w;
+      const int e = 2 * k;
+      v[k] = fma_fp16(x[e], c[e / per].x, t[e]) |
+             fma_fp16(x[e + 1], c[(e + 1) / per].x, t[e + 1]) << 16;
+      odd |= (v[k] & 0x7fff7fffu) + 0x03ff03ffu;  // past infinity: bit 15
     }
-    return odd & kSigns;
+    if (odd & kSigns)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = canonical_fp16(v[k]);
+    return v;
   }
 };
 
@@ -304,55 +320,61 @@ __device__ __forceinline__ int table_column(const RotArgs& ra, int c) {
 // bytes, partner (neox) the bytes of the vector half a rotation away, cs the
 // pairs of its column. Vectors past the rotated region are returned unchanged.
 // kScaled: the values are multiplied by the layer's scale first and by its
-// inverse after. The sums are fused by name, so that every kernel rounds alike.
+// inverse after. The sums are fused by name (the cosine's product exact), so that
+// every kernel rounds alike.
 template <int DT, int STYLE, bool kScaled>
 __device__ __forceinline__ u32x4 rotate_pairs(const RotArgs& ra, u32x4 own, u32x4 partner, int c,
                                               const float2* cs, float scale, float inv_scale) {
   using C = Codec<DT>;
   constexpr int VE = C::VE;
-  float x[VE];
+  constexpr int kPer = STYLE == DSR_ROPE_NEOX ? 1 : 2;  // elements per pair
+  float x[VE], t[VE];  // t: the sines' products
   C::decode(own, x);
+  if (kScaled) {
+#pragma unroll
+    for (int e = 0; e < VE; ++e) x[e] *= scale;
+  }
   if (STYLE == DSR_ROPE_NEOX) {
     // first half: x c - p s; second half: x c + p s. The sign goes into the
     // partner's bits, which is exact.
     const uint32_t flip = c < ra.half_vecs ? C::kSigns : 0u;
-    float z[VE];
-    C::decode(partner ^ flip, z);
+    C::decode(partner ^ flip, t);
 #pragma unroll
-    for (int e = 0; e < VE; ++e) {
-      const float xo = kScaled ? x[e] * scale : x[e];
-      const float xp = kScaled ? z[e] * scale : z[e];
-      const float y = __builtin_fmaf(xp, cs[e].y, xo * cs[e].x);
-      x[e] = kScaled ? y * inv_scale : y;
-    }
+    for (int e = 0; e < VE; ++e) t[e] = (kScaled ? t[e] * scale : t[e]) * cs[e].y;
   } else {
 #pragma unroll
-    for (int e = 0; e < VE / 2; ++e) {
-      const float x1 = kScaled ? x[2 * e] * scale : x[2 * e];
-      const float x2 = kScaled ? x[2 * e + 1] * scale : x[2 * e + 1];
-      const float y1 = __builtin_fmaf(-x2, cs[e].y, x1 * cs[e].x);
-      const float y2 = __builtin_fmaf(x1, cs[e].y, x2 * cs[e].x);
-      x[2 * e] = kScaled ? y1 * inv_scale : y1;
-      x[2 * e + 1] = kScaled ? y2 * inv_scale : y2;
+    for (int e = 0; e < VE; e += 2) {
+      t[e] = -x[e + 1] * cs[e / 2].y;
+      t[e + 1] = x[e] * cs[e / 2].y;
     }
   }
   u32x4 v;
-  if (C::encode_quick(x, &v)) v = C::encode(x);
+  if constexpr (DT == DSR_DTYPE_FP16) {
+    v = C::template encode_sums<kPer>(x, cs, t);
+  } else {
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+      const float y = __builtin_fmaf(x[e], cs[e / kPer].x, t[e]);
+      x[e] = kScaled ? y * inv_scale : y;
+    }
+    if (C::encode_quick(x, &v)) v = C::encode(x);
+  }
   return c >= ra.rot_vecs ? own : v;
 }
 
-// The scale of an 8-bit layer cancels: R(s k) / s = R(k), with two roundings
-// less for each value. Scales whose inverse or products leave fp32's range
-// (zero, infinities, NaN among them) keep the multiplications and what they
-// give.
-__device__ __forceinline__ bool scale_cancels(float scale) {
-  const float m = __builtin_fabsf(scale);
-  return m >= 0x1p-100f && m <= 0x1p+100f;
+// An 8-bit layer's scale is multiplied in and its inverse out again: two
+// roundings of each value that decide a few ties. A power of two rounds nothing, so
+// it is left out (1.0, the scale of uncalibrated caches, among them); the range
+// keeps every product normal. The multiplications cost a Llama-3-8B e4m3 load
+// nothing, 70B and TP8 loads 1%, Gemma-2-9B head-major ones 2%.
+__device__ __forceinline__ bool scale_is_exact(float scale) {
+  const uint32_t u = __float_as_uint(scale) & 0x7fffffffu;
+  return (u & 0x007fffffu) == 0 && u >= 0x2f800000u && u <= 0x4f800000u;  // 2^-32 to 2^32
 }
 template <int DT, int STYLE>
 __device__ __forceinline__ u32x4 rotate_vec(const RotArgs& ra, u32x4 own, u32x4 partner, int c,
                                             const float2* cs, float scale, float inv_scale) {
-  if (is_fp8<DT>() && !scale_cancels(scale))
+  if (is_fp8<DT>() && !scale_is_exact(scale))
     return rotate_pairs<DT, STYLE, true>(ra, own, partner, c, cs, scale, inv_scale);
   return rotate_pairs<DT, STYLE, false>(ra, own, partner, c, cs, scale, inv_scale);
 }
@@ -627,7 +649,7 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_lds_kernel(RotAr
   if (kScaled) {
     scale = ra.k_scale[ra.u.layer0 + l];
     inv_scale = 1.0f / scale;
-    if (scale_cancels(scale)) scale = inv_scale = 1.0f;
+    if (scale_is_exact(scale)) scale = inv_scale = 1.0f;
   }
   const uint32_t* bw = reinterpret_cast<const uint32_t*>(buf);
   const int rv = ra.row_vecs, half = ra.rot_half, rot = 2 * ra.rot_half;
@@ -665,7 +687,7 @@ __global__ __launch_bounds__(kThreads) void kv_scatter_rerotate_lds_kernel(RotAr
         const float2 cs = tab[jj];
         const float xo = kScaled ? x[e] * scale : x[e];
         const float xp = kScaled ? pv * scale : pv;
-        const float y = __builtin_fmaf(sg * xp, cs.y, xo * cs.x);
+        const float y = __builtin_fmaf(xo, cs.x, sg * xp * cs.y);
         x[e] = kScaled ? y * inv_scale : y;
         mask[e / PER] |= ((1u << EB) - 1u) << (EB * (e % PER));
       }

@@ -754,6 +754,8 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   a.layer0 = layer0;
   a.block_size = block_size;
   a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
+  const int64_t vpr = row_bytes >> 4;
+  a.least_row = vpr <= 8 && (vpr & (vpr - 1)) == 0 && a.block_shift >= 0 ? 0 : INT64_MIN;
   const SlotShape h = slot_shape(&a);
   if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   const bool large = slots_large(a);
@@ -825,6 +827,7 @@ int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_s
   a.layer0 = layer0;
   a.block_size = block_size;
   a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
+  a.least_row = INT64_MIN;
   RotArgs ra{};
   ra.u.layer0 = layer0;
   ra.cos_sin = reinterpret_cast<const float2*>(cos_sin);

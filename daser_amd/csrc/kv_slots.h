@@ -35,6 +35,7 @@ struct SlotArgs {
   int32_t block_size;
   int32_t block_shift;  // log2(block_size) when a power of two, else -1
   int32_t unit_tokens;  // tokens per unit
+  int64_t least_row;    // the smallest row offset taken (dsr_gather_slots)
   FastDiv row;          // wide rows: pieces per row; others: vectors per row
 };
 
@@ -81,10 +82,10 @@ __device__ __forceinline__ bool slot_pos(const SlotArgs& a, const FlatMap& m, Sl
   }
   const int64_t t = (int64_t)tb * a.unit_tokens + in_unit;
   if (t >= a.n_tokens) return false;
-  const int64_t slot = a.slot_mapping[t];
-  const int64_t off = a.row_offsets[t] + (int64_t)(a.layer0 + (int)l) * a.layer_bytes;
+  const int64_t slot = a.slot_mapping[t], row = a.row_offsets[t];
+  const int64_t off = row + (int64_t)(a.layer0 + (int)l) * a.layer_bytes;
   const int64_t blk = slot >= 0 ? slot_block(a, slot) : -1;
-  if (blk < 0 || blk >= a.num_blocks) return false;
+  if (blk < 0 || blk >= a.num_blocks || row < a.least_row) return false;
   if (off < 0 || off + a.page_bytes + a.row_bytes > a.staging_bytes) return false;
   o->cache = reinterpret_cast<uint8_t*>(a.layer_base[l]) + blk * a.page_stride +
              (slot - blk * a.block_size) * a.row_bytes;

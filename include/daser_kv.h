@@ -413,7 +413,11 @@ int dsr_scatter_rerotate_hnd(const uint64_t* layer_base, int n_layers,
  *                   + (slot % block_size) * row_bytes
  * to  staging + row_offsets[t] + (layer0 + l) * layer_bytes,
  * and its V row (+ kv_stride in the cache) to the same place + page_bytes.
- * Tokens with slot < 0 (vLLM's padding) are skipped. With row_offsets[t] =
+ * Tokens with slot < 0 (vLLM's padding) are skipped, and so are out-of-range
+ * slots and, layer by layer, rows that leave the staging buffer. Rows of 16, 32, 64
+ * or 128 bytes in blocks of a power of two tokens are skipped in every layer if
+ * row_offsets[t] is negative (dsr_scatter_slots alike); for others its place in
+ * the layer alone counts, so that a buffer may hold the later layers only. With row_offsets[t] =
  * record(t / block_size) + (t % block_size) * row_bytes this writes exactly
  * the slot records of dsr_gather, restricted to the valid tokens (a partial
  * last page leaves its tail rows untouched).

@@ -339,3 +339,43 @@ def test_saves_from_another_stream_wait_for_the_tables(gpu, tmp_path, save_strea
     torch.cuda.synchronize()
     assert torch.equal(arena.view(torch.int16), want.view(torch.int16).flatten())
     plane.close()
+
+
+@pytest.mark.parametrize("heads,dim,skipped", [(1, 8, True), (1, 16, True), (1, 32, True),
+                                               (1, 64, True), (3, 8, False), (1, 128, False),
+                                               (8, 128, False)])
+@pytest.mark.parametrize("load", [False, True])
+def test_negative_row_offsets(gpu, heads, dim, skipped, load):
+    """Device tables with row offsets below the staging buffer. Power-of-two
+    rows of up to 128 bytes: the token is skipped in every layer; others: in the
+    layers where its row lies outside."""
+    print(f"case: negative rows H{heads} D{dim} load {load}", flush=True)
+    layers, block, n = 3, 4, 6
+    whole, views, _, _ = _setup(gpu, n, layers, block, heads, dim, "nhd", seed=dim)
+    table = ops.LayerTable(views)
+    lay, row = table.layout, heads * dim * 2
+    slots = np.arange(6, dtype=np.int64)
+    rows = lay.slot_bytes + np.arange(6) * row
+    rows[1], rows[4] = -16, -16 - 2 * row  # in layers 1 and 2: the first record's part
+    rows[5] = lay.slot_bytes + row
+    g = torch.Generator(device=gpu).manual_seed(3)
+    staging = torch.randint(0, 256, (2 * lay.slot_bytes,), generator=g, device=gpu,
+                            dtype=torch.uint8)
+    cells = whole.view(torch.uint8).view(layers, 2, -1, row)  # by slot
+    want_s, want_c = staging.clone(), cells.clone()
+    for t, (s, r) in enumerate(zip(slots, rows)):
+        for layer in range(layers):
+            off = int(r) + layer * lay.layer_bytes
+            if off < 0 or (r < 0 and skipped):
+                continue
+            for half in range(2):
+                at = slice(off + half * lay.page_bytes, off + half * lay.page_bytes + row)
+                if load:
+                    want_c[layer, half, s] = staging[at]
+                else:
+                    want_s[at] = cells[layer, half, s]
+    fn = ops.scatter_slots if load else ops.gather_slots
+    fn(table, torch.from_numpy(slots).to(gpu), torch.from_numpy(rows).to(gpu), staging)
+    torch.cuda.synchronize()
+    assert torch.equal(staging, want_s)
+    assert torch.equal(whole.view(torch.uint8).view(layers, 2, -1, row), want_c)

@@ -226,10 +226,10 @@ int dsr_plan_slots(const int64_t* slots, const int64_t* rows, const int64_t* rop
     if (rope_idx && (rope_idx[i] < -1 || rope_idx[i] >= n_tables)) return DSR_PLAN_ERR_ROPE;
     if (slots[i] < 0) continue;
     if (slots[i] >= num_slots) return DSR_PLAN_ERR_SLOT;
-    if (rows[i] < 0 || rows[i] > staging_bytes - row_end) return DSR_PLAN_ERR_ROW;
+    if (mode == 1 && check_record(rows[i], row_end, staging_bytes)) return DSR_PLAN_ERR_ROW;
     odd |= (rows[i] & 15) != 0;
   }
-  if (odd) return DSR_PLAN_ERR_ROWALIGN;
+  if (mode == 1 && odd) return DSR_PLAN_ERR_ROWALIGN;
   try {
     std::vector<int32_t> order;
     order.reserve(n);
@@ -272,6 +272,14 @@ int dsr_plan_slots(const int64_t* slots, const int64_t* rows, const int64_t* rop
         if (i + 1 == all.size() || slots[all[i]] != slots[all[i + 1]]) order.push_back(all[i]);
     }
     const int m = (int)order.size();
+    if (mode == 0) {  // a load: the rows that are read, not those of entries left out
+      odd = false;
+      for (int i = 0; i < m; ++i) {
+        if (check_record(rows[order[i]], row_end, staging_bytes)) return DSR_PLAN_ERR_ROW;
+        odd |= (rows[order[i]] & 15) != 0;
+      }
+      if (odd) return DSR_PLAN_ERR_ROWALIGN;
+    }
     // whole blocks: their first entry's index in `order`
     std::vector<int32_t> first;
     std::vector<uint8_t> paged((size_t)m, 0);

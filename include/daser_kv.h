@@ -520,9 +520,10 @@ int dsr_plan_gather(const int64_t* page_ids, const int64_t* slot_offsets, int n,
  * last layer that the call moves. mode 0: a load; blocks whose every slot is
  * listed with consecutive record rows and one table index become pages (for
  * dsr_plan_load: ids, offsets and rope as int64), the other tokens follow in slot
- * order; of a slot listed more than once the last one. mode 1: a save; tokens as
- * given, of a row listed more than once the last one. The sections from
- * off_slots on (slots and rows as int64, rope as int32) are one upload.
+ * order; of a slot listed more than once the last one, and the rows of the others
+ * are not checked. mode 1: a save; tokens as given, of a row listed more than
+ * once the last one. The sections from off_slots on (slots and rows as int64,
+ * rope as int32) are one upload.
  */
 #define DSR_PLAN_ERR_SLOT (-25)    /* a slot outside the block pool              */
 #define DSR_PLAN_ERR_ROW (-26)     /* a row outside the staging buffer           */

@@ -174,3 +174,18 @@ def test_plan_slots_refusals():
     assert call(slots, rows - 16, rope) == _lib.DSR_PLAN_ERR_ROW
     assert call(slots, rows + 8, rope, total=512) == _lib.DSR_PLAN_ERR_ROWALIGN
     assert call(slots, rows, rope, tables=1) == _lib.DSR_PLAN_ERR_ROPE
+
+
+@pytest.mark.parametrize("bad,code", [(-16, _lib.DSR_PLAN_ERR_ROW), (256, _lib.DSR_PLAN_ERR_ROW),
+                                      (8, _lib.DSR_PLAN_ERR_ROWALIGN)])
+@pytest.mark.parametrize("num_blocks", [2, 1 << 40])
+def test_plan_slots_rows_of_entries_left_out(bad, code, num_blocks):
+    """A load reads the last entry of a repeated slot: the rows of the ones before
+    are not looked at. A save refuses every bad row."""
+    slots, rows = np.array([5, 5, 2], np.int64), np.array([bad, 64, 0], np.int64)
+    rc, plan, out = _slots(slots, rows, None, num_blocks, 4, 64, 192, 256)
+    assert rc == 0 and plan.n_tokens == 2
+    assert np.array_equal(_section(out, plan.off_slots, 2, np.int64), [2, 5])
+    assert np.array_equal(_section(out, plan.off_rows, 2, np.int64), [0, 64])
+    assert _slots(slots, rows[[1, 0, 2]], None, num_blocks, 4, 64, 192, 256)[0] == code
+    assert _slots(slots, rows, None, num_blocks, 4, 64, 192, 256, mode=1)[0] == code

@@ -346,20 +346,24 @@ def _upload_plan(host: torch.Tensor, at: int, nbytes: int, device: torch.device,
 class _HostPlan:
     """Host tables of one call, planned by the library (dsr_plan_load,
     dsr_plan_gather) into one buffer and uploaded with one kernel (up to
-    DSR_PUT_BYTES) or one asynchronous copy from pinned memory. ``ptr`` holds
-    the device addresses of its sections."""
+    DSR_PUT_BYTES) or one asynchronous copy from pinned memory. ``offsets``,
+    ``start``, ``ids`` and ``rope`` are the addresses of its sections."""
 
     def __init__(self, n: int, device: torch.device, fill) -> None:
         """``fill(address, size, plan)`` has the library write the tables."""
-        if torch.cuda.is_current_stream_capturing():
+        cuda = device.type == "cuda"
+        if cuda and torch.cuda.is_current_stream_capturing():
             raise ValueError("host index tables cannot be used under graph capture: pass "
                              "device tensors")
         size = _lib.plan_bytes(n)
-        host = _plan_room(size)
+        host = _plan_room(size) if cuda else torch.empty(size, dtype=torch.uint8)
         self.plan = plan = _lib.Plan()
         fill(host.data_ptr(), size, ctypes.addressof(plan))
-        self.stream = _stream_handle(device)
-        self.buf = _upload_plan(host, 0, plan.bytes, device, self.stream)
+        if cuda:
+            self.stream = _stream_handle(device)
+            self.buf = _upload_plan(host, 0, plan.bytes, device, self.stream)
+        else:  # caches in host memory: the tables stay there
+            self.stream, self.buf = None, host[:plan.bytes]
         base = self.buf.data_ptr()
         self.offsets, self.start = base, base + plan.off_start
         self.ids, self.rope = base + plan.off_ids, base + plan.off_rope

@@ -6,6 +6,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from daser_amd import _lib, ops
 
@@ -189,3 +190,15 @@ def test_plan_slots_rows_of_entries_left_out(bad, code, num_blocks):
     assert np.array_equal(_section(out, plan.off_rows, 2, np.int64), [0, 64])
     assert _slots(slots, rows[[1, 0, 2]], None, num_blocks, 4, 64, 192, 256)[0] == code
     assert _slots(slots, rows, None, num_blocks, 4, 64, 192, 256, mode=1)[0] == code
+
+
+def test_fanout_tables_of_caches_in_host_memory():
+    """A fan-out load is prepared (checked, grouped) without a GPU."""
+    caches = [torch.zeros(2, 8, 16, 2, 64, dtype=torch.bfloat16) for _ in range(2)]
+    table = ops.LayerTable(caches)
+    slot = table.layout.slot_bytes
+    staging = torch.zeros(2 * slot, dtype=torch.uint8)
+    load = ops.PreparedFanout(table, [6, 1, 3, 6], [0, slot, 0, slot], staging)
+    assert (load.n_src, load.n_dst) == (2, 3)
+    with pytest.raises(IndexError):
+        ops.PreparedFanout(table, [6, 8], [0, slot], staging)

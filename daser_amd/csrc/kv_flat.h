@@ -52,7 +52,10 @@ constexpr int kPiece = kWave * 16;  // bytes of one wave instruction
 // are written at once. Against chunks of 32, 128 were 0-1% ahead at 4 and 32 KiB
 // pages and 1-3% at 64 and 96 KiB ones and at 80 layers of e4m3; of 16, 1-6%;
 // of 1,024 and 16,384, 0-2%.
-constexpr uint32_t kChunkLog2 = 7;
+constexpr uint32_t kChunk = 128;
+// Launches whose pages share records: each XCD takes one contiguous eighth of
+// the waves (copy_shape in kv_move.hip has the figures).
+constexpr uint32_t kEighths = ~0u;
 
 // The waves of one launch: wave w of it moves piece wave0 + w, counted from
 // the first piece of unit unit0.
@@ -60,7 +63,8 @@ struct FlatMap {
   FastDiv per_unit;  // pieces per unit
   FastDiv minor;     // page-major: layers; layer-major: pages
   uint32_t unit0, wave0, n_waves;
-  uint32_t chunked;  // workgroups dealt to the XCDs in chunks up to this one
+  FastDiv chunk;     // workgroups dealt to the XCDs in chunks of chunk.d
+  uint32_t chunked;  // up to this one
 };
 
 struct FlatPos {
@@ -76,7 +80,8 @@ __device__ __forceinline__ uint32_t flat_wave(const FlatMap& m) {
   uint32_t b = blockIdx.x;
   if (b < m.chunked) {
     const uint32_t x = b % kXcds, j = b / kXcds;
-    b = (((j >> kChunkLog2) * kXcds + x) << kChunkLog2) + (j & ((1u << kChunkLog2) - 1));
+    const uint32_t q = div_by(j, m.chunk);
+    b = (q * kXcds + x) * m.chunk.d + (j - q * m.chunk.d);
   }
   return b * (kThreads / kWave) +
          (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);

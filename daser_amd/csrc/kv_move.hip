@@ -134,23 +134,29 @@ int launch_page_ranges(const UnitArgs& a, int n_pages, F launch) {
 
 // Launches of a flat kernel over every piece of n_units units (one launch
 // unless the workgroups exceed max_wg_per_launch()), `minor` the inner extent
-// of the unit order: launch(map, grid).
+// of the unit order: launch(map, grid). `chunk`: consecutive workgroups that stay
+// on one XCD (0: dealt one by one; kEighths).
 template <class F>
-int launch_flat(int64_t n_units, int64_t pieces_per_unit, int64_t minor, bool chunked, F launch) {
+int launch_flat(int64_t n_units, int64_t pieces_per_unit, int64_t minor, uint32_t chunk, F launch) {
   constexpr int kWaves = kThreads / kWave;
   const int64_t total = n_units * pieces_per_unit;
   const int64_t per = max_wg_per_launch() * kWaves;
   for (int64_t g0 = 0; g0 < total; g0 += per) {
     const int64_t n = total - g0 < per ? total - g0 : per;
-    const unsigned grid = (unsigned)((n + kWaves - 1) / kWaves);
+    unsigned grid = (unsigned)((n + kWaves - 1) / kWaves);
     FlatMap m;
     m.per_unit = fast_div((uint32_t)pieces_per_unit);
     m.minor = fast_div((uint32_t)minor);
     m.unit0 = (uint32_t)(g0 / pieces_per_unit);
     m.wave0 = (uint32_t)(g0 % pieces_per_unit);
     m.n_waves = (uint32_t)n;
-    constexpr unsigned kRound = kXcds << kChunkLog2;
-    m.chunked = chunked ? grid / kRound * kRound : 0;
+    uint32_t c = chunk;
+    if (chunk == kEighths) {
+      grid = (grid + kXcds - 1) / kXcds * kXcds;  // the waves past the end leave at once
+      c = grid / kXcds;
+    }
+    m.chunk = fast_div(c ? c : 1);
+    m.chunked = c ? grid / (kXcds * c) * (kXcds * c) : 0;
     launch(m, grid);
     const int rc = (int)hipGetLastError();
     if (rc != 0) return rc;
@@ -199,7 +205,7 @@ size_t occupancy_lds(int wg_per_cu, int64_t static_lds) {
 //   of these, from 20 to 32 MiB, which is one workgroup per CU: each wave holds
 //     8 KiB of K and of V, so that no second generation of waves starts: 7.14 ->
 //     5.77 us at 29 MB (single pieces 6.53), a layer's save 7.24 -> 6.24 at 34;
-//   above: nt sc0 sc1 stores, in chunks of workgroups (kChunkLog2): 50.3 -> 42.1
+//   above: nt sc0 sc1 stores, in chunks of workgroups (kChunk): 50.3 -> 42.1
 //     us at 268 MB (nt 42.9), 185 -> 163 at 1.07 GB (nt 169), 738 -> 664 at 4.3
 //     GB (nt 681).
 // Where the same few buffers stay in the memory-side cache, sc0 sc1 stores are
@@ -208,15 +214,26 @@ size_t occupancy_lds(int wg_per_cu, int64_t static_lds) {
 // Four workgroups of single pieces per CU: 32 KiB of reads in flight there hide
 // the latency, and 6 or 8 per CU widen the written window (0-8% slower).
 constexpr int kCopyWgPerCu = 4;
+//
+// Several pages reading the same records (DSR_SHARED_RECORDS): kEighths at every
+// size, copies at 6 workgroups per CU. Without the flag -> with it, and the
+// per-page kernels of one workgroup per unit: Llama-3-70B, 32,768 pages of 2,048
+// records 50.9 -> 49.5 ms (50.2), its TP8 share 6.24 -> 6.14 (6.69); re-rotation
+// 50.1 -> 49.0 (50.4) and 6.24 -> 6.20 (6.66); TP8, 64 chunks of 16 pages out of 16:
+// 209 -> 176 us (181). Against it: 32 and 64 KiB pages of 10 GB and more in pools
+// without a power of two of blocks, copies 1-2% slower (8B, 4,096 pages of 1,024
+// records 2,544 -> 2,604 us; 2,862).
+constexpr int kSharedWgPerCu = 6;
 struct CopyShape {
-  bool nt;       // stores: nt, else nt sc0 sc1
-  bool whole;    // 8 pieces per wave
-  bool chunked;  // workgroups dealt in chunks
+  bool nt;         // stores: nt, else nt sc0 sc1
+  bool whole;      // 8 pieces per wave
+  uint32_t chunk;  // workgroups dealt in chunks
 };
-CopyShape copy_shape(const UnitArgs& a) {
+CopyShape copy_shape(const UnitArgs& a, bool shared) {
   const int64_t moved = 4 * a.page_bytes * a.n_units;
   const bool large = moved > (200 << 20);
-  CopyShape c{!large, moved > (20 << 20) && moved <= (32 << 20), large};
+  CopyShape c{!large, moved > (20 << 20) && moved <= (32 << 20),
+              shared ? kEighths : large ? kChunk : 0};
   if (const int64_t t = tune(DSR_TUNE_COPY_STORES)) c.nt = t == 1;
   if (const int64_t t = tune(DSR_TUNE_COPY_PIECES)) c.whole = t == 8;
   if (a.page_bytes % (8 * kPiece)) c.whole = false;
@@ -224,12 +241,12 @@ CopyShape copy_shape(const UnitArgs& a) {
 }
 
 template <bool kGather>
-int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s) {
-  const CopyShape c = copy_shape(a);
+int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s, bool shared = false) {
+  const CopyShape c = copy_shape(a, shared);
   const int64_t pieces = c.whole ? a.page_bytes / (8 * kPiece) : (a.page_bytes + kPiece - 1) / kPiece;
   const int64_t t = tune(DSR_TUNE_COPY_WG_PER_CU);
-  const size_t dyn = occupancy_lds(t ? (int)t : kCopyWgPerCu, 0);
-  return launch_flat(a.n_units, pieces, kGather ? a.n_layers : n_pages, c.chunked,
+  const size_t dyn = occupancy_lds(t ? (int)t : shared ? kSharedWgPerCu : kCopyWgPerCu, 0);
+  return launch_flat(a.n_units, pieces, kGather ? a.n_layers : n_pages, c.chunk,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_COPY(HND, POLICY, U) \
   kv_flat_copy_kernel<kGather, HND, POLICY, U><<<grid, kThreads, dyn, s>>>(a, m)
@@ -272,9 +289,9 @@ int launch_rerotate_pairs(const RotArgs& ra, int n_pages, int style, hipStream_t
 constexpr int kRotFlatWgPerCu = 6;
 
 template <int DT, int LAYOUT>
-int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_vecs,
+int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_vecs, bool shared,
                          hipStream_t s) {
-  const CopyShape c = copy_shape(ra.u);
+  const CopyShape c = copy_shape(ra.u, shared);
   const int64_t nvec = ra.u.page_bytes >> 4;
   const FastDiv row = fast_div((uint32_t)ra.row_vecs);
   int wg = kRotFlatWgPerCu;
@@ -283,7 +300,7 @@ int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_ve
   const size_t tabs = sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave);
   const size_t lds = occupancy_lds(wg, 0);
   const size_t dyn = lds > tabs ? lds : tabs;
-  return launch_flat(ra.u.n_units, (nvec + piece_vecs - 1) / piece_vecs, n_pages, c.chunked,
+  return launch_flat(ra.u.n_units, (nvec + piece_vecs - 1) / piece_vecs, n_pages, c.chunk,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_ROT(STYLE, POLICY)                                                          \
   kv_flat_rerotate_kernel<DT, STYLE, LAYOUT, POLICY><<<grid, kThreads, dyn, s>>>(ra, m, row, \
@@ -300,8 +317,8 @@ int launch_flat_rerotate(const RotArgs& ra, int n_pages, int style, int piece_ve
 }
 
 template <int DT>
-int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipStream_t s,
-                    int layout) {
+int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, bool shared,
+                    hipStream_t s, int layout) {
   const int h = ra.half_vecs;
   if (!vec_ok) {  // rotary width not in whole vectors: the LDS kernel
     return launch_page_ranges(ra.u, n_pages, [&](const UnitArgs& b, unsigned grid) {
@@ -316,8 +333,10 @@ int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipS
   }
   // split-x K: the caller checked the kx_phys conditions, which make every
   // neox partner lane ^ 32
-  if (layout == kRotKx) return launch_flat_rerotate<DT, kRotKx>(ra, n_pages, style, kWave, s);
-  if (layout == kRotHnd) return launch_flat_rerotate<DT, kRotHnd>(ra, n_pages, style, kWave, s);
+  if (layout == kRotKx)
+    return launch_flat_rerotate<DT, kRotKx>(ra, n_pages, style, kWave, shared, s);
+  if (layout == kRotHnd)
+    return launch_flat_rerotate<DT, kRotHnd>(ra, n_pages, style, kWave, shared, s);
   const bool contig = style == DSR_ROPE_GPTJ ||
                       (h > 0 && h <= 32 && (h & (h - 1)) == 0 && ra.row_vecs % (2 * h) == 0);
   // other neox rows of <= 64 vectors: pieces of whole rows (the
@@ -326,7 +345,7 @@ int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, hipS
                     tune(DSR_TUNE_ROT_KERNEL) != kRotPairs;
   if (contig || rows)
     return launch_flat_rerotate<DT, kRotNhd>(
-        ra, n_pages, style, contig ? kWave : kWave / ra.row_vecs * ra.row_vecs, s);
+        ra, n_pages, style, contig ? kWave : kWave / ra.row_vecs * ra.row_vecs, shared, s);
   return launch_rerotate_pairs<DT>(ra, n_pages, style, s);
 }
 
@@ -406,8 +425,7 @@ int dsr_scatter_ex(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
   UnitArgs a = make_unit(layer_base, n_layers, kv_stride, page_stride, page_bytes,
                          num_blocks, page_ids, slot_offsets, n_pages, staging,
                          staging_bytes, layer_bytes, layer0);
-  (void)flags;  // the flat copy is the choice for shared records too
-  return launch_copy<false>(a, n_pages, (hipStream_t)stream);
+  return launch_copy<false>(a, n_pages, (hipStream_t)stream, flags & DSR_SHARED_RECORDS);
 }
 
 int dsr_scatter(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
@@ -500,6 +518,7 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
   ra.rot_vecs = rot_dim * esize / 16;
   ra.half_vecs = rope_style == DSR_ROPE_NEOX && vec_ok ? rot_dim / 2 * esize / 16 : 0;
   ra.k_scale = k_scale;
+  const bool shared = flags & DSR_REROTATE_SHARED_RECORDS;
   hipStream_t s = (hipStream_t)stream;
   if (hnd_block > 0) {
     // head-major pages: rows and partners stay whole in record order, the cache
@@ -515,13 +534,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
     ra.u.hnd_row_vecs = ra.row_vecs;
     switch (dtype) {
       case DSR_DTYPE_BF16:
-        return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, kRotHnd);
+        return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, shared, s, kRotHnd);
       case DSR_DTYPE_FP16:
-        return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, kRotHnd);
+        return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, shared, s, kRotHnd);
       case DSR_DTYPE_FP8_E4M3:
-        return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, kRotHnd);
+        return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, shared, s, kRotHnd);
       default:
-        return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, kRotHnd);
+        return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, shared, s, kRotHnd);
     }
   }
   if (kx_block > 0) {
@@ -539,13 +558,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
       ra.row_vecs = (int)hv;
       switch (dtype) {
         case DSR_DTYPE_BF16:
-          return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, s, kRotKx);
+          return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, true, shared, s, kRotKx);
         case DSR_DTYPE_FP16:
-          return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, s, kRotKx);
+          return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, true, shared, s, kRotKx);
         case DSR_DTYPE_FP8_E4M3:
-          return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, s, kRotKx);
+          return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, true, shared, s, kRotKx);
         default:
-          return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, s, kRotKx);
+          return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, true, shared, s, kRotKx);
       }
     }
     switch (dtype) {
@@ -561,13 +580,13 @@ int scatter_rerotate_any(const uint64_t* layer_base, int n_layers,
   }
   switch (dtype) {
     case DSR_DTYPE_BF16:
-      return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
+      return launch_rerotate<DSR_DTYPE_BF16>(ra, n_pages, rope_style, vec_ok, shared, s, kRotNhd);
     case DSR_DTYPE_FP16:
-      return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
+      return launch_rerotate<DSR_DTYPE_FP16>(ra, n_pages, rope_style, vec_ok, shared, s, kRotNhd);
     case DSR_DTYPE_FP8_E4M3:
-      return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
+      return launch_rerotate<DSR_DTYPE_FP8_E4M3>(ra, n_pages, rope_style, vec_ok, shared, s, kRotNhd);
     default:
-      return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, vec_ok, s, kRotNhd);
+      return launch_rerotate<DSR_DTYPE_FP8_E5M2>(ra, n_pages, rope_style, vec_ok, shared, s, kRotNhd);
   }
 }
 
@@ -761,7 +780,7 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   const bool large = slots_large(a);
   const hipStream_t s = (hipStream_t)stream;
   const size_t dyn = occupancy_lds(slots_wg_per_cu(gather, h.wide), 0);
-  return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units, large,
+  return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units, large ? kChunk : 0,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_SLOTS(WIDE, POLICY)                                                              \
   (gather ? kv_slots_flat_kernel<true, WIDE, POLICY><<<grid, kThreads, dyn, s>>>(a, m)       \
@@ -849,7 +868,7 @@ int slots_rerotate_launch(const uint64_t* layer_base, int n_layers, int64_t kv_s
   const size_t tabs = sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave);
   const size_t lds = occupancy_lds(t ? (int)t : kRotFlatWgPerCu, 0);
   const size_t dyn = lds > tabs ? lds : tabs;
-  return launch_flat(h.units * n_layers, h.pieces, h.units, large,
+  return launch_flat(h.units * n_layers, h.pieces, h.units, large ? kChunk : 0,
                      [&](const FlatMap& m, unsigned grid) {
     const bool neox = rope_style == DSR_ROPE_NEOX;
 #define DSR_SLOT_ROT_P(DT, WIDE, POLICY)                                                     \
@@ -1065,7 +1084,8 @@ int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
   const size_t dyn = lds > tabs ? lds : tabs;
   const FastDiv row = fast_div((uint32_t)(ROT ? ra.row_vecs : 1));
   return launch_flat((int64_t)fa.n_src * ra.u.n_layers, (ra.u.page_bytes + kPiece - 1) / kPiece,
-                     many ? ra.u.n_layers : fa.n_src, many, [&](const FlatMap& m, unsigned grid) {
+                     many ? ra.u.n_layers : fa.n_src, many ? kChunk : 0,
+                     [&](const FlatMap& m, unsigned grid) {
     kv_fanout_kernel<DT, STYLE, LAYOUT, ROT><<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
   });
 }

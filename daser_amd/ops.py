@@ -560,13 +560,17 @@ def scatter(
     page_ids, slot_offsets, _ = dest_order(page_ids, slot_offsets)
     args, _tables = _copy_args(table, page_ids, slot_offsets, staging, layer0, layers)
     stream = _stream_handle(table.layout.device)
-    if shared_records and table.layout.k_layout != "hnd":
-        rc = _lib.lib().dsr_scatter_ex(*args, _lib.DSR_SHARED_RECORDS, stream)
-        _lib.check("dsr_scatter_ex", rc)
+    _scatter(table.layout, args, shared_records, stream)
+
+
+def _scatter(lay: PagedKVLayout, args, shared: bool, stream: int) -> None:
+    """The layout's copy entry point on device tables."""
+    if shared and lay.k_layout != "hnd":
+        _lib.check("dsr_scatter_ex",
+                   _lib.lib().dsr_scatter_ex(*args, _lib.DSR_SHARED_RECORDS, stream))
         return
-    fn, name, extra = _copy_entry(table.layout, "dsr_scatter")
-    rc = fn(*args, *extra, stream)
-    _lib.check(name, rc)
+    fn, name, extra = _copy_entry(lay, "dsr_scatter")
+    _lib.check(name, fn(*args, *extra, stream))
 
 
 def _host_tables(table: LayerTable, page_ids, slot_offsets):
@@ -608,8 +612,7 @@ def _load_host(table: LayerTable, ids: np.ndarray, offs: np.ndarray, staging: to
             lay.num_blocks, p.ids, p.offsets, plan.n_pages, staging.data_ptr(), nbytes,
             lay.layer_bytes, layer0 + first)
     if rope is None:
-        fn, name, extra = _copy_entry(lay, "dsr_scatter")
-        _lib.check(name, fn(*args, *extra, p.stream))
+        _scatter(lay, args, shared, p.stream)
         return
     _, cos_sin, rot_dim, style, n_tables, n_groups, lg_d, ks_ptr = rope
     _rerotate(lay, args, cos_sin.data_ptr(), p.rope, n_tables, n_groups, lg_d, rot_dim, style,

@@ -232,9 +232,8 @@ int dsr_scatter_ex(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
  *             V is copied as raw bytes, never decoded.
  *   flags     0, or DSR_REROTATE_SHARED_RECORDS when several pages of the
  *             call read the same records (one cached chunk placed in several
- *             requests): their repeated reads are served by the caches, and
- *             the launch is shaped for that (more workgroups per CU). A
- *             performance hint only: results are identical either way.
+ *             requests): each XCD then takes one contiguous eighth of the
+ *             pages. A performance hint only: results are identical either way.
  */
 int dsr_scatter_rerotate(const uint64_t* layer_base, int n_layers,
                          int64_t kv_stride, int64_t page_stride,

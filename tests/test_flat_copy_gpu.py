@@ -379,3 +379,42 @@ def test_negative_row_offsets(gpu, heads, dim, skipped, load):
     torch.cuda.synchronize()
     assert torch.equal(staging, want_s)
     assert torch.equal(whole.view(torch.uint8).view(layers, 2, -1, row), want_c)
+
+
+@pytest.mark.parametrize("block,heads,dim,layout", [
+    (1, 1, 8, "nhd"), (16, 1, 64, "nhd"), (16, 5, 128, "nhd"), (16, 8, 64, "kx"),
+    (16, 4, 128, "hnd")])
+@pytest.mark.parametrize("n,max_wg", [(1, 0), (7, 0), (40, 0), (40, 24), (333, 0)])
+def test_shared_records_order(gpu, tuning, block, heads, dim, layout, n, max_wg):
+    """The launch for shared records (each XCD one eighth: grids of fewer than 8
+    workgroups, of no multiple of 8, cut launches) writes what the plain one does."""
+    print(f"case: shared order bs{block} H{heads} D{dim} {layout} {n} {max_wg}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    layers = 3
+    g = torch.Generator(device=gpu).manual_seed(n)
+    inner = {"nhd": (block, heads, dim), "hnd": (heads, block, dim),
+             "kx": (block * heads * dim,)}[layout]
+    geo = dict(block_size=block, head_dim=dim) if layout == "kx" else {}
+    outs = [torch.zeros((layers, 2, n + 2, *inner), dtype=torch.bfloat16, device=gpu)
+            for _ in range(2)]
+    views = [[w.transpose(2, 3) if layout == "hnd" else w for w in o.unbind(0)] for o in outs]
+    tables = [ops.LayerTable(v, **geo) for v in views]
+    slot = tables[0].layout.slot_bytes
+    n_rec = max(1, n // 3)
+    staging = torch.randn(n_rec * slot // 2, generator=g, device=gpu).to(torch.bfloat16) \
+        .view(torch.uint8)
+    rng = np.random.default_rng(n)
+    ids = torch.from_numpy(np.sort(rng.permutation(n + 2)[:n]).astype(np.int32)).to(gpu)
+    offs = torch.from_numpy(rng.integers(0, n_rec, n) * slot).to(gpu)
+    ridx = torch.from_numpy((np.arange(n) % 3 - 1).astype(np.int32)).to(gpu)
+    ang = torch.rand((2, dim // 2), generator=g, device=gpu) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1)
+    for rotate in (False, True):
+        for table, shared in zip(tables, (False, True)):
+            if rotate and dim >= 16:
+                ops.scatter_rerotate(table, ids, offs, staging, tabs, ridx, shared_records=shared)
+            else:
+                ops.scatter(table, ids, offs, staging, shared_records=shared)
+        torch.cuda.synchronize()
+        assert torch.equal(*(o.view(torch.int16) for o in outs))
+        assert outs[0].view(torch.int16).any()

@@ -23,12 +23,14 @@ struct FanArgs {
   const int32_t* dst_pages;    // block id of each destination
   const int32_t* dst_rope;     // table index of each destination (-1: K copied); null: no rotation
   int32_t n_src;
+  int32_t n_dst;               // for the launch's shape
 };
 
 // A destination's table is fetched while the one before is being written (the
 // first 128 pairs; wider tables read the rest when they are needed). ROT false:
-// a plain copy. Cache layouts (LAYOUT) as in kv_flat_rerotate_kernel.
-template <int DT, int STYLE, int LAYOUT, bool ROT>
+// a plain copy. Cache layouts (LAYOUT) as in kv_flat_rerotate_kernel; POLICY: the
+// stores' cache policy.
+template <int DT, int STYLE, int LAYOUT, bool ROT, int POLICY>
 __global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa, FlatMap m, FastDiv row,
                                                              bool layer_major) {
   extern __shared__ float2 lds_tab[];
@@ -135,8 +137,8 @@ __global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa, FlatMap
       }
       if (blk < 0 || blk >= a.num_blocks) continue;  // skipped, as by the page scatter
       uint8_t* const cache = lbase + blk * a.page_stride;
-      bstore_as<kStoreNtSc>(make_rsrc(cache + a.kv_stride, n), vc, v);
-      bstore_as<kStoreNtSc>(make_rsrc(cache, n), kc, kk);
+      bstore_as<POLICY>(make_rsrc(cache + a.kv_stride, n), vc, v);
+      bstore_as<POLICY>(make_rsrc(cache, n), kc, kk);
     }
   }
 }

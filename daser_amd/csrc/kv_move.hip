@@ -1060,17 +1060,29 @@ int dsr_scatter_rerotate_static(const uint64_t* layer_base, int n_layers,
 
 namespace {
 
-// Unit order and workgroups per CU of the fan-out, whose destinations lie
-// anywhere: that bounds it (5.0-5.3 TB/s where ordered pages take 6.4 or more).
-// Few sources: layer-major in dispatch order, 6 per CU; the chip then writes one
-// layer's pages, and every wave its source's in block order. From 512 sources
-// up that span (all of a layer's pages) is too wide, and source-major, 4 per CU,
-// in chunks of workgroups is ahead. Measured, per-unit workgroups -> layer-major
-// / source-major: 8B bf16, 256 sources 657 -> 585 / 609 us, 640 sources 2,420 ->
-// 2,320 / 2,327; 7B bf16, 640 sources 1,054 -> 1,083 / 1,033; 8B e4m3, 256 sources
-// 388 -> 288 / 308, 640 sources 1,421 -> 1,176 / 1,153; 70B bf16, 512 sources 4,806 ->
-// 4,703 / 4,657. DSR_TUNE_FANOUT_WG_PER_CU overrides the workgroups.
+// Unit order, stores and workgroups per CU of the fan-out, whose destinations lie
+// anywhere. All figures in us, in one process in turn: the kernel of one workgroup
+// per unit that this one replaced / this choice / the other one.
+//   From kFanManySources records up source-major (a record's layers follow each
+//   other), else layer-major, workgroups dealt one by one. Layer-major writes one
+//   layer's pages at a time, which is ahead by 1-6% while they are few (8B bf16, 1,024
+//   pages of 128 records 484 / 446 / 474; 0.5B, 4,096 of 256 165 / 165 / 169) and behind
+//   where they are many (8B, 5,120 of 640 2,005 / 1,915 / 2,185; 70B, 32,768 of 2,048
+//   27,968 / 28,041 / 32,728; its TP8 share 3,955 / 3,926 / 4,258); from 384 to 2,048
+//   records of 8B and TP8 in pools without a power of two of blocks the two are within
+//   3%, either way. Chunks of 128 workgroups (the page copies') cost source-major plain
+//   loads 1-3%: 70B 28,041 -> 28,805.
+//   Stores sc0 sc1 from 1 GiB read and written up: 1-5% ahead of nt sc0 sc1 (8B, 4,096 of
+//   256 1,655 against 1,697; 70B TP8 rotated 3,489 against 3,633), which a smaller load
+//   takes (1,024 TP8 pages of 256 165 against 169; on buffers in turn that the
+//   memory-side cache does not hold, up to 10% ahead at 128 pages).
+//   4 workgroups per CU, for few destinations 6, on such buffers: 0.5B rotated, 512 of
+//   64 1.01 times the old kernel's rate at 4, 0.94 at 6; 8B rotated, 128 of 64 1.33 and
+//   1.38, TP8 plain, 64 of 32 1.10 and 1.16.
+// DSR_TUNE_FANOUT_WG_PER_CU overrides the workgroups.
 constexpr int64_t kFanManySources = 512;
+constexpr int64_t kFanLargeBytes = 1 << 30;
+constexpr int kFanFewPages = 256;
 
 template <int DT, int STYLE, int LAYOUT, bool ROT>
 int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
@@ -1079,14 +1091,21 @@ int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
   const size_t tabs =
       ROT ? sizeof(float2) * (ra.rot_half + ra.rot_half / col * 2) * (kThreads / kWave) : 0;
   const bool many = fa.n_src >= kFanManySources;
+  const bool large =
+      2 * ra.u.page_bytes * ra.u.n_layers * ((int64_t)fa.n_src + fa.n_dst) > kFanLargeBytes;
   const int64_t t = tune(DSR_TUNE_FANOUT_WG_PER_CU);
-  const size_t lds = occupancy_lds(t ? (int)t : many ? 4 : 6, 0);
+  const size_t lds = occupancy_lds(t ? (int)t : fa.n_dst > kFanFewPages ? 4 : 6, 0);
   const size_t dyn = lds > tabs ? lds : tabs;
   const FastDiv row = fast_div((uint32_t)(ROT ? ra.row_vecs : 1));
   return launch_flat((int64_t)fa.n_src * ra.u.n_layers, (ra.u.page_bytes + kPiece - 1) / kPiece,
-                     many ? ra.u.n_layers : fa.n_src, many ? kChunk : 0,
+                     many ? ra.u.n_layers : fa.n_src, 0,
                      [&](const FlatMap& m, unsigned grid) {
-    kv_fanout_kernel<DT, STYLE, LAYOUT, ROT><<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
+    if (large)
+      kv_fanout_kernel<DT, STYLE, LAYOUT, ROT, kStorePolicy>
+          <<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
+    else
+      kv_fanout_kernel<DT, STYLE, LAYOUT, ROT, kStoreNtSc>
+          <<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
   });
 }
 
@@ -1225,6 +1244,7 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
   fa.dst_pages = dst_page_ids;
   fa.dst_rope = dst_rope_idx;
   fa.n_src = n_src;
+  fa.n_dst = n_dst;
   hipStream_t s = (hipStream_t)stream;
   switch (dt) {
     case DSR_DTYPE_BF16: return launch_fanout<DSR_DTYPE_BF16>(fa, style, layout, s);

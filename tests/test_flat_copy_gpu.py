@@ -296,6 +296,38 @@ def test_flat_fanout(gpu, n_src, n_dst, heads, dim, dt, layout, rot):
     assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
 
 
+@pytest.mark.parametrize("n_src,n_dst", [(300, 3800), (1000, 3100)])
+def test_large_fanout(gpu, n_src, n_dst):
+    """The fan-out's launch above 1 GiB, both unit orders: what the per-page load
+    writes, K rotated or not."""
+    print(f"case: large fanout {n_src}->{n_dst}", flush=True)
+    layers, nb = 4, n_dst + 9
+    g = torch.Generator(device=gpu).manual_seed(n_src)
+    rng = np.random.default_rng(n_src)
+    staging = torch.randn((n_src, layers, 2, 16, 8, 128), generator=g, device=gpu) \
+        .to(torch.bfloat16).view(-1).view(torch.uint8)
+    caches = [torch.zeros((layers, 2, nb, 16, 8, 128), dtype=torch.bfloat16, device=gpu)
+              for _ in range(2)]
+    tables = [ops.LayerTable(list(c.unbind(0))) for c in caches]
+    slot = tables[0].layout.slot_bytes
+    assert (n_src + n_dst) * slot > 1 << 30
+    ids = rng.permutation(nb)[:n_dst].astype(np.int64)
+    src = np.concatenate([np.arange(n_src), rng.integers(0, n_src, n_dst - n_src)])
+    offs = rng.permutation(src).astype(np.int64) * slot
+    ang = torch.rand((5, 64), generator=g, device=gpu, dtype=torch.float64) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    ridx = rng.integers(-1, 5, n_dst)
+    ops.PreparedFanout(tables[0], ids, offs, staging, rope=(ridx, tabs, 128, "neox", None, None))()
+    ops.scatter_rerotate(tables[1], ids, offs, staging, tabs, ridx, shared_records=False)
+    torch.cuda.synchronize()
+    assert torch.equal(*(c.view(torch.int16) for c in caches))
+    assert caches[0].view(torch.int16).any()
+    ops.PreparedFanout(tables[0], ids, offs, staging)()
+    ops.scatter(tables[1], ids, offs, staging, shared_records=False)
+    torch.cuda.synchronize()
+    assert torch.equal(*(c.view(torch.int16) for c in caches))
+
+
 @pytest.mark.parametrize("n,rot", [(1, 128), (7, 128), (8, 128), (60, 20), (1024, 128)])
 def test_delta_tables_on_the_device(gpu, n, rot):
     """The device's float64 tables (more than a kernel's arguments hold) are the

@@ -729,9 +729,8 @@ SlotShape slot_shape(SlotArgs* a) {
 
 // Stores and order of a token-form launch, by the bytes it moves, as for the
 // page copies (copy_shape).
-bool slots_large(const SlotArgs& a) {
-  return 4 * a.row_bytes * a.n_tokens * a.n_layers > (200 << 20);
-}
+int64_t slots_moved(const SlotArgs& a) { return 4 * a.row_bytes * a.n_tokens * a.n_layers; }
+bool slots_large(const SlotArgs& a) { return slots_moved(a) > (200 << 20); }
 
 // Workgroups per CU: 6, wide rows' scatters 4 (8B bf16 rows 5.92 TB/s at 4, 5.78 at
 // 6; one-head e4m3 rows 5.78 at 4, 5.88 at 6, gathers 5.75 and 5.89).
@@ -739,6 +738,17 @@ int slots_wg_per_cu(bool gather, bool wide) {
   const int64_t t = tune(DSR_TUNE_SLOTS_WG_PER_CU);
   return t ? (int)t : wide && !gather ? 4 : 6;
 }
+
+// Gathers of rows up to 4 KiB that move more than 16 GiB: sc0 sc1 stores, workgroups
+// dealt one by one. The kernel of 16 tokens per workgroup that this one replaced /
+// chunks and nt sc0 sc1 stores / this: 2 KiB rows of 32 layers 70,000 tokens 2,863 / 2,913 /
+// 2,893 us, 283,000 11,533 / 11,682 / 11,588, of 80 layers 70,000 7,481 / 7,433 / 7,218; 4 KiB
+// rows of 42 layers 108,000 12,557 / 12,309 / 12,065; 1 KiB rows of 32 layers 283,000 7,046 /
+// 6,327 / 5,976. Smaller gathers: within 1% either way, 1 KiB rows of 11,000 tokens 294 / 236 /
+// 241; rows of 6 KiB 13,387 / 11,694 / 12,568. (One piece per wave throughout: 2, 4 and 8 were
+// 1-10% behind.)
+constexpr int64_t kSlotsHugeBytes = 16ll << 30;
+constexpr int64_t kSlotsHugeRow = 4 << 10;
 
 int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t kv_stride,
                  int64_t page_stride, int64_t page_bytes, int64_t num_blocks, int block_size,
@@ -778,14 +788,18 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   const SlotShape h = slot_shape(&a);
   if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   const bool large = slots_large(a);
+  const bool huge = gather && h.wide && row_bytes <= kSlotsHugeRow &&
+                    slots_moved(a) > kSlotsHugeBytes;
   const hipStream_t s = (hipStream_t)stream;
   const size_t dyn = occupancy_lds(slots_wg_per_cu(gather, h.wide), 0);
-  return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units, large ? kChunk : 0,
+  return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units,
+                     large && !huge ? kChunk : 0,
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_SLOTS(WIDE, POLICY)                                                              \
   (gather ? kv_slots_flat_kernel<true, WIDE, POLICY><<<grid, kThreads, dyn, s>>>(a, m)       \
           : kv_slots_flat_kernel<false, WIDE, POLICY><<<grid, kThreads, dyn, s>>>(a, m))
     if (!h.wide) DSR_SLOTS(false, kStoreNt);
+    else if (huge) kv_slots_flat_kernel<true, true, kStorePolicy><<<grid, kThreads, dyn, s>>>(a, m);
     else if (large) DSR_SLOTS(true, kStoreNtSc);
     else DSR_SLOTS(true, kStoreNt);
 #undef DSR_SLOTS

@@ -252,6 +252,33 @@ def test_flat_slots(gpu, tuning, heads, dim, dt, block, max_wg):
     assert torch.equal(rot.view(torch.uint8), exp.view(torch.uint8))
 
 
+@pytest.mark.parametrize("heads,dim", [(5, 104), (16, 128)])
+def test_huge_slot_gather(gpu, heads, dim):
+    """The token gather's launch above 16 GiB moved, rows of 65 vectors and of the
+    largest length it takes: the records of the page form, tokens that are left
+    out untouched."""
+    print(f"case: huge slot gather H{heads} D{dim}", flush=True)
+    layers, block, row = 64, 16, heads * dim * 2
+    n = (16 << 30) // (4 * layers * block * row) + 2
+    g = torch.Generator(device=gpu).manual_seed(dim)
+    rng = np.random.default_rng(dim)
+    whole = torch.empty((layers, 2, n, block, heads, dim), dtype=torch.bfloat16, device=gpu)
+    whole.view(-1).view(torch.int64).random_(generator=g)
+    table = ops.LayerTable(list(whole.unbind(0)))
+    lay = table.layout
+    ids = rng.permutation(n)
+    tokens = n * block - 1  # short of the last page by a token
+    slots = ops.slot_mapping_for([ids], [tokens], block)
+    rows = ops.token_row_offsets([tokens], lay.slot_bytes, block, row)
+    assert 4 * tokens * row * layers > 16 << 30
+    want, got = (torch.zeros(n * lay.slot_bytes, dtype=torch.uint8, device=gpu) for _ in range(2))
+    ops.gather(table, ids, np.arange(n, dtype=np.int64) * lay.slot_bytes, want)
+    want.view(n, layers, 2, block, row)[-1, :, :, -1] = 0
+    ops.gather_slots(table, torch.from_numpy(slots).to(gpu), torch.from_numpy(rows).to(gpu), got)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and got.any()
+
+
 @pytest.mark.parametrize("n_src,n_dst,heads,dim,dt,layout,rot", [
     (3, 300, 1, 64, "bf16", "nhd", 64), (511, 1100, 1, 128, "e4m3", "nhd", 128),
     (512, 1100, 1, 128, "bf16", "nhd", 64), (600, 1300, 2, 64, "e5m2", "hnd", 64),

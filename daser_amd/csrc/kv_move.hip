@@ -250,15 +250,14 @@ int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s, bool shared = fal
                      [&](const FlatMap& m, unsigned grid) {
 #define DSR_COPY(HND, POLICY, U) \
   kv_flat_copy_kernel<kGather, HND, POLICY, U><<<grid, kThreads, dyn, s>>>(a, m)
-    if (a.hnd_heads) {
-      if (c.whole) DSR_COPY(true, kStoreNt, 8);
-      else if (c.nt) DSR_COPY(true, kStoreNt, 1);
-      else DSR_COPY(true, kStoreNtSc, 1);
-    } else {
-      if (c.whole) DSR_COPY(false, kStoreNt, 8);
-      else if (c.nt) DSR_COPY(false, kStoreNt, 1);
-      else DSR_COPY(false, kStoreNtSc, 1);
-    }
+#define DSR_COPY_U(HND, U)                     \
+  if (c.nt) DSR_COPY(HND, kStoreNt, U);        \
+  else DSR_COPY(HND, kStoreNtSc, U)
+    if (a.hnd_heads && c.whole) DSR_COPY_U(true, 8);
+    else if (a.hnd_heads) DSR_COPY_U(true, 1);
+    else if (c.whole) DSR_COPY_U(false, 8);
+    else DSR_COPY_U(false, 1);
+#undef DSR_COPY_U
 #undef DSR_COPY
   });
 }

@@ -35,7 +35,7 @@ def _records(views, ids):
     (16, 2, 128, "nhd"), (16, 5, 96, "nhd"), (16, 16, 128, "nhd"),
     (1, 1, 8, "hnd"), (5, 3, 24, "hnd"), (16, 4, 128, "hnd")])
 @pytest.mark.parametrize("policy,pieces,max_wg", [(0, 0, 0), (1, 8, 0), (1, 1, 16), (3, 0, 16),
-                                                  (0, 8, 24)])
+                                                  (0, 8, 24), (3, 8, 0)])
 def test_flat_copies(gpu, tuning, block, heads, dim, layout, policy, pieces, max_wg):
     print(f"case: flat bs{block} H{heads} D{dim} {layout} {policy} {pieces} {max_wg}", flush=True)
     tuning("scatter_kernel", policy)

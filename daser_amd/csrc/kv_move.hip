@@ -263,8 +263,8 @@ int launch_copy(const UnitArgs& a, int n_pages, hipStream_t s, bool shared = fal
 }
 
 
-// The pair-task kernel alone: the split-x K layout, whose rotation partners
-// are a whole block of vectors apart.
+// The pair-task kernel: neox rows of more than 64 vectors whose partner distance
+// is no power of two, and split-x K pages whose head blocks are none.
 template <int DT>
 int launch_rerotate_pairs(const RotArgs& ra, int n_pages, int style, hipStream_t s) {
   const size_t dyn =
@@ -338,11 +338,9 @@ int launch_rerotate(const RotArgs& ra, int n_pages, int style, bool vec_ok, bool
     return launch_flat_rerotate<DT, kRotHnd>(ra, n_pages, style, kWave, shared, s);
   const bool contig = style == DSR_ROPE_GPTJ ||
                       (h > 0 && h <= 32 && (h & (h - 1)) == 0 && ra.row_vecs % (2 * h) == 0);
-  // other neox rows of <= 64 vectors: pieces of whole rows (the
-  // DSR_TUNE_ROT_KERNEL override "pairs" takes the pair-task kernel)
-  const bool rows = !contig && ra.row_vecs <= kWave && h > 0 && 2 * h <= ra.row_vecs &&
-                    tune(DSR_TUNE_ROT_KERNEL) != kRotPairs;
-  if (contig || rows)
+  // other neox rows of <= 64 vectors: pieces of whole rows
+  const bool rows = !contig && ra.row_vecs <= kWave && h > 0 && 2 * h <= ra.row_vecs;
+  if ((contig || rows) && tune(DSR_TUNE_ROT_KERNEL) != kRotPairs)
     return launch_flat_rerotate<DT, kRotNhd>(
         ra, n_pages, style, contig ? kWave : kWave / ra.row_vecs * ra.row_vecs, shared, s);
   return launch_rerotate_pairs<DT>(ra, n_pages, style, s);

@@ -67,7 +67,7 @@ def _geometry(shape, cache):
 
 
 @pytest.mark.parametrize("heads,head_dim,dt,style,rot_dim,groups", [
-    (8, 128, "bf16", 0, 128, False),   # 32 KiB pages, U = 8
+    (8, 128, "bf16", 0, 128, False),   # 32 KiB pages
     (4, 128, "bf16", 0, 128, True),    # 16 KiB, layer groups
     (2, 128, "fp16", 1, 128, False),   # 8 KiB, gptj
     (1, 128, "bf16", 0, 64, False),    # 4 KiB, partial rotary
@@ -76,12 +76,12 @@ def _geometry(shape, cache):
     (2, 64, "bf16", 0, 64, False),     # 4 KiB, partner 4 vectors away
     (16, 128, "e4m3", 1, 96, False),   # 32 KiB e4m3, gptj, partial rotary
 ])
-@pytest.mark.parametrize("parts", [1, 2])
-def test_fanout_matches_per_page_rerotate(tuning, parts, heads, head_dim, dt, style, rot_dim,
+@pytest.mark.parametrize("wg_per_cu", [0, 2])
+def test_fanout_matches_per_page_rerotate(tuning, wg_per_cu, heads, head_dim, dt, style, rot_dim,
                                           groups):
     print(f"case: fanout H{heads} D{head_dim} {dt} style{style} rot{rot_dim} groups{groups} "
-          f"parts{parts}", flush=True)
-    tuning("fanout_parts", parts)
+          f"{wg_per_cu}", flush=True)
+    tuning("fanout_wg_per_cu", wg_per_cu)
     shape, nb, recs, a, b, page_ids, offs, ridx, tabs, lg, ks, n_tables = _case(
         heads, head_dim, dt, style, rot_dim, groups, n_src=7, n=60, seed=heads * 7 + head_dim)
     kv_stride, page_stride = _geometry(shape, a[0])
@@ -122,15 +122,13 @@ def test_fanout_matches_per_page_rerotate(tuning, parts, heads, head_dim, dt, st
     assert torch.equal(got, rec[int(offs[p] // shape.slot_bytes), 1, 1])
 
 
-@pytest.mark.parametrize("max_wg,parts", [(0, 1), (16, 1), (0, 2), (16, 4)])
-def test_fanout_plain_copy_matches_scatter(tuning, max_wg, parts):
+@pytest.mark.parametrize("max_wg,wg_per_cu", [(0, 0), (16, 0), (0, 2), (24, 4)])
+def test_fanout_plain_copy_matches_scatter(tuning, max_wg, wg_per_cu):
     """dst_rope_idx null: the plain load, bit-exact to dsr_scatter, also when
-    the sources are split over several launches and units over several
-    workgroups."""
-    print(f"case: fanout copy max_wg={max_wg} parts={parts}", flush=True)
-    if max_wg:
-        tuning("max_wg_per_launch", max_wg)
-    tuning("fanout_parts", parts)
+    the sources are split over several launches, inside a unit too."""
+    print(f"case: fanout copy max_wg={max_wg} {wg_per_cu}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    tuning("fanout_wg_per_cu", wg_per_cu)
     shape, nb, recs, a, b, page_ids, offs, *_ = _case(8, 128, "bf16", 0, 128, False,
                                                       n_src=9, n=70, seed=5)
     kv_stride, page_stride = _geometry(shape, a[0])

@@ -275,7 +275,7 @@ def test_fp8_rerotate_full_size_oracle_sample(gpu):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("cfg", [3, 6])  # 6: one KV head, 4 KiB pages (grouped kernels)
+@pytest.mark.parametrize("cfg", [3, 6])  # 6: one KV head, 4 KiB pages
 def test_rerotate_full_size_properties(gpu, cfg):
     print(f"case: full-size rerotate cfg{cfg}", flush=True)
     wl = workloads.config(cfg)

@@ -63,17 +63,17 @@ def test_scatter_cfg1_bit_exact_and_round_trip(gpu):
 
 @pytest.mark.parametrize("heads,head_dim,dt", [(8, 128, "bf16"), (16, 128, "bf16"),
                                                 (8, 128, "e4m3"), (4, 96, "bf16")])
-@pytest.mark.parametrize("kernel,wg_per_cu", [(0, 0), (1, 0), (2, 0), (1, 1), (2, 1), (2, 2),
-                                              (3, 1), (3, 2), (1, 3)])
-def test_page_copy_kernels_and_occupancy_match_oracle(gpu, tuning, heads, head_dim, dt,
-                                                      kernel, wg_per_cu):
-    """Both one-unit scatter kernels (load-all-then-store, streaming in
-    either unit order) at every occupancy the launch policy or an override may pick, and the
-    gather at the same occupancies: the oracle's bytes, with ragged requests
-    and partial last pages (pages of 32, 64, 16 and 12 KiB)."""
-    print(f"case: page copy H{heads} D{head_dim} {dt} kernel={kernel} wpc={wg_per_cu}",
+@pytest.mark.parametrize("stores,wg_per_cu", [(0, 0), (1, 0), (3, 0), (1, 1), (3, 1), (1, 2),
+                                              (3, 2), (0, 6), (1, 3)])
+def test_page_copy_stores_and_occupancy_match_oracle(gpu, tuning, heads, head_dim, dt,
+                                                     stores, wg_per_cu):
+    """The page copies with either store policy (1: nt, 3: nt sc0 sc1, 0: the
+    launch's own) at the occupancies that the launch or an override may pick:
+    the oracle's bytes, with ragged requests and partial last pages (pages of 32,
+    64, 16 and 12 KiB)."""
+    print(f"case: page copy H{heads} D{head_dim} {dt} stores={stores} wpc={wg_per_cu}",
           flush=True)
-    tuning("scatter_kernel", kernel)
+    tuning("scatter_kernel", stores)
     tuning("copy_wg_per_cu", wg_per_cu)
     shape = KVShape(3, heads, head_dim, 16, 1 if dt in FP8 else 2)
     wl = workloads.ragged(shape, 6, 1, 400, seed=heads + head_dim, pool_slack=1.3)
@@ -91,15 +91,15 @@ def test_page_copy_kernels_and_occupancy_match_oracle(gpu, tuning, heads, head_d
 
 
 @pytest.mark.parametrize("heads,dt", [(8, "bf16"), (16, "bf16"), (8, "e4m3"), (1, "bf16")])
-@pytest.mark.parametrize("split", [0, 1, 2, 4, 8])
+@pytest.mark.parametrize("pieces,stores", [(0, 0), (1, 1), (1, 3), (8, 1), (8, 3)])
 @pytest.mark.parametrize("n_pages", [1, 5, 64, 700])
-def test_gather_split_units_match_oracle(gpu, tuning, heads, dt, split, n_pages):
-    """The one-unit gather with each (page, layer) unit shared by several
-    workgroups (launches of few units; split 0 = the launch policy's
-    choice): the oracle's records, for pages of 32, 64, 16 and 4 KiB (the
-    last cannot split) and one or all layers per launch."""
-    print(f"case: gather split={split} H{heads} {dt} pages={n_pages}", flush=True)
-    tuning("gather_split", split)
+def test_gather_pieces_match_oracle(gpu, tuning, heads, dt, pieces, stores, n_pages):
+    """The gather with 1 and 8 pieces per wave and either store policy (0 = the
+    launch's own): the oracle's records, for pages of 32, 64, 16 and 4 KiB (the
+    last has no 8 pieces) and one or all layers per launch."""
+    print(f"case: gather pieces={pieces} {stores} H{heads} {dt} pages={n_pages}", flush=True)
+    tuning("gather_split", pieces)
+    tuning("scatter_kernel", stores)
     shape = KVShape(3, heads, 128, 16, 1 if dt in FP8 else 2)
     nb = 2 * n_pages + 3
     rng = np.random.default_rng(n_pages + heads)
@@ -243,11 +243,11 @@ def test_prepared_gather_matches_gather(gpu):
 
 
 @pytest.mark.parametrize("heads,head_dim,dt", [
-    (8, 128, "bf16"),   # 32 KiB pages: grouped kernel, one unit per workgroup
-    (1, 128, "bf16"),   # 4 KiB: grouped, 8 units per workgroup
-    (8, 128, "e4m3"),   # 16 KiB e4m3: contig kernel
-    (1, 128, "e4m3"),   # 2 KiB e4m3: grouped
-    (4, 96, "e4m3"),    # row-aligned kernel
+    (8, 128, "bf16"),   # 32 KiB pages
+    (1, 128, "bf16"),   # 4 KiB
+    (8, 128, "e4m3"),   # 16 KiB e4m3
+    (1, 128, "e4m3"),   # 2 KiB e4m3
+    (4, 96, "e4m3"),    # pieces of whole rows
 ])
 def test_per_layer_rerotate_matches_all_layer_launch(gpu, heads, head_dim, dt):
     """Re-rotation launched per layer range (layers=(l, 1)) writes the same
@@ -422,7 +422,7 @@ def _exact_rotation(staging, offsets, shape, layer, page_delta, rot_dim, style, 
         ("e5m2", "gptj", 128, 96),
         ("e5m2", "neox", 192, 192),
         ("e5m2", "neox", 128, 40),
-        # partner distance not a power of two: the row-aligned kernel
+        # partner distance not a power of two: pieces of whole rows
         ("bf16", "neox", 80, 80),
         ("fp16", "neox", 96, 96),
         ("e4m3", "neox", 192, 192),
@@ -467,7 +467,7 @@ def test_rerotate_matches_oracle(gpu, dt, style, head_dim, rot_dim):
 @pytest.mark.parametrize("dt,head_dim", [("bf16", 80), ("fp16", 96), ("e4m3", 192)])
 def test_rerotate_pair_task_kernel_matches_oracle(gpu, tuning, dt, head_dim):
     """The pair-task kernel (kept for rows of more than 64 vectors), forced
-    on the shapes the row-aligned kernel serves by default."""
+    on the shapes that the flat kernel moves in pieces of whole rows."""
     print(f"case: rerotate pair-task {dt} D{head_dim}", flush=True)
     tuning("rot_kernel", "pairs")
     shape, dst, dst_ref, page_ids, page_delta = _rerotate_case(
@@ -589,24 +589,22 @@ def test_rerotate_special_values(gpu, dt):
     None,                          # config 1, Qwen2-0.5B: 256-byte rows (16 vectors)
     KVShape(6, 1, 64, 16, 2),      # 128-byte rows
     KVShape(5, 2, 128, 16, 2),     # 512-byte rows (32 vectors)
-    KVShape(4, 4, 128, 16, 2),     # 1 KiB rows: the large-row kernel
+    KVShape(4, 4, 128, 16, 2),     # 1 KiB rows: cut by themselves
     KVShape(5, 1, 128, 16, 1),     # e4m3, 128-byte rows
     KVShape(3, 1, 32, 32, 2),      # 64-byte rows (4 vectors), block size 32
     KVShape(3, 1, 16, 8, 1),       # 16-byte rows (1 vector)
     KVShape(3, 1, 64, 12, 2),      # 128-byte rows, block size 12 (not a power of two)
 ], ids=["cfg1", "row128", "row512", "row1k", "e4m3_row128", "row64_bs32", "row16",
         "row128_bs12"])
-@pytest.mark.parametrize("unroll,form", [("default", "host"), ("4", "host"),
-                                          ("default", "device")])
-def test_slots_gather_scatter_match_oracle(gpu, tuning, shape, unroll, form):
+@pytest.mark.parametrize("max_wg,form", [(0, "host"), (24, "host"), (0, "device")])
+def test_slots_gather_scatter_match_oracle(gpu, tuning, shape, max_wg, form):
     """slot_mapping-driven token gather/scatter with ragged requests, partial
-    last pages and padding tokens, at each row-size class of the kernels
-    (rows of <= 8 vectors: the packed kernel, at both unrolls). Host tables
-    scatter whole pages through the page kernel and the rest through the
-    token kernel; device tables take the token kernel for every token."""
-    print(f"case: slots gather/scatter {shape} unroll {unroll} {form}", flush=True)
-    if unroll != "default":
-        tuning("slots_unroll", int(unroll))
+    last pages and padding tokens, rows of 1 to 64 vectors, in one launch and
+    in launches of at most 24 workgroups. Host tables scatter whole pages
+    through the page kernel and the rest through the token kernel; device
+    tables take the token kernel for every token."""
+    print(f"case: slots gather/scatter {shape} max_wg {max_wg} {form}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
     wl = workloads.config(1) if shape is None else workloads.ragged(
         shape, 8, 100, 2000, seed=3, num_blocks=1024)
     shape = wl.shape
@@ -725,28 +723,26 @@ def test_large_page_geometry(gpu):
 
 
 # ---------------------------------------------------------------------------
-# pages of whole 4 KiB slices: several units per workgroup
+# small pages: several units per workgroup
 
 
 @pytest.mark.parametrize("layers,heads,head_dim,dt", [
-    (7, 1, 128, "bf16"),   # 4 KiB pages: one slice per unit
-    (5, 2, 128, "bf16"),   # 8 KiB: two slices per unit
+    (7, 1, 128, "bf16"),   # 4 KiB pages
+    (5, 2, 128, "bf16"),   # 8 KiB
     (6, 2, 64, "bf16"),    # Qwen2-0.5B geometry
     (5, 2, 128, "e4m3"),   # 4 KiB e4m3
-    (5, 1, 128, "e4m3"),   # 2 KiB: two units per workgroup slice
+    (5, 1, 128, "e4m3"),   # 2 KiB: two units per workgroup
     (4, 1, 64, "bf16"),    # 2 KiB
     (3, 1, 64, "e4m3"),    # 1 KiB: one unit per wave
 ])
-@pytest.mark.parametrize("group_cap", ["1", "2", "3", ""])
-def test_grouped_units_match_oracle(gpu, tuning, layers, heads, head_dim, dt, group_cap):
-    """Groups span layer boundaries (3 pages, fewer than a group) and end
-    part-way; every grouping (1 = the one-unit kernels) gives the oracle's
-    bytes for gather, scatter and re-rotation."""
-    print(f"case: grouped L{layers} H{heads} D{head_dim} {dt} cap={group_cap!r}", flush=True)
-    if group_cap:
-        tuning("units_per_group", int(group_cap))
-    else:
-        tuning("units_per_group", 0)
+@pytest.mark.parametrize("max_wg,stores", [(0, 0), (16, 1), (16, 3), (24, 0)])
+def test_small_pages_match_oracle(gpu, tuning, layers, heads, head_dim, dt, max_wg, stores):
+    """A workgroup's four waves span units and layers, the last one ends part-way
+    (3 pages), launches end inside a unit (at most max_wg workgroups): the
+    oracle's bytes for gather, scatter and re-rotation."""
+    print(f"case: small pages L{layers} H{heads} D{head_dim} {dt} {max_wg} {stores}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    tuning("scatter_kernel", stores)
     shape = KVShape(layers, heads, head_dim, 16, 1 if dt in FP8 else 2)
     nb = 9
     src = rand_caches(shape, nb, dt, gpu, seed=60, scale=40.0 if dt in FP8 else 1.0)
@@ -794,15 +790,12 @@ def test_grouped_units_match_oracle(gpu, tuning, layers, heads, head_dim, dt, gr
         assert ok, f"layer {l}: {msg}"
 
 
-@pytest.mark.parametrize("group_cap", ["1", ""])
-def test_grouped_units_skip_out_of_range(gpu, tuning, group_cap):
-    """Device tables with an out-of-range block inside a group: that unit is
-    skipped in every layer, its neighbours in the group still move."""
-    print(f"case: grouped skip cap={group_cap!r}", flush=True)
-    if group_cap:
-        tuning("units_per_group", int(group_cap))
-    else:
-        tuning("units_per_group", 0)
+@pytest.mark.parametrize("max_wg", [0, 16])
+def test_small_pages_skip_out_of_range(gpu, tuning, max_wg):
+    """Device tables with an out-of-range block: that page is skipped in every
+    layer, its neighbours in the workgroup still move."""
+    print(f"case: small pages skip {max_wg}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
     shape = KVShape(5, 1, 128, 16, 2)
     src = rand_caches(shape, 8, "bf16", gpu, seed=61)
     staging = torch.zeros(3 * shape.slot_bytes, dtype=torch.uint8, device=gpu)
@@ -834,9 +827,9 @@ def test_grouped_units_skip_out_of_range(gpu, tuning, group_cap):
 
 
 @pytest.mark.parametrize("layers,heads,head_dim,dt", [
-    (4, 8, 128, "bf16"),    # one-unit kernels
-    (7, 1, 128, "bf16"),    # grouped (4 KiB pages)
-    (5, 1, 128, "e4m3"),    # grouped (2 KiB pages)
+    (4, 8, 128, "bf16"),    # 32 KiB pages
+    (7, 1, 128, "bf16"),    # 4 KiB
+    (5, 1, 128, "e4m3"),    # 2 KiB
 ])
 def test_launch_split_matches_single_launch(gpu, tuning, layers, heads, head_dim, dt):
     """Calls whose workgroups exceed one launch's limit run as several
@@ -1055,7 +1048,7 @@ def test_random_geometry_parity(gpu, dt, D, H, bs, style, R, L, seed):
             assert torch.equal(back.view(torch.uint8), rot[l].view(torch.uint8)), \
                 f"split-x layer {l}"
     # head-major (HND) pages holding the same values: the same records, and
-    # (where the contig / grouped kernels apply) the same re-rotated bits
+    # (where the head-major kernels apply) the same re-rotated bits
     if H > 1 and bs > 1:
         def hnd_like(cs):
             out = []
@@ -1297,32 +1290,35 @@ def test_shared_records_hint_does_not_change_results(gpu, heads, head_dim, dt):
 
 @pytest.mark.parametrize("heads,head_dim,dt", [(1, 128, "bf16"), (1, 128, "e4m3"),
                                               (2, 64, "bf16")])
-def test_rerotate_contig_override_on_small_pages(gpu, tuning, heads, head_dim, dt):
-    """Small pages default to the grouped kernel; the "contig" rot_kernel override runs
-    the one-unit contig kernel instead, which must then be launched with one
-    unit per workgroup (every page written, same bits as the grouped
-    kernel)."""
-    print(f"case: contig override H{heads} D{head_dim} {dt}", flush=True)
-    shape, dst, dst_ref, page_ids, _ = _rerotate_case(gpu, dt, "neox", head_dim, head_dim,
+@pytest.mark.parametrize("style", ["neox", "gptj"])
+def test_rerotate_pairs_override_on_small_pages(gpu, tuning, heads, head_dim, dt, style):
+    """Small pages through the flat kernel and, by the "pairs" override, through
+    the pair-task kernel: the same bits, and the oracle's within the tolerance."""
+    print(f"case: pairs override H{heads} D{head_dim} {dt} {style}", flush=True)
+    shape, dst, dst_ref, page_ids, _ = _rerotate_case(gpu, dt, style, head_dim, head_dim,
                                                       heads=heads, layers=3, seed=8)
-    tuning("rot_kernel", "contig")
-    shape2, dst2, _, page_ids2, _ = _rerotate_case(gpu, dt, "neox", head_dim, head_dim,
+    tuning("rot_kernel", "pairs")
+    shape2, dst2, _, page_ids2, _ = _rerotate_case(gpu, dt, style, head_dim, head_dim,
                                                    heads=heads, layers=3, seed=8)
     torch.cuda.synchronize()
     assert np.array_equal(page_ids, page_ids2)
-    for a, b in zip(dst, dst2):
+    for l, (a, b) in enumerate(zip(dst, dst2)):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        got = to_bits_np(a, dt)
+        assert np.array_equal(got[1], dst_ref[l][1])
+        ok, msg = rotation_within_tolerance(got[0], dst_ref[l][0], dt)
+        assert ok, f"layer {l}: {msg}"
 
 
 @pytest.mark.parametrize("heads,head_dim,dt,kernel", [
-    (8, 128, "bf16", None),    # grouped kernel, one unit per workgroup
-    (1, 128, "bf16", None),    # grouped, several units per workgroup
-    (8, 128, "e4m3", None),    # contig kernel
-    (8, 128, "e5m2", None),    # contig kernel, e5m2
-    (1, 128, "e5m2", None),    # grouped, e5m2
-    (4, 96, "bf16", None),     # row-aligned kernel
+    (8, 128, "bf16", None),    # 32 KiB pages
+    (1, 128, "bf16", None),    # 4 KiB
+    (8, 128, "e4m3", None),    # 16 KiB
+    (8, 128, "e5m2", None),    # 16 KiB, e5m2
+    (1, 128, "e5m2", None),    # 2 KiB, e5m2
+    (4, 96, "bf16", None),     # pieces of whole rows
     (4, 96, "bf16", "pairs"),  # pair-task kernel
-    (16, 128, "bf16", None),   # 64 KiB pages: contig kernel in rounds
+    (16, 128, "bf16", None),   # 64 KiB pages
     (4, 96, "bf16", "lds24"),  # rotary width 24 of 96: the LDS kernel
 ])
 def test_rerotate_per_layer_groups(gpu, tuning, heads, head_dim, dt, kernel):
@@ -1538,8 +1534,8 @@ def _hnd_caches(shape, nb, dt, gpu, seed, scale=1.0):
 
 @pytest.mark.parametrize("heads,head_dim,bs,dt", [
     (8, 128, 16, "bf16"), (2, 64, 16, "bf16"), (4, 128, 32, "e4m3"), (3, 96, 16, "bf16"),
-    (2, 32, 16, "bf16"),   # 2 KiB pages: the grouped copies
-    (4, 64, 16, "e4m3"),   # 4 KiB e4m3: grouped scatter, one-unit gather
+    (2, 32, 16, "bf16"),   # 2 KiB pages
+    (4, 64, 16, "e4m3"),   # 4 KiB e4m3 pages
 ])
 def test_hnd_copies_match_oracle(gpu, heads, head_dim, bs, dt):
     """Gather from head-major pages writes the records of the logical page
@@ -1580,10 +1576,10 @@ def test_hnd_copies_match_oracle(gpu, heads, head_dim, bs, dt):
 @pytest.mark.parametrize("heads,head_dim,rot,dt,style", [
     (8, 128, 128, "bf16", "neox"), (2, 64, 64, "bf16", "neox"), (4, 128, 128, "e4m3", "neox"),
     (2, 128, 128, "bf16", "gptj"), (4, 128, 64, "bf16", "neox"),
-    (2, 128, 128, "e4m3", "neox"),  # 4 KiB e4m3 pages: grouped
+    (2, 128, 128, "e4m3", "neox"),  # 4 KiB e4m3 pages
     (4, 128, 128, "e5m2", "gptj"),
-    (2, 32, 32, "bf16", "neox"),    # 2 KiB pages: grouped, 16 units per workgroup
-    (16, 128, 128, "bf16", "neox"),  # 64 KiB pages: contig in rounds
+    (2, 32, 32, "bf16", "neox"),    # 2 KiB pages
+    (16, 128, 128, "bf16", "neox"),  # 64 KiB pages
 ])
 def test_hnd_rerotate_equals_token_major(gpu, heads, head_dim, rot, dt, style):
     """Re-rotation into head-major pages gives, per logical element, exactly
@@ -1630,22 +1626,18 @@ def test_hnd_rerotate_unsupported_width_refused(gpu):
         ops.scatter_rerotate(ops.LayerTable(caches), [1], [0], st, tabs, [0])
 
 
-@pytest.mark.parametrize("H,D,bs,style,parts", [
-    (8, 128, 32, "neox", 0), (8, 256, 16, "neox", 0), (8, 128, 32, "gptj", 0),
-    (32, 96, 16, "neox", 0), (32, 96, 16, "neox", 2), (8, 128, 32, "neox", 1),
-    (8, 128, 48, "neox", 0), (8, 128, 32, "neox", -64), (32, 96, 16, "neox", -64)])
-def test_large_pages_in_parts_match_oracle(gpu, tuning, H, D, bs, style, parts):
-    """Pages above 32 KiB move in parts of whole rows, one workgroup each:
-    the gather, the streaming scatter, the grouped re-rotation (64 KiB
-    pages) and the row-aligned re-rotation (head_dim 96, 96 KiB pages) give
-    the oracle's bytes and rotation (parts 0 = the launch policy's choice,
-    1 = whole pages; 96 KiB pages at block_size 48; -n: the policy's parts
-    with launches cut to n workgroups, so one call runs as many launches)."""
-    print(f"case: large pages H{H} D{D} bs{bs} {style} parts={parts}", flush=True)
-    if parts > 0:
-        tuning("page_parts", parts)
-    elif parts < 0:
-        tuning("max_wg_per_launch", -parts)
+@pytest.mark.parametrize("H,D,bs,style,max_wg,stores", [
+    (8, 128, 32, "neox", 0, 0), (8, 256, 16, "neox", 0, 0), (8, 128, 32, "gptj", 0, 0),
+    (32, 96, 16, "neox", 0, 0), (32, 96, 16, "neox", 0, 1), (8, 128, 32, "neox", 0, 3),
+    (8, 128, 48, "neox", 0, 0), (8, 128, 32, "neox", 64, 0), (32, 96, 16, "neox", 64, 0)])
+def test_large_pages_match_oracle(gpu, tuning, H, D, bs, style, max_wg, stores):
+    """Pages above 32 KiB (64 KiB, 96 KiB of 96-dim heads and of block_size 48): the
+    gather, the scatter and the re-rotation give the oracle's bytes and
+    rotation, with either store policy and with launches cut to max_wg
+    workgroups, inside a page."""
+    print(f"case: large pages H{H} D{D} bs{bs} {style} {max_wg} {stores}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    tuning("scatter_kernel", stores)
     shape = KVShape(3, H, D, bs, 2)
     wl = workloads.ragged(shape, 5, 30, 900, seed=H + D + bs, pool_slack=1.2)
     caches = rand_caches(shape, wl.num_blocks, "bf16", gpu, seed=71)

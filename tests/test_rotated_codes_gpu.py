@@ -51,6 +51,7 @@ def _codes(stored, tabs, rot, style, dt, whole_vectors):
 @pytest.mark.parametrize("kernel,heads,dim,rot,style", [
     ("pages", 8, 128, 128, "neox"), ("pages", 2, 64, 64, "gptj"), ("pages", 4, 96, 96, "neox"),
     ("pages", 4, 96, 24, "neox"), ("pages", 2, 96, 20, "gptj"), ("pairs", 4, 96, 96, "neox"),
+    ("pairs", 8, 128, 128, "neox"), ("pairs", 2, 64, 32, "gptj"),
     ("hnd", 4, 128, 128, "neox"), ("kx", 8, 128, 128, "neox"), ("fanout", 8, 128, 64, "neox"),
     ("fanout", 8, 128, 128, "gptj"), ("tokens", 1, 128, 128, "neox"),
     ("tokens", 8, 128, 128, "neox"), ("tokens", 2, 64, 64, "gptj")])

@@ -14,8 +14,8 @@
 // Measured against workgroups of whole units (16 KiB pages 1,127 of 28
 // layers, 64 KiB pages 42 layers, both ways in one process): scatter 5.54 ->
 // 6.11 and 5.90 -> 6.57 TB/s, gather 5.94 -> 6.26 and 6.57 -> 6.57; 4 KiB pages
-// scatter 5.32 -> 5.94; a 16-page load of 24 layers 9.7 -> 5.9 us, whose
-// workgroup of whole units had 24 workgroups in all.
+// scatter 5.32 -> 5.94; a 16-page load of 24 layers takes 3.4 us, by the
+// profiler.
 
 #pragma once
 

@@ -1160,7 +1160,7 @@ int dsr_scatter_fanout(const uint64_t* layer_base, int n_layers, int64_t kv_stri
   if (rc != DSR_OK) return rc;
   // the geometry is checked before the empty-work return below, so that a
   // call with n_dst = 0 tells whether the fan-out takes a geometry
-  // pages of at most 32 KiB
+  // pages of at most 32 KiB (larger ones are refused, unmeasured)
   if (page_bytes > (32 << 10)) return DSR_ERR_SHAPE;
   RotArgs ra{};
   ra.u = make_unit(layer_base, n_layers, kv_stride, page_stride, page_bytes, num_blocks,

@@ -133,7 +133,9 @@ __global__ __launch_bounds__(kThreads) void kv_slots_flat_kernel(SlotArgs a, Fla
 // lanes read their token's pairs themselves, 64 or 128 bytes for each 16 that
 // they move (one-head e4m3 rows: 2.9 TB/s, 4.2 through LDS). Lanes without a valid
 // token take part in the shuffles and move nothing.
-constexpr int kSlotRotMaxHalf = 128;  // rot_dim <= 256
+// rot_dim <= 256. The kernel takes more (its tables are sized at launch); wider
+// ones are refused, unmeasured.
+constexpr int kSlotRotMaxHalf = 128;
 
 template <int DT, int STYLE, bool WIDE, int POLICY>
 __global__ __launch_bounds__(kThreads) void kv_slots_flat_rerotate_kernel(SlotArgs a, RotArgs ra,

@@ -21,7 +21,8 @@ namespace {
 int64_t round16(int64_t v) { return (v + 15) & ~(int64_t)15; }
 
 // Numbers the distinct values of v in the order of their first appearance:
-// open addressing over twice as many places.
+// open addressing over twice as many places, by the multipliers of Steele, Lea
+// and Flood's SplitMix64.
 class Distinct {
  public:
   explicit Distinct(int n) {

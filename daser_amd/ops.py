@@ -693,7 +693,8 @@ class PreparedFanout:
     """A load of host tables whose pages share records (a cached chunk
     placed in several requests), through dsr_scatter_fanout: each record is
     read once and written to all of its pages. The tables are checked,
-    grouped by record (:func:`fanout_tables`) and uploaded once; each call
+    grouped by record (dsr_plan_load, as :func:`fanout_tables`) and uploaded
+    once; each call
     launches the load on the current stream. ``rope``: None for a plain
     copy, else (rope_idx, cos_sin, rot_dim, style, k_scale, layer_group) as
     for :func:`scatter_rerotate`. Pages must satisfy
@@ -1036,7 +1037,8 @@ def scatter_slots(table: LayerTable, slot_mapping, row_offsets, staging: torch.T
     """Inverse of :func:`gather_slots`. Host tables are processed in
     destination-slot order (near-sequential writes), like :func:`scatter`,
     and blocks whose every slot is listed with consecutive record rows go
-    as whole pages through the page scatter (:func:`whole_pages`); the other
+    as whole pages through the page scatter (dsr_plan_slots, as
+    :func:`whole_pages`); the other
     tokens (the ragged edges of requests) go through the token kernel;
     whole pages that share records load through :class:`PreparedFanout`,
     as in :func:`scatter`. Device tables go to the token kernel as given."""

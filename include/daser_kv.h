@@ -51,7 +51,9 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  * re-rotations' flags, 5 the head-major (_hnd) entry points, 6
  * dsr_set_tuning, 7 dsr_scatter_ex, 8 dsr_scatter_slots_rerotate, 9
  * DSR_RING_MMAP and dsr_ring_is_mapped, 10 dsr_scatter_rerotate_static, 11
- * dsr_scatter_fanout. Callers check dsr_abi_version() against it. */
+ * dsr_scatter_fanout, 12 the host-table planners (dsr_plan_*), dsr_put,
+ * dsr_delta_tables and dsr_gather_layers. Callers check dsr_abi_version()
+ * against it. */
 #define DSR_ABI_VERSION 12
 
 /*
@@ -61,7 +63,8 @@ typedef struct ihipStream_t* dsr_stream_t; /* == hipStream_t */
  * geometry's own choice):
  *   DSR_TUNE_MAX_WG_PER_LAUNCH    split calls into launches of <= n workgroups
  *   DSR_TUNE_ROT_KERNEL           1: the pair-task re-rotation kernel where
- *                                 the flat one applies too
+ *                                 the flat one applies too (token-major and
+ *                                 split-x pages)
  *   DSR_TUNE_ROT_WG_PER_CU        workgroups per CU of the re-rotation
  *   DSR_TUNE_COPY_WG_PER_CU       workgroups per CU of the page gather / scatter
  *   DSR_TUNE_COPY_STORES          (DSR_TUNE_SCATTER_KERNEL) store policy of the
@@ -207,7 +210,9 @@ int dsr_scatter_ex(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
  * saturate too (a saturate-to-finite encode, the mode vLLM's fp8 cache
  * writes use, not torch's float8_e5m2 cast, which keeps infinities); NaN
  * -> 0x7F.
- * bf16/fp16: round-to-nearest-even from fp32; NaN -> canonical quiet NaN.
+ * In all formats p * s is rounded to fp32 and the sum x * c + (p * s) is fused.
+ * bf16: round-to-nearest-even from fp32. fp16: the fused sum is rounded to fp16
+ * at once (rotary widths of part vectors: from fp32). NaN -> canonical quiet NaN.
  *
  * The reference has no re-rotation (daser/position/fixed_offset.py:11-50
  * only carries an integer offset, which this path consumes); the copy it
@@ -263,7 +268,8 @@ int dsr_scatter_rerotate(const uint64_t* layer_base, int n_layers,
  * request's pages copied from its staged chunk), for requests that share
  * cached chunks; the reference reads a shared chunk once per request.
  *
- * Geometry: pages of at most 32 KiB (8 vectors per lane); with rotation,
+ * Geometry: pages of at most 32 KiB (the kernel has no such limit; larger ones
+ * are refused, unmeasured, and take the per-page entry points); with rotation,
  * whole-vector rotary widths and neox partners a power of two <= 32 vectors
  * apart dividing the row, or gptj. k_layout names the cache pages:
  * DSR_K_NHD token-major (block_size and num_heads unused), DSR_K_KX the

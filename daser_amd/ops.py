@@ -900,7 +900,8 @@ def _slots_host(table: LayerTable, slot_mapping, row_offsets, staging: torch.Ten
     """A token-form call with host tables: planned by the library, its whole
     pages (loads) through the page form, the other tokens through the token
     kernels. ``rope`` as for :func:`_load_host`. False, having done nothing, for
-    tables that the library cannot plan (device tables, empty or odd ones)."""
+    tables that the library cannot plan (device tables, empty or odd ones) and
+    for padding alone."""
     if _on_device(slot_mapping):
         return False
     lay = table.layout
@@ -928,6 +929,8 @@ def _slots_host(table: LayerTable, slot_mapping, row_offsets, staging: torch.Ten
         _addr(sm), _addr(ro), _addr(ridx), sm.size, lay.num_blocks, lay.block_size, row,
         max(end, 0), nbytes, n_tables, mode, host.data_ptr(), size, ctypes.addressof(plan)),
         lay.num_blocks)
+    if not plan.n_pages and not plan.n_tokens:  # padding alone: the launch's checks remain
+        return False
     if plan.n_pages:
         at = host.numpy()
         ids, offs, prope = (at[o:o + 8 * plan.n_pages].view(np.int64) for o in

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from daser_amd import ops
+from daser_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -250,6 +250,33 @@ def test_flat_slots(gpu, tuning, heads, dim, dt, block, max_wg):
             exp[:, :, int(ids[t // block]), t % block] = tmp[:, :, int(ids[t // block]), t % block]
     torch.cuda.synchronize()
     assert torch.equal(rot.view(torch.uint8), exp.view(torch.uint8))
+
+
+@pytest.mark.parametrize("where", ["host", "device"])
+def test_padding_alone_is_checked(gpu, where):
+    """A token load whose slots are all padding is refused where its geometry is
+    (96-dim neox heads), and else moves nothing."""
+    for dim in (96, 128):
+        print(f"case: padding alone {where} D{dim}", flush=True)
+        whole, views, _, _ = _setup(gpu, 2, 2, 8, 2, dim, "nhd", seed=1)
+        before = whole.clone()
+        table = ops.LayerTable(views)
+        staging = torch.ones(table.layout.slot_bytes, dtype=torch.uint8, device=gpu)
+        dev = gpu if where == "device" else "cpu"
+        slots = torch.full((5,), -1, dtype=torch.int64, device=dev)
+        rows = torch.arange(5, dtype=torch.int64, device=dev) * dim * 4
+        ridx = torch.zeros(5, dtype=torch.int32, device=dev)
+        tabs = torch.ones((1, dim // 2, 2), device=gpu)
+        if dim == 96:
+            with pytest.raises(_lib.DaserKVError):
+                ops.scatter_slots_rerotate(table, slots, rows, staging, tabs, ridx)
+        else:
+            ops.scatter_slots_rerotate(table, slots, rows, staging, tabs, ridx)
+        ops.scatter_slots(table, slots, rows, staging)
+        ops.gather_slots(table, slots, rows, staging)
+        torch.cuda.synchronize()
+        assert torch.equal(whole.view(torch.int16), before.view(torch.int16))
+        assert (staging == 1).all()
 
 
 @pytest.mark.parametrize("heads,dim", [(5, 104), (16, 128)])

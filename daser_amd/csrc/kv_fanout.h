@@ -29,9 +29,12 @@ struct FanArgs {
 // A destination's table is fetched while the one before is being written (the
 // first 128 pairs; wider tables read the rest when they are needed). ROT false:
 // a plain copy. Cache layouts (LAYOUT) as in kv_flat_rerotate_kernel; POLICY: the
-// stores' cache policy.
+// stores' cache policy. A source's destinations may be dealt to several waves
+// (`split` shares of each piece): where few waves hold many destinations, each a
+// table's way through LDS after the other, that chain bounds the load.
 template <int DT, int STYLE, int LAYOUT, bool ROT, int POLICY>
 __global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa, FlatMap m, FastDiv row,
+                                                             FastDiv pieces, int split,
                                                              bool layer_major) {
   extern __shared__ float2 lds_tab[];
   const RotArgs& ra = fa.ra;
@@ -40,13 +43,17 @@ __global__ __launch_bounds__(kThreads) void kv_fanout_kernel(FanArgs fa, FlatMap
   if (w >= m.n_waves) return;
   const uint32_t g = m.wave0 + w;
   const uint32_t qu = div_by(g, m.per_unit);
-  const uint32_t part = g - qu * m.per_unit.d;
+  const uint32_t share = div_by(g - qu * m.per_unit.d, pieces);
+  const uint32_t part = g - qu * m.per_unit.d - share * pieces.d;
   const uint32_t un = m.unit0 + qu;
   const uint32_t hi = div_by(un, m.minor);
   const uint32_t lo = un - hi * m.minor.d;
   const uint32_t s = layer_major ? lo : hi, l = layer_major ? hi : lo;
   const int64_t off = fa.src_offsets[s] + (int64_t)(a.layer0 + (int)l) * a.layer_bytes;
-  const int d0 = fa.dst_start[s], d1 = fa.dst_start[s + 1];
+  const int all0 = fa.dst_start[s], all1 = fa.dst_start[s + 1];
+  const int each = (all1 - all0 + split - 1) / split;
+  const int d0 = all0 + (int)share * each;
+  const int d1 = d0 + each < all1 ? d0 + each : all1;
   if (off < 0 || off + 2 * a.page_bytes > a.staging_bytes || d1 <= d0) return;
   const int lane = (int)threadIdx.x % kWave;
   const int first = (int)part * kWave;

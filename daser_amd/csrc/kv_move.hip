@@ -1087,6 +1087,13 @@ namespace {
 //   256 1,655 against 1,697; 70B TP8 rotated 3,489 against 3,633), which a smaller load
 //   takes (1,024 TP8 pages of 256 165 against 169; on buffers in turn that the
 //   memory-side cache does not hold, up to 10% ahead at 128 pages).
+//   Rotated loads of fewer waves than 4 workgroups per CU hold deal each record's
+//   destinations to as many as fill them, at least 4 to a wave: 0.5B, 64 pages of one
+//   record 1,212 / 322 / 1,675 (40 sets of buffers), 1,000 of one 3,012 / 324 / 4,314 (7),
+//   256 of 4 710 / 301 / 978 (23); pages from 16 KiB also where a record has 64 or more,
+//   16 to a wave: 8B, 1,024 of 16 843 / 816 / 892 (2 sets), e4m3 521 / 438 / 490; 4 KiB
+//   pages of more waves lose 3-10% by it. Up to twice those waves, 8 per CU in place of
+//   4: TP8, 1,024 of 16 279 / 276 / 301 (2), 0.5B, 512 of 64 257 / 243 / 259 (11).
 //   4 workgroups per CU, for few destinations 6, on such buffers: 0.5B rotated, 512 of
 //   64 1.01 times the old kernel's rate at 4, 0.94 at 6; 8B rotated, 128 of 64 1.33 and
 //   1.38, TP8 plain, 64 of 32 1.10 and 1.16.
@@ -1094,6 +1101,8 @@ namespace {
 constexpr int64_t kFanManySources = 512;
 constexpr int64_t kFanLargeBytes = 1 << 30;
 constexpr int kFanFewPages = 256;
+constexpr int64_t kFanFillWaves = 4096;  // 4 workgroups on each of 256 CUs
+constexpr int64_t kFanMaxSplit = 64;
 
 template <int DT, int STYLE, int LAYOUT, bool ROT>
 int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
@@ -1104,19 +1113,33 @@ int launch_fanout_s(const FanArgs& fa, hipStream_t s) {
   const bool many = fa.n_src >= kFanManySources;
   const bool large =
       2 * ra.u.page_bytes * ra.u.n_layers * ((int64_t)fa.n_src + fa.n_dst) > kFanLargeBytes;
-  const int64_t t = tune(DSR_TUNE_FANOUT_WG_PER_CU);
-  const size_t lds = occupancy_lds(t ? (int)t : fa.n_dst > kFanFewPages ? 4 : 6, 0);
+  const int64_t pieces = (ra.u.page_bytes + kPiece - 1) / kPiece;
+  const int64_t waves = (int64_t)fa.n_src * ra.u.n_layers * pieces;
+  int wg = fa.n_dst > kFanFewPages ? 4 : 6;
+  int64_t split = 1;
+  if (ROT) {
+    const int64_t dests = fa.n_dst / fa.n_src;
+    split = kFanFillWaves / waves;
+    if (ra.u.page_bytes >= 16 << 10 && dests >= 64 && split < dests / 16) split = dests / 16;
+    if (split > dests / 4) split = dests / 4;
+    if (split > kFanMaxSplit) split = kFanMaxSplit;
+    if (split < 1) split = 1;
+    if (split == 1 && waves > kFanFillWaves && waves <= 2 * kFanFillWaves) wg = 8;
+  }
+  if (const int64_t t = tune(DSR_TUNE_FANOUT_WG_PER_CU)) wg = (int)t;
+  const size_t lds = occupancy_lds(wg, 0);
   const size_t dyn = lds > tabs ? lds : tabs;
   const FastDiv row = fast_div((uint32_t)(ROT ? ra.row_vecs : 1));
-  return launch_flat((int64_t)fa.n_src * ra.u.n_layers, (ra.u.page_bytes + kPiece - 1) / kPiece,
+  const FastDiv share = fast_div((uint32_t)pieces);
+  return launch_flat((int64_t)fa.n_src * ra.u.n_layers, pieces * split,
                      many ? ra.u.n_layers : fa.n_src, 0,
                      [&](const FlatMap& m, unsigned grid) {
     if (large)
       kv_fanout_kernel<DT, STYLE, LAYOUT, ROT, kStorePolicy>
-          <<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
+          <<<grid, kThreads, dyn, s>>>(fa, m, row, share, (int)split, !many);
     else
       kv_fanout_kernel<DT, STYLE, LAYOUT, ROT, kStoreNtSc>
-          <<<grid, kThreads, dyn, s>>>(fa, m, row, !many);
+          <<<grid, kThreads, dyn, s>>>(fa, m, row, share, (int)split, !many);
   });
 }
 

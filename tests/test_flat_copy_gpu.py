@@ -350,6 +350,40 @@ def test_flat_fanout(gpu, n_src, n_dst, heads, dim, dt, layout, rot):
     assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
 
 
+@pytest.mark.parametrize("counts,heads,dim,layout,max_wg", [
+    ((1000,), 1, 64, "nhd", 0), ((700, 1, 3, 0, 96), 2, 64, "nhd", 0),
+    ((700, 1, 3, 0, 96), 2, 64, "hnd", 16), ((64,), 8, 128, "kx", 0),
+    ((130, 62), 8, 128, "nhd", 0), ((7, 9), 8, 128, "nhd", 24), ((65, 66, 64), 5, 128, "nhd", 0)])
+def test_fanout_shares_of_destinations(gpu, tuning, counts, heads, dim, layout, max_wg):
+    """Few records of many destinations: each record's are dealt to several waves,
+    uneven counts (records of none among them): bit for bit the per-page load."""
+    print(f"case: fanout shares {counts} H{heads} D{dim} {layout} {max_wg}", flush=True)
+    tuning("max_wg_per_launch", max_wg)
+    layers, block, n = 2, 16, sum(counts)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    rng = np.random.default_rng(n)
+    inner = {"nhd": (block, heads, dim), "hnd": (heads, block, dim),
+             "kx": (block * heads * dim,)}[layout]
+    geo = dict(block_size=block, head_dim=dim) if layout == "kx" else {}
+    caches = [torch.zeros((layers, 2, n + 3, *inner), dtype=torch.bfloat16, device=gpu)
+              for _ in range(2)]
+    tables = [ops.LayerTable([w.transpose(2, 3) if layout == "hnd" else w for w in c.unbind(0)],
+                             **geo) for c in caches]
+    slot = tables[0].layout.slot_bytes
+    staging = torch.randn(len(counts) * slot // 2, generator=g, device=gpu).to(torch.bfloat16) \
+        .view(torch.uint8)
+    ids = rng.permutation(n + 3)[:n].astype(np.int64)
+    offs = np.repeat(np.arange(len(counts), dtype=np.int64), counts) * slot
+    ang = torch.rand((5, dim // 2), generator=g, device=gpu, dtype=torch.float64) * 6.28
+    tabs = torch.stack([ang.cos(), ang.sin()], -1).float()
+    ridx = rng.integers(-1, 5, n)
+    ops.PreparedFanout(tables[0], ids, offs, staging, rope=(ridx, tabs, dim, "neox", None, None))()
+    ops.scatter_rerotate(tables[1], ids, offs, staging, tabs, ridx, shared_records=False)
+    torch.cuda.synchronize()
+    assert torch.equal(*(c.view(torch.int16) for c in caches))
+    assert caches[0].view(torch.int16).any()
+
+
 @pytest.mark.parametrize("n_src,n_dst", [(300, 3800), (1000, 3100)])
 def test_large_fanout(gpu, n_src, n_dst):
     """The fan-out's launch above 1 GiB, both unit orders: what the per-page load

@@ -208,9 +208,10 @@ size_t occupancy_lds(int wg_per_cu, int64_t static_lds) {
 //   above: nt sc0 sc1 stores, in chunks of workgroups (kChunk): 50.3 -> 42.1
 //     us at 268 MB (nt 42.9), 185 -> 163 at 1.07 GB (nt 169), 738 -> 664 at 4.3
 //     GB (nt 681).
-// Where the same few buffers stay in the memory-side cache, sc0 sc1 stores are
-// up to 8% ahead of nt between 60 and 170 MB; a load's pages and records are
-// not there.
+// Where the same buffers come again at once and stay in the memory-side cache, the
+// replaced kernels' sc0 sc1 stores were 10-20% ahead from 60 to 500 MB moved (8B
+// gather of 500 MB 62.1 -> 78.5 us; on four sets in turn 83.4 -> 78.8, scatter 92.2 ->
+// 76.3); a load's pages and records are not there.
 // Four workgroups of single pieces per CU: 32 KiB of reads in flight there hide
 // the latency, and 6 or 8 per CU widen the written window (0-8% slower).
 constexpr int kCopyWgPerCu = 4;

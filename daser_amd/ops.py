@@ -452,9 +452,14 @@ def gather(
     record index of table layer ``first + i`` is ``layer0 + first + i``.
     """
     lay = table.layout
+    fn, name, extra = _copy_entry(lay, "dsr_gather")
+    if _on_device(page_ids):
+        args, _tables = _copy_args(table, page_ids, slot_offsets, staging, layer0, layers,
+                                   records_written=True)
+        _lib.check(name, fn(*args, *extra, _stream_handle(lay.device)))
+        return
     (ids, offs), _plan = _gather_tables(table, page_ids, slot_offsets, staging, layer0, layers)
     first, count = _layer_range(lay, layers)
-    fn, name, extra = _copy_entry(lay, "dsr_gather")
     rc = fn(table.ptr(first), count, lay.kv_stride, lay.page_stride, lay.page_bytes,
             lay.num_blocks, ids.data_ptr(), offs.data_ptr(), ids.numel(), staging.data_ptr(),
             staging.numel() * staging.element_size(), lay.layer_bytes, layer0 + first, *extra,

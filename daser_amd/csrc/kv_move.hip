@@ -150,13 +150,9 @@ int launch_flat(int64_t n_units, int64_t pieces_per_unit, int64_t minor, uint32_
     m.unit0 = (uint32_t)(g0 / pieces_per_unit);
     m.wave0 = (uint32_t)(g0 % pieces_per_unit);
     m.n_waves = (uint32_t)n;
-    uint32_t c = chunk;
-    if (chunk == kEighths) {
-      grid = (grid + kXcds - 1) / kXcds * kXcds;  // the waves past the end leave at once
-      c = grid / kXcds;
-    }
-    m.chunk = fast_div(c ? c : 1);
-    m.chunked = c ? grid / (kXcds * c) * (kXcds * c) : 0;
+    if (chunk == kEighths) grid = (grid + kXcds - 1) / kXcds * kXcds;  // the rest leave at once
+    m.chunked = chunk == kEighths ? kEighthsBit | grid / kXcds
+                : chunk == kChunk ? grid / (kXcds * kChunk) * (kXcds * kChunk) : 0;
     launch(m, grid);
     const int rc = (int)hipGetLastError();
     if (rc != 0) return rc;

@@ -657,7 +657,8 @@ def fanout_tables(page_ids: np.ndarray, slot_offsets: np.ndarray,
     """Host tables of a scatter (destination order, one entry per block)
     grouped by source record: (src_offsets, dst_start, dst_pages, dst_rope),
     where the destinations of source s are entries dst_start[s] to
-    dst_start[s + 1] - 1, in block order."""
+    dst_start[s + 1] - 1, in block order. For callers of the C ABI; the loads
+    here have the library group them (dsr_plan_load)."""
     ids = np.asarray(page_ids, np.int64)
     offs = np.asarray(slot_offsets, np.int64)
     order = np.argsort(offs, kind="stable")  # keeps block order inside a source
@@ -995,7 +996,9 @@ def whole_pages(slot_mapping: np.ndarray, row_offsets: np.ndarray, block_size: i
                 row_bytes: int, rope_idx: Optional[np.ndarray] = None):
     """Splits the host tables of a token-form scatter into whole pages and
     the rest. The entries must be in slot order with no slot listed twice
-    (padding, -1, anywhere). A block is whole when its block_size slots sit
+    (padding, -1, anywhere). :func:`scatter_slots` has the library make the same
+    split (dsr_plan_slots); this one is for callers whose tables stay resident.
+    A block is whole when its block_size slots sit
     in consecutive entries, in order, with consecutive record rows
     (row_offsets stepping by row_bytes: the block's K rows form one record
     page, its V rows the page after) and, with rope_idx, one table index.

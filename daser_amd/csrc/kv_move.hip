@@ -703,17 +703,17 @@ int dsr_scatter_hnd(const uint64_t* layer_base, int n_layers, int64_t kv_stride,
 namespace {
 
 // The token form's pieces: rows of 64 vectors and more are cut by themselves,
-// 16 tokens to a unit; of shorter rows a unit holds at least 256 vectors, one
+// `wide_tokens` tokens to a unit; of shorter rows a unit holds at least 256 vectors, one
 // workgroup's.
 struct SlotShape {
   bool wide;
   int64_t pieces;  // per unit
   int64_t units;   // per layer
 };
-SlotShape slot_shape(SlotArgs* a) {
+SlotShape slot_shape(SlotArgs* a, int wide_tokens = 16) {
   const int64_t vpr = a->row_bytes >> 4;
   SlotShape h{vpr >= kWave, 0, 0};
-  a->unit_tokens = (int32_t)(vpr >= 16 ? 16 : 16 * ((16 + vpr - 1) / vpr));
+  a->unit_tokens = (int32_t)(h.wide ? wide_tokens : vpr >= 16 ? 16 : 16 * ((16 + vpr - 1) / vpr));
   const int64_t per_row = h.wide ? (vpr + kWave - 1) / kWave : vpr;
   a->row = fast_div((uint32_t)per_row);
   h.pieces = h.wide ? a->unit_tokens * per_row : (a->unit_tokens * vpr + kWave - 1) / kWave;
@@ -734,15 +734,18 @@ int slots_wg_per_cu(bool gather, bool wide) {
 }
 
 // Gathers of rows up to 4 KiB that move more than 16 GiB: sc0 sc1 stores, workgroups
-// dealt one by one. The kernel of 16 tokens per workgroup that this one replaced /
-// chunks and nt sc0 sc1 stores / this: 2 KiB rows of 32 layers 70,000 tokens 2,863 / 2,913 /
-// 2,893 us, 283,000 11,533 / 11,682 / 11,588, of 80 layers 70,000 7,481 / 7,433 / 7,218; 4 KiB
-// rows of 42 layers 108,000 12,557 / 12,309 / 12,065; 1 KiB rows of 32 layers 283,000 7,046 /
-// 6,327 / 5,976. Smaller gathers: within 1% either way, 1 KiB rows of 11,000 tokens 294 / 236 /
-// 241; rows of 6 KiB 13,387 / 11,694 / 12,568. (One piece per wave throughout: 2, 4 and 8 were
-// 1-10% behind.)
+// dealt one by one, and of rows up to 2 KiB the layers of 2 tokens at a time, not of 16.
+// The kernel of 16 tokens per workgroup that this one replaced / this with units of 16 /
+// of 2: 2 KiB rows of 32 layers 70,000 tokens 2,866 / 2,905 / 2,873 us, 283,000 11,259 / 11,522 /
+// 11,282, of 80 layers 70,000 7,157 / 7,240 / 7,114; 1.5 KiB rows 171,000 5,333 / 5,475 / 5,348; 1
+// KiB rows 283,000 7,150 / 6,069 / 5,803; 4 KiB rows of 42 layers 108,000 11,842 / 11,404 /
+// 11,523. Without it (chunks, nt sc0 sc1): 2 KiB rows 283,000 tokens 11,533 -> 11,682, of 80
+// layers 70,000 7,481 -> 7,433 against 7,218 with it. Smaller gathers: within 1% either way, 1
+// KiB rows of 11,000 tokens 294 / 236 / 241; rows of 6 KiB 13,387 / 11,694 / 12,568. (One piece
+// per wave throughout: 2, 4 and 8 were 1-10% behind.)
 constexpr int64_t kSlotsHugeBytes = 16ll << 30;
 constexpr int64_t kSlotsHugeRow = 4 << 10;
+constexpr int64_t kSlotsPairRow = 2 << 10;
 
 int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t kv_stride,
                  int64_t page_stride, int64_t page_bytes, int64_t num_blocks, int block_size,
@@ -779,11 +782,13 @@ int slots_launch(bool gather, const uint64_t* layer_base, int n_layers, int64_t 
   a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
   const int64_t vpr = row_bytes >> 4;
   a.least_row = vpr <= 8 && (vpr & (vpr - 1)) == 0 && a.block_shift >= 0 ? 0 : INT64_MIN;
-  const SlotShape h = slot_shape(&a);
-  if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   const bool large = slots_large(a);
-  const bool huge = gather && h.wide && row_bytes <= kSlotsHugeRow &&
+  const bool huge = gather && vpr >= kWave && row_bytes <= kSlotsHugeRow &&
                     slots_moved(a) > kSlotsHugeBytes;
+  const bool pairs = huge && row_bytes <= kSlotsPairRow &&
+                     ((int64_t)n_tokens + 1) / 2 * n_layers <= 0x7fffffffLL;
+  const SlotShape h = slot_shape(&a, pairs ? 2 : 16);
+  if (h.units * n_layers > 0x7fffffffLL) return DSR_ERR_ARG;
   const hipStream_t s = (hipStream_t)stream;
   const size_t dyn = occupancy_lds(slots_wg_per_cu(gather, h.wide), 0);
   return launch_flat(h.units * n_layers, h.pieces, gather ? n_layers : h.units,

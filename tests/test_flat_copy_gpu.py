@@ -279,10 +279,10 @@ def test_padding_alone_is_checked(gpu, where):
         assert (staging == 1).all()
 
 
-@pytest.mark.parametrize("heads,dim", [(5, 104), (16, 128)])
+@pytest.mark.parametrize("heads,dim", [(5, 104), (8, 128), (16, 128)])
 def test_huge_slot_gather(gpu, heads, dim):
-    """The token gather's launch above 16 GiB moved, rows of 65 vectors and of the
-    largest length it takes: the records of the page form, tokens that are left
+    """The token gather's launch above 16 GiB moved, rows of 65 vectors, of 2 KiB
+    (in units of 2 tokens up to there) and of 4 KiB: the records of the page form, tokens that are left
     out untouched."""
     print(f"case: huge slot gather H{heads} D{dim}", flush=True)
     layers, block, row = 64, 16, heads * dim * 2
